@@ -5,7 +5,7 @@
 // include/outer.hpp:15-48, whose simd_loop<OUTER> does c[i] += a[i] * b[j]
 // line by line, include/simd_loop.hpp:38-50).  Every element is one fused
 // multiply-add, c = fma(alpha * x[i], y[j], c), in whichever storage order C
-// has: a workgroup walks whole lines of C along its unit-stride index with
+// has: a workgroup updates one row of C along its unit-stride index with
 // 128-bit read-modify-writes.
 //
 // Transpose, C = A^T (counterpart of amt::transpose_helper,
@@ -33,81 +33,118 @@ __device__ inline void st4u(float* p, float4 v) {
     __builtin_nontemporal_store(t, reinterpret_cast<f32x4_u*>(p));
 }
 
+constexpr int kLine = 32;  // floats per 128-byte line
+// Updates of more than this are read with the non-temporal hint: a C that
+// outgrows the caches gains by it (10007 x 8191, 328 MB: 113.5 against 121.5
+// us), one that a later pass finds in the 256 MB last-level cache loses
+// (3001 x 2003, 24 MB: 10.1 against 8.7 us); 2000 x 15000 (120 MB): equal.
+constexpr int64_t kStreamBytes = (int64_t)96 << 20;
+
+// Floats from p to the next 128-byte line: the head of a row, which is written
+// element by element so that the 128-bit groups after it fill whole lines.
+// A 1 KB wavefront store that starts inside a line leaves two lines of every
+// nine partly written, and each is then merged in memory.
+__device__ inline int line_head(const float* p) {
+    return (int)((0 - (reinterpret_cast<uintptr_t>(p) >> 2)) & (kLine - 1));
+}
+
+// Row of this thread's L threads among the workgroup's NT / L: uniform over a
+// wavefront, kept scalar so that row addresses are.
+template <int L>
+__device__ inline int row_in_group() {
+    return L == NT ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / L);
+}
+
+template <bool COLSCALE>
+__device__ inline float4 update4(float alpha, float ur, float4 w, float4 c) {
+    if (COLSCALE)
+        return make_float4(fmaf(alpha * w.x, ur, c.x), fmaf(alpha * w.y, ur, c.y),
+                           fmaf(alpha * w.z, ur, c.z), fmaf(alpha * w.w, ur, c.w));
+    return make_float4(fmaf(ur, w.x, c.x), fmaf(ur, w.y, c.y), fmaf(ur, w.z, c.z),
+                       fmaf(ur, w.w, c.w));
+}
+
 // Rank-1 update of a row-major view D (R x Cc, rows ld apart): D[r][c] +=
 // a(r, c) * b(r, c) with a = alpha * (COLSCALE ? v[c] : u[r]) and b the other
 // vector's element, so that the x factor of C += alpha x y^T is the scaled
-// one in both storage orders.  Workgroups take rows in a grid stride; the
-// threads of a workgroup cover a row with 128-bit groups.
-template <bool COLSCALE>
+// one in both storage orders.  L threads (a workgroup, or a wavefront for
+// short rows) cover a row with 128-bit groups that start on the row's first
+// whole line.  Bound by
+// HBM reads and writes.  10007 x 8191 (rows 4-byte aligned): 152 us with
+// groups from the row's first element and 4 workgroups per CU striding over
+// the rows, 131 us from the first whole line, 113.5 us (5.8 TB/s) with a
+// workgroup per row as well; 16384^2: 381 -> 372 us.
+// STREAM: C is read with the non-temporal hint (see kStreamBytes).
+template <bool COLSCALE, bool STREAM, int L, bool LINES>
 __global__ __launch_bounds__(NT) void ger_kernel(int64_t R, int64_t Cc, float alpha,
                                                  const float* __restrict__ u,
                                                  const float* __restrict__ v, float* D,
                                                  int64_t ld) {
-    const int64_t nq = Cc >> 2;
-    for (int64_t r = blockIdx.x; r < R; r += gridDim.x) {
+    const int lane = threadIdx.x % L;
+    for (int64_t r = (int64_t)blockIdx.x * (NT / L) + row_in_group<L>(); r < R;
+         r += (int64_t)gridDim.x * (NT / L)) {
         float* row = D + r * ld;
         const float ur = COLSCALE ? u[r] : alpha * u[r];
-        int64_t q = threadIdx.x;
-        for (; q + NT * (GER_UNROLL - 1) < nq; q += NT * GER_UNROLL) {
+        const int head = LINES ? (int)std::min<int64_t>(line_head(row), Cc) : 0;
+        const int64_t nq = (Cc - head) >> 2;
+        float* body = row + head;
+        const float* w0 = v + head;
+        // head and tail element of this lane (at most 31 + 3 per row), loaded
+        // before the groups so that a short row is one round trip
+        const int64_t e = lane < head ? lane : 4 * nq + lane;
+        float ce = 0.f, we = 0.f;
+        if (LINES && e < Cc) ce = row[e], we = v[e];
+        int64_t q = lane;
+        for (; q + L * (GER_UNROLL - 1) < nq; q += L * GER_UNROLL) {
             float4 c[GER_UNROLL], w[GER_UNROLL];
 #pragma unroll
             for (int k = 0; k < GER_UNROLL; ++k) {
-                c[k] = ld4u_nt(row + 4 * (q + NT * k));
-                w[k] = ld4u(v + 4 * (q + NT * k));
+                c[k] = STREAM ? ld4u_nt(body + 4 * (q + L * k)) : ld4u(body + 4 * (q + L * k));
+                w[k] = ld4u(w0 + 4 * (q + L * k));
             }
 #pragma unroll
-            for (int k = 0; k < GER_UNROLL; ++k) {
-                float4 o;
-                if (COLSCALE) {
-                    o.x = fmaf(alpha * w[k].x, ur, c[k].x);
-                    o.y = fmaf(alpha * w[k].y, ur, c[k].y);
-                    o.z = fmaf(alpha * w[k].z, ur, c[k].z);
-                    o.w = fmaf(alpha * w[k].w, ur, c[k].w);
-                } else {
-                    o.x = fmaf(ur, w[k].x, c[k].x);
-                    o.y = fmaf(ur, w[k].y, c[k].y);
-                    o.z = fmaf(ur, w[k].z, c[k].z);
-                    o.w = fmaf(ur, w[k].w, c[k].w);
-                }
-                st4u(row + 4 * (q + NT * k), o);
-            }
+            for (int k = 0; k < GER_UNROLL; ++k)
+                st4u(body + 4 * (q + L * k), update4<COLSCALE>(alpha, ur, w[k], c[k]));
         }
-        for (; q < nq; q += NT) {
-            const float4 c = ld4u(row + 4 * q), w = ld4u(v + 4 * q);
-            float4 o;
-            if (COLSCALE) {
-                o = make_float4(fmaf(alpha * w.x, ur, c.x), fmaf(alpha * w.y, ur, c.y),
-                                fmaf(alpha * w.z, ur, c.z), fmaf(alpha * w.w, ur, c.w));
-            } else {
-                o = make_float4(fmaf(ur, w.x, c.x), fmaf(ur, w.y, c.y), fmaf(ur, w.z, c.z),
-                                fmaf(ur, w.w, c.w));
-            }
-            st4u(row + 4 * q, o);
-        }
-        const int64_t t = (nq << 2) + threadIdx.x;
-        if (t < Cc) row[t] = COLSCALE ? fmaf(alpha * v[t], ur, row[t]) : fmaf(ur, v[t], row[t]);
+        for (; q < nq; q += L)
+            st4u(body + 4 * q, update4<COLSCALE>(alpha, ur, ld4u(w0 + 4 * q), ld4u(body + 4 * q)));
+        if (!LINES && e < Cc) ce = row[e], we = v[e];
+        if (e < Cc) row[e] = COLSCALE ? fmaf(alpha * we, ur, ce) : fmaf(ur, we, ce);
     }
 }
 
-// D (R x Cc, ldd) = S (R x Cc, lds), both row-major: a line copy.
+// D (R x Cc, ldd) = S (R x Cc, lds), both row-major: a line copy, the 128-bit
+// groups starting on D's first whole line of each row.  STREAM: S is read
+// with the non-temporal hint, only where S's groups start on lines too:
+// otherwise neighbouring wavefronts share S's lines, and the hint makes each
+// fetch them again.
+template <bool STREAM, int L, bool LINES>
 __global__ __launch_bounds__(NT) void copy_lines_kernel(int64_t R, int64_t Cc,
                                                         const float* __restrict__ S, int64_t lds,
                                                         float* __restrict__ D, int64_t ldd) {
-    const int64_t nq = Cc >> 2;
-    for (int64_t r = blockIdx.x; r < R; r += gridDim.x) {
-        const float* s = S + r * lds;
-        float* d = D + r * ldd;
-        int64_t q = threadIdx.x;
-        for (; q + NT * (GER_UNROLL - 1) < nq; q += NT * GER_UNROLL) {
+    const int lane = threadIdx.x % L;
+    for (int64_t r = (int64_t)blockIdx.x * (NT / L) + row_in_group<L>(); r < R;
+         r += (int64_t)gridDim.x * (NT / L)) {
+        float* row = D + r * ldd;
+        const int head = LINES ? (int)std::min<int64_t>(line_head(row), Cc) : 0;
+        const int64_t nq = (Cc - head) >> 2;
+        const float* s = S + r * lds + head;
+        float* d = row + head;
+        const int64_t e = lane < head ? lane : 4 * nq + lane;  // as in ger_kernel
+        float se = 0.f;
+        if (LINES && e < Cc) se = S[r * lds + e];
+        int64_t q = lane;
+        for (; q + L * (GER_UNROLL - 1) < nq; q += L * GER_UNROLL) {
             float4 t[GER_UNROLL];
 #pragma unroll
-            for (int k = 0; k < GER_UNROLL; ++k) t[k] = ld4u_nt(s + 4 * (q + NT * k));
+            for (int k = 0; k < GER_UNROLL; ++k)
+                t[k] = STREAM ? ld4u_nt(s + 4 * (q + L * k)) : ld4u(s + 4 * (q + L * k));
 #pragma unroll
-            for (int k = 0; k < GER_UNROLL; ++k) st4u(d + 4 * (q + NT * k), t[k]);
+            for (int k = 0; k < GER_UNROLL; ++k) st4u(d + 4 * (q + L * k), t[k]);
         }
-        for (; q < nq; q += NT) st4u(d + 4 * q, ld4u(s + 4 * q));
-        const int64_t t = (nq << 2) + threadIdx.x;
-        if (t < Cc) d[t] = s[t];
+        for (; q < nq; q += L) st4u(d + 4 * q, ld4u(s + 4 * q));
+        if (!LINES && e < Cc) se = S[r * lds + e];
+        if (e < Cc) row[e] = se;
     }
 }
 
@@ -265,8 +302,22 @@ __global__ __launch_bounds__(NT) void transpose_inplace_kernel(int64_t n, float*
     if (bi != bj) tile_store_t(t1, A, ld, n, n, c0, r0);
 }
 
-int64_t row_grid(int64_t rows) {
-    return std::max<int64_t>(1, std::min<int64_t>(rows, 4 * (int64_t)device_cu_count()));
+// Split of the rows for the rank-1 and copy kernels, by what bounds them:
+// rows of more than 1024 floats take a workgroup each and start on whole
+// lines; shorter ones are bound by the rate workgroups start at and by the
+// round trips of a row, so up to 512 floats a wavefront takes each row (outer
+// 16382 x 300: 11.3 -> 9.3 us; a workgroup per row 12.8), and between the two
+// 4 workgroups per CU stride over the rows (copy of 16000 x 900: 18.8 us; a
+// wavefront per row 26, a workgroup per row 19.6).
+struct RowSplit {
+    bool by_wave, lines;
+    unsigned grid;
+};
+RowSplit row_split(int64_t rows, int64_t Cc) {
+    const bool by_wave = Cc <= 512, lines = Cc > 1024;
+    const int64_t most = by_wave || lines ? 1 << 22 : 4 * (int64_t)device_cu_count();
+    const int64_t groups = by_wave ? ceil_div(rows, NT / 64) : rows;
+    return {by_wave, lines, (unsigned)std::max<int64_t>(1, std::min(groups, most))};
 }
 
 bool overlaps(const float* a, int64_t na, const float* b, int64_t nb) {
@@ -298,12 +349,21 @@ extern "C" omb_status omb_sger(int64_t M, int64_t N, float alpha, const float* x
     int64_t ld = 0;
     OMB_TRY(resolve_layout("omb_sger C", M, N, rsC, csC, &row, &ld));
     hipStream_t s = (hipStream_t)stream;
-    if (row)
-        hipLaunchKernelGGL(ger_kernel<false>, dim3((unsigned)row_grid(M)), dim3(NT), 0, s, M, N,
-                           alpha, x, y, C, ld);
-    else  // column-major C: its lines are the columns, rows of the view are j
-        hipLaunchKernelGGL(ger_kernel<true>, dim3((unsigned)row_grid(N)), dim3(NT), 0, s, N, M,
-                           alpha, y, x, C, ld);
+    // row-major C: its rows; column-major C: its columns are the lines, and
+    // rows of the view are j
+    const int64_t R = row ? M : N, Cc = row ? N : M;
+    const bool stream_c = R * Cc > kStreamBytes / (int64_t)sizeof(float);
+    const RowSplit sp = row_split(R, Cc);
+    const float *u = row ? x : y, *v = row ? y : x;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(sp.grid), dim3(NT), 0, s, R, Cc, alpha, u, v, C, ld);
+    };
+    if (sp.by_wave && row) launch(ger_kernel<false, false, 64, false>);
+    else if (sp.by_wave) launch(ger_kernel<true, false, 64, false>);
+    else if (!sp.lines && row) launch(ger_kernel<false, false, NT, false>);
+    else if (!sp.lines) launch(ger_kernel<true, false, NT, false>);
+    else if (row) launch(stream_c ? ger_kernel<false, true, NT, true> : ger_kernel<false, false, NT, true>);
+    else launch(stream_c ? ger_kernel<true, true, NT, true> : ger_kernel<true, false, NT, true>);
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
@@ -353,8 +413,17 @@ extern "C" omb_status omb_stranspose(int64_t M, int64_t N, const float* A, int64
             hipLaunchKernelGGL(transpose_edge_kernel, dim3((unsigned)nedge), dim3(NT), 0, s, R, Cc,
                                A, lda, C, ldc);
     } else {
-        hipLaunchKernelGGL(copy_lines_kernel, dim3((unsigned)row_grid(R)), dim3(NT), 0, s, R, Cc,
-                           A, lda, C, ldc);
+        // whole-line groups of C are whole-line groups of A on every row
+        const bool stream = (reinterpret_cast<uintptr_t>(A) - reinterpret_cast<uintptr_t>(C)) %
+                                    (kLine * sizeof(float)) == 0 &&
+                            (lda - ldc) % kLine == 0;
+        const RowSplit sp = row_split(R, Cc);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(sp.grid), dim3(NT), 0, s, R, Cc, A, lda, C, ldc);
+        };
+        if (sp.by_wave) launch(copy_lines_kernel<false, 64, false>);
+        else if (!sp.lines) launch(copy_lines_kernel<false, NT, false>);
+        else launch(stream ? copy_lines_kernel<true, NT, true> : copy_lines_kernel<false, NT, true>);
     }
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
