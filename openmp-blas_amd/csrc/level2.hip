@@ -68,12 +68,11 @@ __device__ inline float4 update4(float alpha, float ur, float4 w, float4 c) {
 // a(r, c) * b(r, c) with a = alpha * (COLSCALE ? v[c] : u[r]) and b the other
 // vector's element, so that the x factor of C += alpha x y^T is the scaled
 // one in both storage orders.  L threads (a workgroup, or a wavefront for
-// short rows) cover a row with 128-bit groups that start on the row's first
-// whole line.  Bound by
-// HBM reads and writes.  10007 x 8191 (rows 4-byte aligned): 152 us with
-// groups from the row's first element and 4 workgroups per CU striding over
-// the rows, 131 us from the first whole line, 113.5 us (5.8 TB/s) with a
-// workgroup per row as well; 16384^2: 381 -> 372 us.
+// short rows) cover a row with 128-bit groups, from the row's first whole
+// line with LINES.  Bound by HBM reads and writes.  10007 x 8191 (rows 4-byte
+// aligned): 152 us with groups from the row's first element and 4 workgroups
+// per CU striding over the rows, 131 us from the first whole line, 113.5 us
+// (5.8 TB/s) with a workgroup per row as well; 16384^2: 381 -> 372 us.
 // STREAM: C is read with the non-temporal hint (see kStreamBytes).
 template <bool COLSCALE, bool STREAM, int L, bool LINES>
 __global__ __launch_bounds__(NT) void ger_kernel(int64_t R, int64_t Cc, float alpha,
@@ -209,77 +208,95 @@ __device__ inline void tile_put(float (*tile)[TPAD], const float4 (&v)[TT / 16])
     }
 }
 
-// D (Cc x R, ldd) = S^T (S: R x Cc, lds), both row-major, over the whole
-// 64x64 tiles (the first TR x TC tiles): each step of a workgroup reads TPB
-// consecutive tiles into registers (all loads in flight at once), parks
-// them in LDS and writes their transposes; grid stride over a fixed grid.
-// No edge guards: guarded loads and stores in this loop measured slower
-// (0.55 of HBM peak at 16384^2 against 0.65), so partial tiles go to
-// transpose_edge_kernel.  One tile per step measured 0.57 (a plain copy,
-// read and write, reaches 0.75 there).
-constexpr int TPB = 4;
-__global__ __launch_bounds__(NT) void transpose_tiles_kernel(int64_t TR, int64_t TC,
+// D (Cc x R, ldd) = S^T (S: R x Cc, lds), both row-major: one tile of RT rows
+// of S and CT rows of D per workgroup, through LDS.  Each row of D is written
+// from its tile's start moved back by the row's offset in its 128-byte line
+// (0 .. 31 floats): every 128-bit store then fills whole lines, with a scalar
+// guard only at the row's ends.  For that the workgroup reads the 31 rows of
+// S before the tile too (none when D's rows start on lines); they are the
+// neighbour's rows, and the workgroups of one XCD take neighbouring tiles
+// along r, so they come from its L2.  Reads are cached, as tiles share S's
+// lines as well.  Bound by HBM.  Measured against 64x64 tiles stored from
+// their own start, with a second launch for partial tiles: 8001 x 12007 (rows
+// 4-byte aligned; partly written lines are merged in memory) 308 -> 150 us
+// (5.1 TB/s), 3001 x 2503 24.7 -> 11.4 us, 4096^2 27.2 -> 21.4 us.
+// diag: tiles step along c with r.  With rows 32 KB apart a column of tiles
+// reads, and a row of them writes, the same memory channels: 8192^2 118 us
+// without, 99 us with it, 16384^2 462 and 412 us; other strides lose 2-9%
+// by it (8000 x 12032: 144 and 158 us).
+template <int RT, int CT>
+__global__ __launch_bounds__(NT) void transpose_lines_kernel(int64_t R, int64_t Cc, int64_t GR,
+                                                             int64_t GC,
                                                              const float* __restrict__ S,
                                                              int64_t lds, float* __restrict__ D,
-                                                             int64_t ldd) {
-    __shared__ float tile[TPB][TT][TPAD];
-    const int64_t ntiles = TR * TC;
-    const int g = threadIdx.x & 15, rr = threadIdx.x >> 4;
-    for (int64_t t0 = (int64_t)blockIdx.x * TPB; t0 < ntiles; t0 += (int64_t)gridDim.x * TPB) {
-        float4 v[TPB][TT / 16];
+                                                             int64_t ldd, int on_lines, int diag) {
+    constexpr int LR = RT + kLine;                      // rows of S held in LDS
+    constexpr int CQ = CT / 4, RPI = NT / CQ;           // loads: groups per row, rows per step
+    constexpr int RQ = RT / 4, CPI = NT / RQ;           // stores: groups per row of D, rows per step
+    static_assert(kLine % RPI == 0 && RT % RPI == 0 && CT % CPI == 0, "whole steps");
+    __shared__ float tile[LR][CT + 1];
+    const int cq = threadIdx.x % CQ, rr = threadIdx.x / CQ;
+    const int g = threadIdx.x % RQ, cc = threadIdx.x / RQ;
+    const int64_t ntiles = GR * GC;
+    // XCD x (workgroups x mod 8) takes tiles [x, x+1) * ntiles / 8, r fastest.
+    const int64_t x = blockIdx.x & 7, end = ntiles * (x + 1) / 8;
+    for (int64_t t = ntiles * x / 8 + (blockIdx.x >> 3); t < end; t += gridDim.x >> 3) {
+        const int64_t gr = t % GR, gc = diag ? (t / GR + gr) % GC : t / GR;
+        const int64_t r0 = gr * RT, c0 = gc * CT;
+        const bool full = (on_lines || r0 >= kLine) && r0 + RT <= R && c0 + CT <= Cc;
+        float4 v[LR / RPI];
+        if (full) {
 #pragma unroll
-        for (int b = 0; b < TPB; ++b) {
-            const int64_t t = t0 + b < ntiles ? t0 + b : ntiles - 1;
-            const int64_t r0 = (t / TC) * TT, c0 = (t % TC) * TT;
+            for (int k = 0; k < LR / RPI; ++k)
+                if (k * RPI >= kLine || !on_lines)
+                    v[k] = ld4u(S + (r0 - kLine + rr + RPI * k) * lds + c0 + 4 * cq);
+        } else {  // clamped indices: what lies outside S is not stored
 #pragma unroll
-            for (int k = 0; k < TT / 16; ++k)
-                v[b][k] = ld4u_nt(S + (r0 + rr + 16 * k) * lds + c0 + 4 * g);
+            for (int k = 0; k < LR / RPI; ++k) {
+                const int64_t r = r0 - kLine + rr + RPI * k, c = c0 + 4 * cq;
+                const float* p = S + std::min(std::max<int64_t>(r, 0), R - 1) * lds;
+                if (c + 3 < Cc) {
+                    v[k] = ld4u(p + c);
+                } else {
+                    v[k] = make_float4(p[std::min(c, Cc - 1)], p[std::min(c + 1, Cc - 1)],
+                                       p[std::min(c + 2, Cc - 1)], 0.f);
+                }
+            }
         }
-        __syncthreads();  // the previous step's tiles have been written out
+        __syncthreads();  // the previous tile has been written out
 #pragma unroll
-        for (int b = 0; b < TPB; ++b) tile_put(tile[b], v[b]);
+        for (int k = 0; k < LR / RPI; ++k) {
+            if (k * RPI < kLine && on_lines) continue;
+            float* p = &tile[rr + RPI * k][4 * cq];
+            p[0] = v[k].x;
+            p[1] = v[k].y;
+            p[2] = v[k].z;
+            p[3] = v[k].w;
+        }
         __syncthreads();
 #pragma unroll
-        for (int b = 0; b < TPB; ++b) {
-            const int64_t t = t0 + b;
-            if (t >= ntiles) break;
-            const int64_t r0 = (t / TC) * TT, c0 = (t % TC) * TT;
-#pragma unroll
-            for (int k = 0; k < TT / 16; ++k) {
-                const int lc = rr + 16 * k;
-                st4u(D + (c0 + lc) * ldd + r0 + 4 * g,
-                     make_float4(tile[b][4 * g][lc], tile[b][4 * g + 1][lc], tile[b][4 * g + 2][lc],
-                                 tile[b][4 * g + 3][lc]));
+        for (int k = 0; k < CT / CPI; ++k) {
+            const int lc = cc + CPI * k;
+            float* d = D + (c0 + lc) * ldd;
+            const int back = (kLine - line_head(d + r0)) & (kLine - 1);
+            const int lr = kLine - back + 4 * g;
+            const int64_t r = r0 - back + 4 * g;
+            const float4 o = make_float4(tile[lr][lc], tile[lr + 1][lc], tile[lr + 2][lc],
+                                         tile[lr + 3][lc]);
+            if (full) {
+                st4u(d + r, o);
+            } else if (c0 + lc < Cc) {
+                if (r >= 0 && r + 3 < R) {
+                    st4u(d + r, o);
+                } else {
+                    if (r >= 0 && r < R) d[r] = o.x;
+                    if (r >= -1 && r + 1 < R) d[r + 1] = o.y;
+                    if (r >= -2 && r + 2 < R) d[r + 2] = o.z;
+                    if (r >= -3 && r + 3 < R) d[r + 3] = o.w;
+                }
             }
         }
     }
-}
-
-// The partial tiles of the same transpose: the last tile column (when Cc %
-// TT != 0) for the TR whole tile rows, then the last tile row (when R % TT
-// != 0) across all tile columns; one tile per workgroup, guarded.
-__global__ __launch_bounds__(NT) void transpose_edge_kernel(int64_t R, int64_t Cc,
-                                                            const float* __restrict__ S,
-                                                            int64_t lds, float* __restrict__ D,
-                                                            int64_t ldd) {
-    __shared__ float tile[TT][TPAD];
-    const int64_t TR = R / TT, TC = Cc / TT, tcol = (Cc + TT - 1) / TT;
-    const int64_t ncol = Cc % TT ? TR : 0;  // right strip
-    const int64_t e = blockIdx.x;
-    int64_t tr, tc;
-    if (e < ncol) {
-        tr = e;
-        tc = TC;
-    } else {
-        tr = TR;
-        tc = e - ncol;
-        if (tc >= tcol) return;
-    }
-    float4 v[TT / 16];
-    tile_regs(v, S, lds, R, Cc, tr * TT, tc * TT);
-    tile_put(tile, v);
-    __syncthreads();
-    tile_store_t(tile, D, ldd, R, Cc, tr * TT, tc * TT);
 }
 
 // Square in-place transpose of A (n x n, row-major view with ld): workgroup
@@ -397,21 +414,17 @@ extern "C" omb_status omb_stranspose(int64_t M, int64_t N, const float* A, int64
     const int64_t R = a_row ? M : N, Cc = a_row ? N : M;
     hipStream_t s = (hipStream_t)stream;
     if (a_row == c_row) {
-        const int64_t TR = R / TT, TC = Cc / TT, ntiles = TR * TC;
-        if (ntiles > 0) {
-            const int64_t grid = std::max<int64_t>(
-                1, std::min<int64_t>(ceil_div(ntiles, TPB), 2 * device_cu_count()));
-            hipLaunchKernelGGL(transpose_tiles_kernel, dim3((unsigned)grid), dim3(NT), 0, s, TR,
-                               TC, A, lda, C, ldc);
-        }
-        const int64_t nedge = (Cc % TT ? TR : 0) + (R % TT ? ceil_div(Cc, TT) : 0);
-        if (nedge > 0x7fffffffLL) {
-            set_error("omb_stranspose: too many edge tiles for one launch");
-            return OMB_EUNSUPPORTED;
-        }
-        if (nedge > 0)
-            hipLaunchKernelGGL(transpose_edge_kernel, dim3((unsigned)nedge), dim3(NT), 0, s, R, Cc,
-                               A, lda, C, ldc);
+        const bool on_lines = reinterpret_cast<uintptr_t>(C) % (kLine * sizeof(float)) == 0 &&
+                              ldc % kLine == 0;
+        const bool diag = on_lines && (lda % 8192 == 0 || ldc % 8192 == 0);
+        const bool big = R * Cc >= (int64_t)1 << 24;
+        const int64_t rt = big ? 128 : 64, ct = big ? 64 : 32;
+        // rows of D moved back by up to 31 floats can need one tile more
+        const int64_t GR = ceil_div(R + (on_lines ? 0 : kLine - 1), rt), GC = ceil_div(Cc, ct);
+        const dim3 grid((unsigned)std::min<int64_t>(round_up(GR * GC, 8), 1 << 24));
+        const auto kernel = big ? transpose_lines_kernel<128, 64> : transpose_lines_kernel<64, 32>;
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, s, R, Cc, GR, GC, A, lda, C, ldc,
+                           on_lines ? 1 : 0, diag ? 1 : 0);
     } else {
         // whole-line groups of C are whole-line groups of A on every row
         const bool stream = (reinterpret_cast<uintptr_t>(A) - reinterpret_cast<uintptr_t>(C)) %
