@@ -41,7 +41,10 @@ omb_status get_workspace(hipStream_t stream, size_t bytes, Workspace** out) {
     OMB_HIP_TRY(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(g_ws_mu);
     auto& slot = ws_map()[WsKey{dev, stream}];
-    if (!slot) slot = std::make_unique<Workspace>();
+    if (!slot) {
+        slot = std::make_unique<Workspace>();
+        slot->arrivals = arrival_counters((int)ws_map().size() - 1);
+    }
     Workspace* ws = slot.get();
     if (bytes > ws->bytes) {
         if (ws->buf) OMB_HIP_TRY(hipFree(ws->buf));  // hipFree waits for work in flight

@@ -34,11 +34,19 @@ __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + 
 __host__ __device__ inline int64_t round_up(int64_t a, int64_t b) { return ceil_div(a, b) * b; }
 
 // --------------------------------------------------------------- workspace --
-// Per-stream scratch memory: one grow-only device buffer.
+// Per-stream scratch memory: one grow-only device buffer, and the stream's
+// own arrival counters (zero between launches; null for streams past the
+// first kArrivalSlots, whose calls add their partials in a second launch).
 struct Workspace {
     void* buf = nullptr;
     size_t bytes = 0;
+    unsigned* arrivals = nullptr;
 };
+constexpr int kArrivalSlots = 64;      // streams with counters, per process
+constexpr int kArrivalCounters = 256;  // per stream
+constexpr int kArrivalStride = 16;     // counters lie 64 bytes apart
+// Counters of workspace `slot` on the current device, or null.
+unsigned* arrival_counters(int slot);
 
 // Compute units of the current device (cached per device).
 int device_cu_count();
@@ -141,7 +149,7 @@ omb_status launch_sdot(int64_t n, const float* x, const float* y, float* result,
 // SDOT with a caller-supplied partial buffer of sdot_blocks(n) doubles.
 int64_t sdot_blocks(int64_t n);
 omb_status launch_sdot_ws(int64_t n, const float* x, const float* y, float* result,
-                          double* part, hipStream_t s);
+                          double* part, hipStream_t s, unsigned* arrivals = nullptr);
 // SDOT with its partials in the library's static device scratch (no
 // allocation); sdot_scratch_setup finds that scratch's address on the
 // current device (once per device) and optionally returns it.
@@ -244,6 +252,40 @@ __device__ inline double wave_max(double v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
     return v;
+}
+
+// Partial results handed from the workgroups of one launch to the last one
+// that arrives.  The values go through agent-scope atomics, which the eight
+// XCDs' L2s keep coherent one by one; a release or acquire fence at agent
+// scope would write back or invalidate the whole L2 instead, which costs a
+// streaming kernel more than a second launch.
+__device__ inline void agent_store(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void agent_store(double* p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ inline T agent_load(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// True in every thread of the last of n workgroups to call this on a counter
+// that is zero; leaves it zero.  Every wavefront first waits until its agent
+// stores have completed (a store counts down vmcnt once it is visible at its
+// scope), then the barrier holds the arrival back until all have.
+__device__ inline bool last_arrival(unsigned* counter, unsigned n) {
+    __shared__ int s_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned before =
+            __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = before == n - 1;
+        if (before == n - 1)
+            __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    return s_last != 0;
 }
 
 // Map a 1-D block id to a tile id so that the blocks the hardware sends to

@@ -6,12 +6,18 @@
 // Here: a workgroup-interleaved grid-stride loop of 128-bit loads (4 float4
 // of x and of y in flight per lane) into FP32 lane sums, a fixed butterfly
 // per wavefront, the four wavefront sums in order, one partial per
-// workgroup; a second one-workgroup kernel adds the partials in a fixed
-// order -- in FP64 when n >= 2^26, in FP32 below.  (A second launch instead of a last-workgroup ticket: on this
-// GPU an agent-scope fence writes back and invalidates the XCD's L2, which
-// costs more than the launch.)  The grid depends on n only and the loads do
-// not depend on alignment, so the result is bitwise reproducible for any
-// placement of the operands.
+// workgroup; the last workgroup to arrive adds the partials in a fixed order
+// -- in FP64 when n >= 2^26, in FP32 below.  It learns that it is the last
+// from the stream's arrival counters, two levels of them past 128
+// workgroups: an arrival on one address takes about 12 ns, so 1024 on one
+// counter took 12 us, in groups of 32 2.4 us.  Below 2^24 elements this beats
+// a second launch (20000: 7.5 -> 5.1 us a call, 1000003: 7.3 -> 6.0); from
+// there the second launch adds the partials, hidden behind the first one's
+// start (2^28: 308 us, 310 with arrivals).  omb_sdot_noalloc and served
+// requests have no counters of their own and take the second launch too, in
+// the same order.  The grid depends on n only and the loads do not depend on
+// alignment, so the result is bitwise reproducible for any placement of the
+// operands.
 #include <algorithm>
 #include <mutex>
 
@@ -24,6 +30,7 @@ constexpr int NT = 256;
 constexpr int UNROLL = 4;
 constexpr int kMaxBlocks = 1024;
 constexpr int64_t kF64Combine = int64_t(1) << 26;
+constexpr int64_t kArrivalMost = int64_t(1) << 24;  // elements up to which arrivals are used
 
 }  // namespace
 }  // namespace omb
@@ -35,12 +42,48 @@ constexpr int64_t kF64Combine = int64_t(1) << 26;
 // address, which set-up obtains with hipGetSymbolAddress per device.
 static __device__ __align__(256) double scratch[omb::kMaxBlocks];
 
+// Arrival counters of every workspace (common.hpp), zero when the module is
+// loaded and again after every launch that uses them.
+static __device__ __align__(256) unsigned
+    arrivals[omb::kArrivalSlots][omb::kArrivalCounters * omb::kArrivalStride];
+
 namespace omb {
 namespace {
 
+// Sum of the per-workgroup partials by one workgroup: thread t takes partials
+// t, t+NT, ... in order, then a fixed tree -- in FP64 or in FP32.
+template <typename Load>
+__device__ inline void combine_partials(int count, int f64, float* result, Load load) {
+    __shared__ double s_red[NT];
+    if (f64) {
+        double s = 0.0;
+        for (int b = threadIdx.x; b < count; b += NT) s += load(b);
+        s_red[threadIdx.x] = s;
+    } else {
+        float s = 0.f;
+        for (int b = threadIdx.x; b < count; b += NT) s += (float)load(b);
+        s_red[threadIdx.x] = (double)s;
+    }
+    __syncthreads();
+    for (int w = NT / 2; w >= 1; w >>= 1) {
+        if (threadIdx.x < w) {
+            if (f64) s_red[threadIdx.x] += s_red[threadIdx.x + w];
+            else s_red[threadIdx.x] = (double)((float)s_red[threadIdx.x] + (float)s_red[threadIdx.x + w]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *result = (float)s_red[0];
+}
+
+// Workgroups per first-level arrival counter; up to kOneLevel share one.
+constexpr int kArrivalGroup = 32, kOneLevel = 128;
+static_assert(kMaxBlocks / kArrivalGroup < kArrivalCounters, "a counter per group and one over them");
+
+// count: this stream's arrival counters, or null (the partials are then added
+// by sdot_combine_kernel).
 __global__ __launch_bounds__(NT) void sdot_kernel(int64_t n, const float* __restrict__ x,
                                                   const float* __restrict__ y, float* result,
-                                                  double* partial) {
+                                                  double* partial, unsigned* count, int f64) {
     const int64_t gtid = (int64_t)blockIdx.x * NT + threadIdx.x;
     const int64_t nthr = (int64_t)gridDim.x * NT;
     float acc = 0.f;
@@ -76,33 +119,25 @@ __global__ __launch_bounds__(NT) void sdot_kernel(int64_t n, const float* __rest
         float s = s_wave[0];
         for (int w = 1; w < NT / 64; ++w) s += s_wave[w];
         if (gridDim.x == 1) *result = s;
+        else if (count) agent_store(&partial[blockIdx.x], (double)s);
         else partial[blockIdx.x] = (double)s;
     }
+    if (gridDim.x == 1 || !count) return;
+    const int blocks = (int)gridDim.x;
+    if (blocks > kOneLevel) {
+        const int g = (int)blockIdx.x / kArrivalGroup;
+        const int in_group = min(kArrivalGroup, blocks - g * kArrivalGroup);
+        if (!last_arrival(count + (1 + g) * kArrivalStride, in_group)) return;
+        if (!last_arrival(count, (unsigned)ceil_div(blocks, kArrivalGroup))) return;
+    } else if (!last_arrival(count, (unsigned)blocks)) {
+        return;
+    }
+    combine_partials(blocks, f64, result, [&](int b) { return agent_load(&partial[b]); });
 }
 
-// One workgroup adds the per-workgroup partials: thread t takes partials
-// t, t+NT, ... in order, then a fixed tree -- in FP64 or in FP32.
 __global__ __launch_bounds__(NT) void sdot_combine_kernel(const double* __restrict__ partial,
                                                           int count, int f64, float* result) {
-    __shared__ double s_red[NT];
-    if (f64) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < count; b += NT) s += partial[b];
-        s_red[threadIdx.x] = s;
-    } else {
-        float s = 0.f;
-        for (int b = threadIdx.x; b < count; b += NT) s += (float)partial[b];
-        s_red[threadIdx.x] = (double)s;
-    }
-    __syncthreads();
-    for (int w = NT / 2; w >= 1; w >>= 1) {
-        if (threadIdx.x < w) {
-            if (f64) s_red[threadIdx.x] += s_red[threadIdx.x + w];
-            else s_red[threadIdx.x] = (double)((float)s_red[threadIdx.x] + (float)s_red[threadIdx.x + w]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *result = (float)s_red[0];
+    combine_partials(count, f64, result, [&](int b) { return partial[b]; });
 }
 
 __global__ void zero_scalar_kernel(float* r) { *r = 0.f; }
@@ -116,7 +151,7 @@ int64_t sdot_blocks(int64_t n) {
 }
 
 omb_status launch_sdot_ws(int64_t n, const float* x, const float* y, float* result,
-                          double* part, hipStream_t s) {
+                          double* part, hipStream_t s, unsigned* arrivals) {
     if (n <= 0) {
         hipLaunchKernelGGL(zero_scalar_kernel, dim3(1), dim3(1), 0, s, result);
         OMB_HIP_TRY(hipGetLastError());
@@ -124,8 +159,10 @@ omb_status launch_sdot_ws(int64_t n, const float* x, const float* y, float* resu
     }
     const int64_t blocks = sdot_blocks(n);
     const int f64 = n >= kF64Combine ? 1 : 0;
-    hipLaunchKernelGGL(sdot_kernel, dim3((unsigned)blocks), dim3(NT), 0, s, n, x, y, result, part);
-    if (blocks > 1)
+    if (n > kArrivalMost) arrivals = nullptr;
+    hipLaunchKernelGGL(sdot_kernel, dim3((unsigned)blocks), dim3(NT), 0, s, n, x, y, result, part,
+                       arrivals, f64);
+    if (blocks > 1 && !arrivals)
         hipLaunchKernelGGL(sdot_combine_kernel, dim3(1), dim3(NT), 0, s, part, (int)blocks, f64,
                            result);
     OMB_HIP_TRY(hipGetLastError());
@@ -178,7 +215,18 @@ omb_status launch_sdot_noalloc(int64_t n, const float* x, const float* y, float*
 omb_status launch_sdot(int64_t n, const float* x, const float* y, float* result, hipStream_t s) {
     Workspace* ws = nullptr;
     OMB_TRY(get_workspace(s, n > 0 ? (size_t)sdot_blocks(n) * sizeof(double) : 0, &ws));
-    return launch_sdot_ws(n, x, y, result, reinterpret_cast<double*>(ws->buf), s);
+    return launch_sdot_ws(n, x, y, result, reinterpret_cast<double*>(ws->buf), s,
+                          ws->arrivals);
+}
+
+unsigned* arrival_counters(int slot) {
+    if (slot < 0 || slot >= kArrivalSlots) return nullptr;
+    void* p = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(arrivals)) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return static_cast<unsigned*>(p) + (size_t)slot * kArrivalCounters * kArrivalStride;
 }
 
 }  // namespace omb
