@@ -66,6 +66,14 @@ struct MatView {
 omb_status resolve_layout(const char* name, int64_t rows, int64_t cols, int64_t rs, int64_t cs,
                           bool* unit_col, int64_t* ld);
 
+// Operands of more bytes than this are read with the non-temporal hint: those
+// that outgrow the caches gain by it (rank-1 update of 10007 x 8191, 328 MB:
+// 113.5 against 121.5 us; column GEMV of 9003 x 6001, 216 MB: 34.4 against
+// 35.7), those that a later pass finds in the 256 MB last-level cache lose
+// (update of 3001 x 2003, 24 MB: 10.1 against 8.7 us; GEMV of 3000^2: 9.1
+// against 7.3); an update of 120 MB: equal.
+constexpr int64_t kStreamBytes = (int64_t)96 << 20;
+
 // ------------------------------------------------------------ kernels -----
 // Plain FP32 SGEMM, row-major C (ldc), A K-contiguous iff a_kc, B N-contiguous
 // iff b_nc.  C = alpha*A*B + beta*C.
@@ -270,20 +278,14 @@ __device__ inline T agent_load(const T* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // True in every thread of the last of n workgroups to call this on a counter
-// that is zero; leaves it zero.  Every wavefront first waits until its agent
+// that is zero; the last arrival wraps it to zero again.  Every wavefront first waits until its agent
 // stores have completed (a store counts down vmcnt once it is visible at its
 // scope), then the barrier holds the arrival back until all have.
 __device__ inline bool last_arrival(unsigned* counter, unsigned n) {
     __shared__ int s_last;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned before =
-            __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = before == n - 1;
-        if (before == n - 1)
-            __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (threadIdx.x == 0) s_last = atomicInc(counter, n - 1) == n - 1;
     __syncthreads();
     return s_last != 0;
 }

@@ -34,12 +34,6 @@ __device__ inline void st4u(float* p, float4 v) {
 }
 
 constexpr int kLine = 32;  // floats per 128-byte line
-// Updates of more than this are read with the non-temporal hint: a C that
-// outgrows the caches gains by it (10007 x 8191, 328 MB: 113.5 against 121.5
-// us), one that a later pass finds in the 256 MB last-level cache loses
-// (3001 x 2003, 24 MB: 10.1 against 8.7 us); 2000 x 15000 (120 MB): equal.
-constexpr int64_t kStreamBytes = (int64_t)96 << 20;
-
 // Floats from p to the next 128-byte line: the head of a row, which is written
 // element by element so that the 128-bit groups after it fill whole lines.
 // A 1 KB wavefront store that starts inside a line leaves two lines of every

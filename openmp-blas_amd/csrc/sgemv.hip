@@ -10,7 +10,8 @@
 // consecutive rows (one 128-bit load per column).  Tall matrices of whole
 // 64-row blocks and 256-column rounds run in one pass of 64-row workgroups;
 // otherwise the columns are split into chunks across workgroups, each chunk
-// writes a partial y, and a second kernel adds the partials in chunk order.
+// writes a partial y, and a row block's last workgroup to arrive adds its
+// partials in chunk order.
 // The result depends only on (M, N) and the device's CU count, never on
 // scheduling.
 #include <algorithm>
@@ -45,94 +46,146 @@ __global__ __launch_bounds__(NT) void sgemv_row_kernel(int64_t M, int64_t N, flo
     }
 }
 
-constexpr int COL_ROWS = 256;     // rows per workgroup: 4 per lane, one float4 per column
-constexpr int COL_UNROLL = 16;    // columns in flight per wavefront (16 KB per wavefront)
+// Sums over a row block's chunks, in chunk order: a thread per row and group of
+// chunks (the RB rows' NT / RB groups are added in group order), 16 loads in
+// flight.  Thread t < RB returns row r0 + t's sum.
+template <int RB, typename Load>
+__device__ __forceinline__ float col_chunk_sum(int64_t r0, int64_t M, const float* partial,
+                                               int64_t mpad, int nchunks, Load load) {
+    constexpr int G = NT / RB, U = 16;
+    const int per = (nchunks + G - 1) / G;
+    const int beg = (int)threadIdx.x / RB * per, end = min(nchunks, beg + per);
+    const float* p = partial + std::min<int64_t>(r0 + threadIdx.x % RB, M - 1);
+    float sum = 0.f;
+    for (int c = beg; c < end; c += U) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = load(p + min(c + u, end - 1) * mpad);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (c + u < end) sum += v[u];
+    }
+    if constexpr (G > 1) {
+        __shared__ float s_group[NT];
+        s_group[threadIdx.x] = sum;
+        __syncthreads();
+        sum = s_group[threadIdx.x % RB];
+#pragma unroll
+        for (int g = 1; g < G; ++g) sum += s_group[g * RB + threadIdx.x % RB];
+    }
+    return sum;
+}
 
-// One lane's sums over columns c0+wave, c0+wave+4, ... < c1 of its 4 rows at
-// ap: FULL lanes (all 4 rows inside A) use 128-bit loads at any alignment,
-// the others guarded scalars (rows past `valid` read as 0).  Four
-// accumulator sets (column j + 4u goes to set u % 4) keep each FP32 running
-// sum to a quarter of the chunk; both forms add in the same order.
-template <bool FULL>
-__device__ __forceinline__ void col_lane_sums(const float* __restrict__ ap, int64_t lda,
-                                              const float* __restrict__ x, int64_t j, int64_t c1,
-                                              int valid, float (&acc)[4][4]) {
-    auto load = [&](int64_t col) -> float4 {
-        const float* c = ap + col * lda;
-        if (FULL) return ld4u_nt(c);
-        return make_float4(valid > 0 ? c[0] : 0.f, valid > 1 ? c[1] : 0.f,
-                           valid > 2 ? c[2] : 0.f, 0.f);
+// Column-major A, any shape: a workgroup owns RB = 4 * LR rows (LR lanes of a
+// wavefront along the rows, 4 consecutive rows and one 128-bit load per column
+// each; its 64 / LR lane groups and 4 wavefronts take interleaved columns) of
+// one chunk of columns, U loads in flight per lane.  The last rows' lanes are
+// moved back inside A (lanes that own a row twice hold the same sum), and the
+// columns past the chunk are clamped and zeroed, so no load is guarded.  The
+// scheduling barrier keeps every load of a round ahead of its FMAs: without
+// it the compiler consumed each as it came (9003 x 6001: 84 us instead of
+// 35).  Four accumulator sets (a lane's u-th column of a round goes to set u
+// % 4) keep each FP32 running sum short.  The launcher makes about one
+// workgroup per CU: fewer, longer column streams keep HBM pages open.
+// Workgroups of one XCD take neighbouring row blocks of a chunk, which share
+// the lines at their borders when columns do not start on lines.
+// Bound by HBM: 9003 x 6001 (216 MB, columns 4-byte aligned) 45 us with a
+// scalar loop over the last partial round and separate row guards, 35 us
+// (6.2 TB/s) so.
+// STREAM: A is read with the non-temporal hint.
+// TINY: fewer than 4 rows, loaded one by one (the last one repeated).
+// Chunks' sums of a row block are added in chunk order by its last workgroup
+// to arrive (count: the stream's arrival counters), or by
+// sgemv_col_combine_kernel where there are none.
+template <int LR, int U, bool STREAM, bool TINY = false>
+__global__ __launch_bounds__(NT) void sgemv_col_kernel(int64_t M, int64_t N, float alpha,
+                                                       const float* __restrict__ A, int64_t lda,
+                                                       const float* __restrict__ x, float beta,
+                                                       float* __restrict__ y, float* partial,
+                                                       int64_t mpad, int nrb, int nchunks,
+                                                       int64_t cols_per_chunk, unsigned* count) {
+    constexpr int CG = 64 / LR, STEP = 4 * CG, RB = 4 * LR;
+    const int64_t b = xcd_remap(blockIdx.x, (int64_t)gridDim.x);
+    const int rb = (int)(b % nrb), ch = (int)(b / nrb);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int cg = lane / LR;
+    const int64_t r0 = (int64_t)rb * RB;
+    const int64_t r = TINY ? 0 : std::min<int64_t>(r0 + 4 * (lane % LR), M - 4);
+    const int64_t c0 = ch * cols_per_chunk, c1 = std::min<int64_t>(N, c0 + cols_per_chunk);
+    const float* ap = A + r;
+    float acc[4][4] = {};
+    auto load = [&](int64_t col) {
+        const float* p = ap + col * lda;
+        if constexpr (TINY) return make_float4(p[0], p[M > 1 ? 1 : 0], p[M - 1], 0.f);
+        else return STREAM ? ld4u_nt(p) : ld4u(p);
     };
-    for (; j + 4 * (COL_UNROLL - 1) < c1; j += 4 * COL_UNROLL) {
-        float4 av[COL_UNROLL];
-        float xv[COL_UNROLL];
+    auto add = [&](const float4 (&av)[U], const float (&xv)[U]) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < COL_UNROLL; ++u) {
-            xv[u] = x[j + 4 * u];
-            av[u] = load(j + 4 * u);
-        }
-#pragma unroll
-        for (int u = 0; u < COL_UNROLL; ++u) {
+        for (int u = 0; u < U; ++u) {
             float* a = acc[u & 3];
             a[0] = fmaf(av[u].x, xv[u], a[0]);
             a[1] = fmaf(av[u].y, xv[u], a[1]);
             a[2] = fmaf(av[u].z, xv[u], a[2]);
             a[3] = fmaf(av[u].w, xv[u], a[3]);
         }
+    };
+    int64_t jr = c0;  // first column of the round
+    for (; jr + STEP * U <= c1; jr += STEP * U) {
+        const int64_t j = jr + wave * CG + cg;
+        float4 av[U];
+        float xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            xv[u] = x[j + STEP * u];
+            av[u] = load(j + STEP * u);
+        }
+        add(av, xv);
     }
-    for (int u = 0; j < c1; j += 4, ++u) {
-        const float xv = x[j];
-        const float4 av = load(j);
-        float* a = acc[u & 3];
-        a[0] = fmaf(av.x, xv, a[0]);
-        a[1] = fmaf(av.y, xv, a[1]);
-        a[2] = fmaf(av.z, xv, a[2]);
-        a[3] = fmaf(av.w, xv, a[3]);
+    if (jr < c1) {
+        const int64_t j = jr + wave * CG + cg;
+        float4 av[U];
+        float xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t c = std::min<int64_t>(j + STEP * u, c1 - 1);
+            xv[u] = x[c];
+            av[u] = load(c);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (j + STEP * u >= c1) {
+                xv[u] = 0.f;
+                av[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+        add(av, xv);
     }
-}
-
-// Column-major A: lane l of every wavefront owns rows r0 + 4l .. r0 + 4l + 3,
-// so each column is read as 1 KB contiguous per wavefront; the 4 wavefronts
-// of a workgroup take interleaved columns of the chunk and their partial
-// sums are added in LDS in wavefront order.  The launcher sizes the grid to
-// about one workgroup per CU: fewer, longer column streams keep HBM pages
-// open (measured 88% of peak at 16384^2 against 68% with 1024 workgroups).
-__global__ __launch_bounds__(NT) void sgemv_col_kernel(int64_t M, int64_t N, float alpha,
-                                                       const float* __restrict__ A, int64_t lda,
-                                                       const float* __restrict__ x, float beta,
-                                                       float* __restrict__ y, float* partial,
-                                                       int64_t mpad, int64_t cols_per_chunk,
-                                                       int nchunks) {
-    // the wavefront index is uniform: its column indices (and x) stay scalar
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t r0 = (int64_t)blockIdx.x * COL_ROWS, ch = blockIdx.y;
-    const int64_t c0 = ch * cols_per_chunk;
-    const int64_t c1 = std::min<int64_t>(N, c0 + cols_per_chunk);
-    const int64_t r = r0 + 4 * lane;  // this lane's 4 rows
-    float acc[4][4] = {};
-    if (r + 3 < M)
-        col_lane_sums<true>(A + r, lda, x, c0 + wave, c1, 4, acc);
-    else if (r < M)  // the lane holding the last 1-3 rows
-        col_lane_sums<false>(A + r, lda, x, c0 + wave, c1, (int)(M - r), acc);
-    // Wavefront partials -> LDS, summed in wavefront order (thread t: row r0 + t).
-    __shared__ float red[4][COL_ROWS];
+    // Lane sums -> LDS, added in (wavefront, lane group) order.
+    __shared__ float red[STEP][RB];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        red[wave][4 * lane + e] = ((acc[0][e] + acc[1][e]) + acc[2][e]) + acc[3][e];
+        if (r + e >= r0)
+            red[wave * CG + cg][r - r0 + e] = ((acc[0][e] + acc[1][e]) + acc[2][e]) + acc[3][e];
     __syncthreads();
     const int t = threadIdx.x;
     const int64_t row = r0 + t;
-    if (row >= M) return;
-    const float sum = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
-    if (nchunks == 1) {
-        float out = alpha * sum;
-        if (beta != 0.f) out += beta * y[row];
-        y[row] = out;
-        return;
+    const bool mine = t < RB && row < M;
+    float sum = 0.f;
+    if (mine) {
+        sum = red[0][t];
+#pragma unroll
+        for (int q = 1; q < STEP; ++q) sum += red[q][t];
     }
-    // Partial sum of this column chunk; sgemv_col_combine_kernel adds the
-    // chunks in order 0..nchunks-1.
-    partial[ch * mpad + row] = sum;
+    if (nchunks > 1) {
+        if (mine) {
+            if (count) agent_store(&partial[ch * mpad + row], sum);
+            else partial[ch * mpad + row] = sum;
+        }
+        if (!count || !last_arrival(count + rb * kArrivalStride, (unsigned)nchunks)) return;
+        sum = col_chunk_sum<RB>(r0, M, partial, mpad, nchunks,
+                                [](const float* p) { return agent_load(p); });
+    }
+    if (mine) y[row] = beta != 0.f ? alpha * sum + beta * y[row] : alpha * sum;
 }
 
 // Column-major A in one pass, for M a multiple of 64 with at least one
@@ -194,19 +247,53 @@ __global__ __launch_bounds__(NT) void sgemv_col_rows64_kernel(int64_t M, int64_t
     }
 }
 
-// y[r] = alpha * sum_c partial[c][r] + beta * y[r], chunks added in order
-// (one row per thread).
+// y = alpha * (sum over the chunks' partials) + beta * y, one row block of
+// sgemv_col_kernel per workgroup, in the same order.
+template <int RB>
 __global__ __launch_bounds__(NT) void sgemv_col_combine_kernel(int64_t M, float alpha,
                                                                const float* __restrict__ partial,
                                                                int64_t mpad, int nchunks,
                                                                float beta, float* __restrict__ y) {
-    const int64_t r = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (r >= M) return;
-    float t = 0.f;
-    for (int c = 0; c < nchunks; ++c) t += partial[(int64_t)c * mpad + r];
-    float out = alpha * t;
-    if (beta != 0.f) out += beta * y[r];
-    y[r] = out;
+    const int64_t r0 = (int64_t)blockIdx.x * RB, row = r0 + threadIdx.x;
+    const float sum = col_chunk_sum<RB>(r0, M, partial, mpad, nchunks,
+                                        [](const float* p) { return *p; });
+    if (threadIdx.x < RB && row < M)
+        y[row] = beta != 0.f ? alpha * sum + beta * y[row] : alpha * sum;
+}
+
+// Rows up to which 64-row blocks are used instead of 256-row ones: fewer row
+// blocks would leave as many chunks as CUs to add per row (100 x 14000: 55 us
+// with 219 chunks added by one thread per row).
+constexpr int64_t kColNarrow = 1024;
+
+template <int LR, int U, bool STREAM, bool TINY = false>
+omb_status launch_col(int64_t M, int64_t N, float alpha, const float* A, int64_t lda,
+                      const float* x, float beta, float* y, hipStream_t s) {
+    constexpr int RB = 4 * LR, QUANTUM = 4 * (64 / LR) * U;  // rows; columns of one round
+    const int64_t nrb = ceil_div(M, RB), cus = device_cu_count();
+    if (nrb > 0x7fffffffLL) {
+        set_error("sgemv: too many row blocks");
+        return OMB_EUNSUPPORTED;
+    }
+    // At most one workgroup per CU (a few more are a second round for some:
+    // 5000 x 12000 with 260 took 48.4 us), chunks of whole rounds.
+    const int64_t want = std::max<int64_t>(1, cus / nrb);
+    const int64_t rounds = ceil_div(N, QUANTUM);
+    const int64_t cpc = ceil_div(rounds, std::min(want, rounds)) * QUANTUM;
+    const int64_t nchunks = ceil_div(N, cpc);
+    const int64_t mpad = round_up(M, 4);
+    Workspace* ws = nullptr;
+    OMB_TRY(get_workspace(s, nchunks > 1 ? (size_t)(nchunks * mpad) * sizeof(float) : 0, &ws));
+    float* part = reinterpret_cast<float*>(ws->buf);
+    unsigned* count = nrb <= kArrivalCounters ? ws->arrivals : nullptr;
+    hipLaunchKernelGGL((sgemv_col_kernel<LR, U, STREAM, TINY>), dim3((unsigned)(nrb * nchunks)),
+                       dim3(NT), 0, s, M, N, alpha, A, lda, x, beta, y, part, mpad, (int)nrb,
+                       (int)nchunks, cpc, count);
+    if (nchunks > 1 && !count)
+        hipLaunchKernelGGL(sgemv_col_combine_kernel<RB>, dim3((unsigned)nrb), dim3(NT), 0, s, M,
+                           alpha, part, mpad, (int)nchunks, beta, y);
+    OMB_HIP_TRY(hipGetLastError());
+    return OMB_OK;
 }
 
 }  // namespace
@@ -248,30 +335,11 @@ omb_status launch_sgemv_col(int64_t M, int64_t N, float alpha, const float* A, i
         OMB_HIP_TRY(hipGetLastError());
         return OMB_OK;
     }
-    const int64_t nrb = ceil_div(M, COL_ROWS);
-    // About one workgroup per CU; every chunk at least 64 columns (one
-    // unrolled step of the 4 wavefronts).
-    int64_t nchunks = nrb >= cus ? 1 : cus / nrb;
-    nchunks = std::max<int64_t>(1, std::min<int64_t>(nchunks, ceil_div(N, 4 * COL_UNROLL)));
-    if (N == 0) nchunks = 1;
-    const int64_t cpc = N > 0 ? ceil_div(N, nchunks) : 0;
-    nchunks = N > 0 ? ceil_div(N, cpc) : 1;
-    if (nrb > 0x7fffffffLL) {
-        set_error("sgemv: too many row blocks");
-        return OMB_EUNSUPPORTED;
-    }
-    const int64_t mpad = round_up(M, 4);
-    Workspace* ws = nullptr;
-    OMB_TRY(get_workspace(s, nchunks > 1 ? (size_t)(nchunks * mpad) * sizeof(float) : 0, &ws));
-    dim3 grid((unsigned)nrb, (unsigned)nchunks);
-    float* part = reinterpret_cast<float*>(ws->buf);
-    hipLaunchKernelGGL(sgemv_col_kernel, grid, dim3(NT), 0, s, M, N, alpha, A, lda, x, beta, y,
-                       part, mpad, cpc, (int)nchunks);
-    if (nchunks > 1)
-        hipLaunchKernelGGL(sgemv_col_combine_kernel, dim3((unsigned)ceil_div(M, NT)),
-                           dim3(NT), 0, s, M, alpha, part, mpad, (int)nchunks, beta, y);
-    OMB_HIP_TRY(hipGetLastError());
-    return OMB_OK;
+    if (M < 4) return launch_col<1, 4, false, true>(M, N, alpha, A, lda, x, beta, y, s);
+    if (M <= kColNarrow) return launch_col<16, 8, false>(M, N, alpha, A, lda, x, beta, y, s);
+    if (M * N * (int64_t)sizeof(float) <= kStreamBytes)
+        return launch_col<64, 16, false>(M, N, alpha, A, lda, x, beta, y, s);
+    return launch_col<64, 16, true>(M, N, alpha, A, lda, x, beta, y, s);
 }
 
 }  // namespace omb
