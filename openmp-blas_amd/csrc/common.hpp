@@ -73,6 +73,7 @@ omb_status resolve_layout(const char* name, int64_t rows, int64_t cols, int64_t 
 // (update of 3001 x 2003, 24 MB: 10.1 against 8.7 us; GEMV of 3000^2: 9.1
 // against 7.3); an update of 120 MB: equal.
 constexpr int64_t kStreamBytes = (int64_t)96 << 20;
+constexpr int kLineFloats = 32;  // floats per 128-byte line
 
 // ------------------------------------------------------------ kernels -----
 // Plain FP32 SGEMM, row-major C (ldc), A K-contiguous iff a_kc, B N-contiguous

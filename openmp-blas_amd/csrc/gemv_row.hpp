@@ -3,12 +3,13 @@
 // standalone row kernel and the grouped persistent kernel so that both give
 // bitwise the same y: lane j accumulates the 4-float column groups j, j+64,
 // ... in order (128-bit loads at any alignment), then the N % 4 trailing
-// columns (lanes 0..2), and a fixed butterfly adds the lanes.  ROWS and
-// UNROLL change only how many loads are in flight and OFF32 only how their
+// columns (lanes 0..2), and a fixed butterfly adds the lanes.  ROWS, UNROLL
+// and BATCH change only how many loads are in flight and OFF32 only how their
 // addresses are formed, never a row's order of accumulation, and neither
 // does the alignment of A, lda or x.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -36,9 +37,15 @@ constexpr int64_t kGemvOff32Cols = (int64_t)1 << 29;
 // a wavefront-uniform r0: the row bases are scalar and every load adds one
 // 32-bit lane offset, which frees about 90 VGPRs of per-row addresses and
 // measured 1.5% more bandwidth in the standalone row kernel, 0.8% in the
-// grouped kernel's GEMV items.)
-template <int ROWS, int UNROLL, bool STREAM, bool OFF32 = false, typename PA, typename PX,
-          typename PY>
+// grouped kernel's GEMV items.  BATCH: a scheduling barrier keeps all ROWS *
+// UNROLL loads of a round ahead of its FMAs, and the last, partial round is
+// one round too, its loads past the row clamped and left out of the sums;
+// without it the compiler consumes loads as they come and the last groups
+// are one round trip each (9003 x 6001 with 2 x 8: 34.7 us, 4 x 4 without
+// BATCH: 43.1).  The 16 x 1 form is the exception: its rounds overlap without
+// a barrier.)
+template <int ROWS, int UNROLL, bool STREAM, bool OFF32 = false, bool BATCH = false, typename PA,
+          typename PX, typename PY>
 __device__ __forceinline__ void gemv_rows_wave(int64_t r0, int nr, int64_t N, float alpha,
                                                PA __restrict__ A, int64_t lda,
                                                PX __restrict__ x, float beta,
@@ -60,7 +67,8 @@ __device__ __forceinline__ void gemv_rows_wave(int64_t r0, int nr, int64_t N, fl
     if constexpr (OFF32) x = wave_uniform_ptr(x);
     const Idx n4 = (Idx)(N >> 2);
     Idx j = lane;
-    for (; j + 64 * (UNROLL - 1) < n4; j += 64 * UNROLL) {
+    // BATCH: every lane of the wavefront takes part in the same rounds
+    for (; (BATCH ? j - lane + 64 * UNROLL <= n4 : j + 64 * (UNROLL - 1) < n4); j += 64 * UNROLL) {
         float4 xv[UNROLL];
         float4 av[ROWS][UNROLL];
 #pragma unroll
@@ -72,17 +80,39 @@ __device__ __forceinline__ void gemv_rows_wave(int64_t r0, int nr, int64_t N, fl
                 const auto p = at(ar[r], j + 64 * u);
                 av[r][u] = STREAM ? ld4u_nt(p) : ld4u(p);
             }
+        if constexpr (BATCH) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) acc[r] = dot4(av[r][u], xv[u], acc[r]);
     }
-    for (; j < n4; j += 64) {
-        const float4 xv = ld4u(at(x, j));
+    if constexpr (BATCH) {
+        if (j - lane < n4) {
+            float4 xv[UNROLL];
+            float4 av[ROWS][UNROLL];
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            const auto p = at(ar[r], j);
-            acc[r] = dot4(STREAM ? ld4u_nt(p) : ld4u(p), xv, acc[r]);
+            for (int u = 0; u < UNROLL; ++u)
+                xv[u] = ld4u(at(x, std::min<Idx>(j + 64 * u, n4 - 1)));
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+                for (int u = 0; u < UNROLL; ++u)
+                    av[r][u] = ld4u(at(ar[r], std::min<Idx>(j + 64 * u, n4 - 1)));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r)
+                    if (j + 64 * u < n4) acc[r] = dot4(av[r][u], xv[u], acc[r]);
+        }
+    } else {
+        for (; j < n4; j += 64) {
+            const float4 xv = ld4u(at(x, j));
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                const auto p = at(ar[r], j);
+                acc[r] = dot4(STREAM ? ld4u_nt(p) : ld4u(p), xv, acc[r]);
+            }
         }
     }
     const Idx t = (n4 << 2) + lane;

@@ -33,7 +33,7 @@ __device__ inline void st4u(float* p, float4 v) {
     __builtin_nontemporal_store(t, reinterpret_cast<f32x4_u*>(p));
 }
 
-constexpr int kLine = 32;  // floats per 128-byte line
+constexpr int kLine = kLineFloats;
 // Floats from p to the next 128-byte line: the head of a row, which is written
 // element by element so that the 128-bit groups after it fill whole lines.
 // A 1 KB wavefront store that starts inside a line leaves two lines of every

@@ -23,11 +23,10 @@ namespace {
 
 constexpr int NT = 256;
 
-// Rows per wavefront and 128-bit loads in flight per row: 16 rows (one
-// workgroup per CU at 16384 rows, measured 86% of HBM peak) for tall
-// matrices, fewer rows per wavefront when that would leave CUs idle.  A
-// row's order of accumulation is the same for every choice.
-template <int ROWS, int UNROLL, bool OFF32 = false>
+// Rows per wavefront, 128-bit loads in flight per row and the form of the loop
+// (gemv_row.hpp); the launcher chooses them.  A row's order of accumulation is
+// the same for every choice.
+template <int ROWS, int UNROLL, bool STREAM, bool OFF32, bool BATCH>
 __global__ __launch_bounds__(NT) void sgemv_row_kernel(int64_t M, int64_t N, float alpha,
                                                        const float* __restrict__ A, int64_t lda,
                                                        const float* __restrict__ x, float beta,
@@ -42,7 +41,7 @@ __global__ __launch_bounds__(NT) void sgemv_row_kernel(int64_t M, int64_t N, flo
          w * ROWS < M; w += waves) {
         const int64_t r0 = w * ROWS;
         const int nr = (int)std::min<int64_t>(ROWS, M - r0);
-        gemv_rows_wave<ROWS, UNROLL, true, OFF32>(r0, nr, N, alpha, A, lda, x, beta, y, lane);
+        gemv_rows_wave<ROWS, UNROLL, STREAM, OFF32, BATCH>(r0, nr, N, alpha, A, lda, x, beta, y, lane);
     }
 }
 
@@ -298,29 +297,45 @@ omb_status launch_col(int64_t M, int64_t N, float alpha, const float* A, int64_t
 
 }  // namespace
 
+// Rows of up to this many columns take 4 rows x 2 loads per wavefront (more
+// loads per row would be past its end: 16000 x 600 9.6 us with 2 x 8, 8.7 us).
+constexpr int64_t kRowShort = 1024;
+
 omb_status launch_sgemv_row(int64_t M, int64_t N, float alpha, const float* A, int64_t lda,
                             const float* x, float beta, float* y, hipStream_t s) {
     if (M <= 0) return OMB_OK;
     const int64_t cus = device_cu_count();
     const int64_t waves_per_wg = NT / 64;
-    int rows = 16;
-    if (M < 16 * waves_per_wg * cus) rows = M < 4 * waves_per_wg * cus ? 1 : 4;
-    // one workgroup per CU for 16-row groups, up to 4 for the smaller ones
-    const int64_t blocks = std::min<int64_t>(ceil_div(ceil_div(M, rows), waves_per_wg),
-                                             rows == 16 ? cus : 4 * cus);
-    const dim3 grid((unsigned)blocks), block(NT);
-    if (rows == 16 && N < kGemvOff32Cols)
-        hipLaunchKernelGGL((sgemv_row_kernel<16, 1, true>), grid, block, 0, s, M, N, alpha, A, lda,
-                           x, beta, y);
-    else if (rows == 16)
-        hipLaunchKernelGGL((sgemv_row_kernel<16, 1>), grid, block, 0, s, M, N, alpha, A, lda, x,
+    // Tall matrices whose rows start on lines: 16 rows x 1 load, one workgroup
+    // per CU (16384^2: 153.4 us, 7.0 TB/s; 8 rows 160).  Rows that do not:
+    // 16384 x 9001 took 101 us so, 87.7 with 2 rows x 8 loads in batches.
+    // Otherwise batches over 2 rows, or over one where 2 would leave fewer than
+    // 3 workgroups per CU (5000 x 12000: 42.1 and 39.8 us), of 8 loads per row
+    // where A streams from memory and of 4 where it may be cached, since a
+    // shorter batch wastes less of a row's last round (6000 x 4001: 17.1 and
+    // 15.9 us).  Before: 4 rows x 4 loads, consumed as they came (50.5 us for
+    // 5000 x 12000, 43.1 -> 35.4 for 9003 x 6001, 20.9 for 6000 x 4001).
+    const int64_t tall = 16 * waves_per_wg * cus;
+    const bool stream = M * N * (int64_t)sizeof(float) > kStreamBytes;
+    auto launch = [&](auto kernel, int rows, int64_t most) {
+        const int64_t blocks = std::min<int64_t>(ceil_div(ceil_div(M, rows), waves_per_wg), most);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(NT), 0, s, M, N, alpha, A, lda, x,
                            beta, y);
-    else if (rows == 4)
-        hipLaunchKernelGGL((sgemv_row_kernel<4, 4>), grid, block, 0, s, M, N, alpha, A, lda, x,
-                           beta, y);
-    else
-        hipLaunchKernelGGL((sgemv_row_kernel<1, 8>), grid, block, 0, s, M, N, alpha, A, lda, x,
-                           beta, y);
+    };
+    if (N >= kGemvOff32Cols) {
+        if (M >= tall) launch(sgemv_row_kernel<16, 1, true, false, false>, 16, cus);
+        else launch(sgemv_row_kernel<1, 8, true, false, true>, 1, 4 * cus);
+    } else if (M >= tall && lda % kLineFloats == 0) {
+        launch(sgemv_row_kernel<16, 1, true, true, false>, 16, cus);
+    } else if (N <= kRowShort) {
+        launch(sgemv_row_kernel<4, 2, false, true, true>, 4, 4 * cus);
+    } else if (M < 6 * waves_per_wg * cus) {
+        launch(stream ? sgemv_row_kernel<1, 8, true, true, true>
+                      : sgemv_row_kernel<1, 4, false, true, true>, 1, 4 * cus);
+    } else {
+        launch(stream ? sgemv_row_kernel<2, 8, true, true, true>
+                      : sgemv_row_kernel<2, 4, false, true, true>, 2, 4 * cus);
+    }
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
