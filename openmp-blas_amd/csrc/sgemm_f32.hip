@@ -11,6 +11,17 @@
 // every thread keeps a (BM/16) x (BN/16) register micro-tile.  Global loads
 // run two slices ahead in registers and LDS fragments one k ahead.
 //
+// What bounds it: the issue of v_fmac_f32, 128 per CU and clock.  Two things
+// keep the k loop near it (4096^3 in us by layout of A and B, row.row, col.row,
+// row.col, col.col: 1538 1539 1453 1547 without them, 1429 1423 1447 1436 with):
+//  - every full slice of every tile is read with unguarded 128-bit loads at any
+//    alignment, addressed by a uniform base and 32-bit byte offsets (see Side);
+//    ragged tiles took guarded loads before, 1.05-1.36x the time;
+//  - an accumulator never lies in the register bank of the B value it is
+//    multiplied with (registers r and r + 4n share a bank, and a v_fmac with two
+//    operands in one bank takes a cycle more): the four accumulators of a B quad
+//    are one 4-register tuple, rotated by one against the quad (acc_slot).
+//
 // Accumulation order: each thread sums 128 consecutive k (8 LDS slices) into
 // an inner register tile, then adds it to an outer tile -- the same for every
 // tile class, so the class never changes an output's bits.  This two-level sum
@@ -64,109 +75,78 @@ struct Args {
     float* part;     // split partial sums [split][M][N], or null (one split)
 };
 
-// Load up to 4 consecutive floats starting at p (n valid, 0..4); zero-fill.
-template <bool VEC>
-__device__ inline float4 load4(const float* p, int n) {
-    if (VEC && n == 4) return *reinterpret_cast<const float4*>(p);
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (n > 0) v.x = p[0];
-    if (n > 1) v.y = p[1];
-    if (n > 2) v.z = p[2];
-    if (n > 3) v.w = p[3];
-    return v;
-}
+// The four columns of a quad lie in its accumulator tuple one place further on:
+// register tuples start on even registers, so with the odd rotation a column
+// of B and its accumulators are never in one bank.
+typedef float acc4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ constexpr int acc_slot(int j) { return (j + 1) & 3; }
 
-__device__ inline int clamp4(int64_t r) { return r <= 0 ? 0 : (r >= 4 ? 4 : (int)r); }
+// One operand's side of a workgroup's tile: E lines (rows of A or columns of
+// B) from line e0 of the operand; KC: k is the unit stride, else the line is.
+// Its 16-k slices are read with 128-bit loads along the unit stride at any
+// alignment, whose lines are clamped into the operand instead of guarded: what
+// the repeated lines give is never stored, so every full slice of every tile,
+// ragged or not, takes the same unguarded loads.  A thread's loads are byte
+// offsets from the slice's first element, of 32 bits unless the leading
+// dimension is too long for that (fits32).
+template <int E, bool KC, typename Off>
+struct Side {
+    static constexpr int L = E / 64;  // float4 per thread and slice
+    const float* p;                   // line e0, this split's first k
+    int64_t ld;
+    int n;                            // lines from e0 inside the operand, at most E
+    Off off[L];                       // this thread's loads of a slice, in bytes
 
-// Global -> registers for one BK slice of a BM x BN tile: LA = BM/64 float4
-// of A and LB = BN/64 float4 of B per thread, each along the operand's
-// unit-stride dimension.
-// FULL: the slice lies wholly inside A and B and the operands are 16-byte
-// aligned, so every load is an unguarded float4.
-template <int BM, int BN, bool A_KC, bool B_NC, bool VEC, bool FULL = false>
-__device__ inline void load_slice(const Args& p, int64_t m0, int64_t n0, int64_t k0, int tid,
-                                  float4 (&ra)[BM / 64], float4 (&rb)[BN / 64]) {
+    __device__ __forceinline__ void init(const float* X, int64_t ld_, int64_t e0, int64_t lines,
+                                         int64_t kbeg, int tid) {
+        ld = ld_;
+        p = X + (KC ? e0 * ld + kbeg : e0 + kbeg * ld);
+        n = (int)std::min<int64_t>(lines - e0, E);
 #pragma unroll
-    for (int i = 0; i < BM / 64; ++i) {
-        const int e = tid + i * NT;
-        if (A_KC) {  // A[m*lda + k]: float4 along k
-            int row = e >> 2, kq = (e & 3) * 4;
-            int64_t m = m0 + row, k = k0 + kq;
-            if constexpr (FULL) {
-                ra[i] = *reinterpret_cast<const float4*>(p.A + m * p.lda + k);
-            } else {
-                int n = m < p.M ? clamp4(p.K - k) : 0;
-                ra[i] = load4<VEC>(p.A + (n ? m * p.lda + k : 0), n);
-            }
-        } else {     // A[k*lda + m]: float4 along m
-            int mq = (e % (BM / 4)) * 4, kk = e / (BM / 4);
-            int64_t m = m0 + mq, k = k0 + kk;
-            if constexpr (FULL) {
-                ra[i] = *reinterpret_cast<const float4*>(p.A + k * p.lda + m);
-            } else {
-                int n = k < p.K ? clamp4(p.M - m) : 0;
-                ra[i] = load4<VEC>(p.A + (n ? k * p.lda + m : 0), n);
-            }
+        for (int i = 0; i < L; ++i) {
+            const int e = tid + i * NT;
+            off[i] = (Off)(4 * (KC ? min(e >> 2, n - 1) * ld + (e & 3) * 4
+                                   : (e / (E / 4)) * ld + min(e % (E / 4) * 4, (n - 1) & ~3)));
         }
     }
+    // k steps at the operand's end that a 4-line load could read past: the
+    // last one, or the last three when lines are less than 4 floats apart.
+    __device__ __forceinline__ int tail() const {
+        return KC || n % 4 == 0 ? 0 : (ld < 4 ? 3 : 1);
+    }
+    __device__ __forceinline__ void load(float4 (&v)[L], int64_t k0) const {
+        const char* q = reinterpret_cast<const char*>(p + (KC ? k0 : k0 * ld));
 #pragma unroll
-    for (int i = 0; i < BN / 64; ++i) {
-        const int e = tid + i * NT;
-        if (B_NC) {  // B[k*ldb + n]: float4 along n
-            int nq = (e % (BN / 4)) * 4, kk = e / (BN / 4);
-            int64_t nn = n0 + nq, k = k0 + kk;
-            if constexpr (FULL) {
-                rb[i] = *reinterpret_cast<const float4*>(p.B + k * p.ldb + nn);
+        for (int i = 0; i < L; ++i) v[i] = ld4u(reinterpret_cast<const float*>(q + off[i]));
+    }
+    // Registers -> LDS, laid out [k][line].
+    __device__ __forceinline__ void store(float (*s)[E + PAD], const float4 (&v)[L], int tid) const {
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int e = tid + i * NT;
+            if (KC) {
+                const int line = e >> 2, kq = (e & 3) * 4;
+                s[kq + 0][line] = v[i].x;
+                s[kq + 1][line] = v[i].y;
+                s[kq + 2][line] = v[i].z;
+                s[kq + 3][line] = v[i].w;
             } else {
-                int n = k < p.K ? clamp4(p.N - nn) : 0;
-                rb[i] = load4<VEC>(p.B + (n ? k * p.ldb + nn : 0), n);
-            }
-        } else {     // B[n*ldb + k]: float4 along k
-            int col = e >> 2, kq = (e & 3) * 4;
-            int64_t nn = n0 + col, k = k0 + kq;
-            if constexpr (FULL) {
-                rb[i] = *reinterpret_cast<const float4*>(p.B + nn * p.ldb + k);
-            } else {
-                int n = nn < p.N ? clamp4(p.K - k) : 0;
-                rb[i] = load4<VEC>(p.B + (n ? nn * p.ldb + k : 0), n);
+                *reinterpret_cast<float4*>(&s[e / (E / 4)][e % (E / 4) * 4]) = v[i];
             }
         }
     }
-}
-
-// Registers -> LDS, laid out [k][m] and [k][n].
-template <int BM, int BN, bool A_KC, bool B_NC>
-__device__ inline void store_slice(float (*As)[BM + PAD], float (*Bs)[BN + PAD], int tid,
-                                   const float4 (&ra)[BM / 64], const float4 (&rb)[BN / 64]) {
-#pragma unroll
-    for (int i = 0; i < BM / 64; ++i) {
-        const int e = tid + i * NT;
-        if (A_KC) {
-            int row = e >> 2, kq = (e & 3) * 4;
-            As[kq + 0][row] = ra[i].x;
-            As[kq + 1][row] = ra[i].y;
-            As[kq + 2][row] = ra[i].z;
-            As[kq + 3][row] = ra[i].w;
-        } else {
-            int mq = (e % (BM / 4)) * 4, kk = e / (BM / 4);
-            *reinterpret_cast<float4*>(&As[kk][mq]) = ra[i];
+    // The slice at k0 with kn valid k, element by element: zeros past them.
+    __device__ __forceinline__ void stage_tail(float (*s)[E + PAD], int64_t k0, int kn, int tid) const {
+#pragma unroll 4
+        for (int e = tid; e < E * BK; e += NT) {
+            const int line = KC ? e / BK : e % E, k = KC ? e % BK : e / E;
+            const int a = min(line, n - 1);
+            const int64_t b = k0 + min(k, kn - 1);
+            const float x = p[KC ? a * ld + b : b * ld + a];
+            s[k][line] = k < kn ? x : 0.f;
         }
     }
-#pragma unroll
-    for (int i = 0; i < BN / 64; ++i) {
-        const int e = tid + i * NT;
-        if (B_NC) {
-            int nq = (e % (BN / 4)) * 4, kk = e / (BN / 4);
-            *reinterpret_cast<float4*>(&Bs[kk][nq]) = rb[i];
-        } else {
-            int col = e >> 2, kq = (e & 3) * 4;
-            Bs[kq + 0][col] = rb[i].x;
-            Bs[kq + 1][col] = rb[i].y;
-            Bs[kq + 2][col] = rb[i].z;
-            Bs[kq + 3][col] = rb[i].w;
-        }
-    }
-}
+};
 
 // Workgroups per CU each class is built for: the 128x128 class holds 2 x 64
 // accumulators per thread (2 workgroups per CU), 128x64 2 x 32 (3), 64x64
@@ -177,9 +157,9 @@ constexpr int occ_of(int tile_elems) {
 
 // Thread (ty, tx) of the 16 x 16 grid owns rows {g*64 + ty*4 + i} (g < GR =
 // BM/64, i < 4) and columns {h*64 + tx*4 + j} (h < GC = BN/64, j < 4).
-template <int BM, int BN, bool A_KC, bool B_NC, bool VEC>
+template <int BM, int BN, bool A_KC, bool B_NC, typename Off>
 __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) {
-    constexpr int GR = BM / 64, GC = BN / 64, TR = 4 * GR, TC = 4 * GC;
+    constexpr int GR = BM / 64, GC = BN / 64, TR = 4 * GR;
     __shared__ float As[2][BK][BM + PAD];
     __shared__ float Bs[2][BK][BN + PAD];
 
@@ -188,12 +168,8 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
     // a multiple of INNER_K, so the 128-k accumulation blocks are the same
     // as without the split.
     Args p = q;
-    const int64_t kbeg = (int64_t)blockIdx.y * q.kchunk;
-    if (q.part) {
-        p.K = q.K - kbeg < q.kchunk ? q.K - kbeg : q.kchunk;
-        p.A = q.A + (A_KC ? kbeg : kbeg * q.lda);
-        p.B = q.B + (B_NC ? kbeg * q.ldb : kbeg);
-    }
+    const int64_t kbeg = q.part ? (int64_t)blockIdx.y * q.kchunk : 0;
+    if (q.part) p.K = q.K - kbeg < q.kchunk ? q.K - kbeg : q.kchunk;
 
     const int tid = threadIdx.x;
     const int64_t ntiles = p.tiles_m * p.tiles_n;
@@ -203,11 +179,11 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
     const int64_t m0 = tm * BM, n0 = tn * BN;
 
     const int tx = tid & 15, ty = tid >> 4;
-    float inner[TR][TC], outer[TR][TC];
+    acc4 inner[TR][GC], outer[TR][GC];
 #pragma unroll
     for (int i = 0; i < TR; ++i)
 #pragma unroll
-        for (int j = 0; j < TC; ++j) inner[i][j] = outer[i][j] = 0.f;
+        for (int h = 0; h < GC; ++h) inner[i][h] = outer[i][h] = acc4{0.f, 0.f, 0.f, 0.f};
 
     const int64_t nk = ceil_div(p.K, BK);
     constexpr int kFold = INNER_K / BK;
@@ -227,78 +203,91 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
 #pragma unroll
         for (int k = 0; k < BK; ++k) {
             if (k + 1 < BK) fragment(k + 1, (k + 1) & 1);
-            float a[TR], b[TC];
+            float a[TR];
 #pragma unroll
             for (int g = 0; g < GR; ++g) {
                 const float4 v = fa[k & 1][g];
                 a[4 * g] = v.x; a[4 * g + 1] = v.y; a[4 * g + 2] = v.z; a[4 * g + 3] = v.w;
             }
 #pragma unroll
-            for (int h = 0; h < GC; ++h) {
-                const float4 v = fb[k & 1][h];
-                b[4 * h] = v.x; b[4 * h + 1] = v.y; b[4 * h + 2] = v.z; b[4 * h + 3] = v.w;
-            }
-#pragma unroll
             for (int i = 0; i < TR; ++i)
 #pragma unroll
-                for (int j = 0; j < TC; ++j) inner[i][j] = fmaf(a[i], b[j], inner[i][j]);
+                for (int h = 0; h < GC; ++h) {
+                    const float4 v = fb[k & 1][h];
+                    acc4& s = inner[i][h];
+                    s[acc_slot(0)] = fmaf(a[i], v.x, s[acc_slot(0)]);
+                    s[acc_slot(1)] = fmaf(a[i], v.y, s[acc_slot(1)]);
+                    s[acc_slot(2)] = fmaf(a[i], v.z, s[acc_slot(2)]);
+                    s[acc_slot(3)] = fmaf(a[i], v.w, s[acc_slot(3)]);
+                }
         }
         if ((kt + 1) % kFold == 0 || kt + 1 == nk) {
 #pragma unroll
             for (int i = 0; i < TR; ++i)
 #pragma unroll
-                for (int j = 0; j < TC; ++j) {
-                    outer[i][j] += inner[i][j];
-                    inner[i][j] = 0.f;
+                for (int h = 0; h < GC; ++h) {
+                    outer[i][h] += inner[i][h];
+                    inner[i][h] = acc4{0.f, 0.f, 0.f, 0.f};
                 }
         }
     };
-    float4 ra0[GR], rb0[GC], ra1[GR], rb1[GC];
-    const bool full = VEC && m0 + BM <= p.M && n0 + BN <= p.N && p.K > 0 && p.K % BK == 0;
-    if (VEC && full) {
-        // Interior tile: unguarded loads with the slice index clamped to the
-        // last one, whole slice pairs, an odd last slice after the loop.  One
-        // path through the loop keeps the compiler's wait counts exact (a
-        // store waits only for its own loads), so the loads stay two slices
-        // ahead.  Same slices and fold order as the guarded loop below.
-        const int64_t klast = nk - 1;
-        auto kc = [&](int64_t k) { return k < klast ? k : klast; };
-        load_slice<BM, BN, A_KC, B_NC, VEC, true>(p, m0, n0, 0, tid, ra0, rb0);
-        store_slice<BM, BN, A_KC, B_NC>(As[0], Bs[0], tid, ra0, rb0);
-        load_slice<BM, BN, A_KC, B_NC, VEC, true>(p, m0, n0, kc(1) * BK, tid, ra1, rb1);
+    // The slices whose loads cannot pass an operand's end, then the rest (K's
+    // last partial slice, or the last one of a tile with a partial quad of
+    // lines) element by element.
+    Side<BM, A_KC, Off> sa;
+    Side<BN, !B_NC, Off> sb;
+    sa.init(p.A, p.lda, m0, p.M, kbeg, tid);
+    sb.init(p.B, p.ldb, n0, p.N, kbeg, tid);
+    const int tail = kbeg + p.K == q.K ? max(sa.tail(), sb.tail()) : 0;
+    const int64_t nfull = p.K > tail ? (p.K - tail) / BK : 0;
+    int64_t kt = 0;
+    if (nfull > 0) {
+        // Slices kt and kt+1 in LDS buffers 0 and 1, loads two slices ahead in
+        // two register sets with the slice index clamped to the last one, in
+        // whole slice pairs: one path through the loop keeps the compiler's
+        // wait counts exact (a store waits only for its own loads).
+        float4 ra0[sa.L], rb0[sb.L], ra1[sa.L], rb1[sb.L];
+        const int64_t klast = nfull - 1;
+        auto kc = [&](int64_t k) { return (k < klast ? k : klast) * BK; };
+        sa.load(ra0, 0);
+        sb.load(rb0, 0);
+        sa.store(As[0], ra0, tid);
+        sb.store(Bs[0], rb0, tid);
+        sa.load(ra1, kc(1));
+        sb.load(rb1, kc(1));
         __syncthreads();
-        int64_t kt = 0;
-        for (; kt + 1 < nk; kt += 2) {
-            load_slice<BM, BN, A_KC, B_NC, VEC, true>(p, m0, n0, kc(kt + 2) * BK, tid, ra0, rb0);
+        for (; kt + 1 < nfull; kt += 2) {
+            // Keeps each tuple in four consecutive registers through the loop.
+#pragma unroll
+            for (int i = 0; i < TR; ++i)
+#pragma unroll
+                for (int h = 0; h < GC; ++h) asm volatile("" : "+v"(inner[i][h]));
+            sa.load(ra0, kc(kt + 2));
+            sb.load(rb0, kc(kt + 2));
             __builtin_amdgcn_sched_barrier(0);
             compute(0, kt);
-            store_slice<BM, BN, A_KC, B_NC>(As[1], Bs[1], tid, ra1, rb1);
+            sa.store(As[1], ra1, tid);
+            sb.store(Bs[1], rb1, tid);
             __syncthreads();
-            load_slice<BM, BN, A_KC, B_NC, VEC, true>(p, m0, n0, kc(kt + 3) * BK, tid, ra1, rb1);
+            sa.load(ra1, kc(kt + 3));
+            sb.load(rb1, kc(kt + 3));
             __builtin_amdgcn_sched_barrier(0);
             compute(1, kt + 1);
-            store_slice<BM, BN, A_KC, B_NC>(As[0], Bs[0], tid, ra0, rb0);
+            sa.store(As[0], ra0, tid);
+            sb.store(Bs[0], rb0, tid);
             __syncthreads();
         }
-        if (kt < nk) compute(0, kt);
-    } else {
-        load_slice<BM, BN, A_KC, B_NC, VEC>(p, m0, n0, 0, tid, ra0, rb0);
-        store_slice<BM, BN, A_KC, B_NC>(As[0], Bs[0], tid, ra0, rb0);
-        if (nk > 1) load_slice<BM, BN, A_KC, B_NC, VEC>(p, m0, n0, BK, tid, ra1, rb1);
+    }
+    // Buffer 0 holds an odd last full slice, if there is one.
+    for (; kt < nk; ++kt) {
+        if (kt >= nfull) {
+            const int kn = (int)std::min<int64_t>(BK, p.K - kt * BK);
+            sa.stage_tail(As[0], kt * BK, kn, tid);
+            sb.stage_tail(Bs[0], kt * BK, kn, tid);
+            __syncthreads();
+        }
+        compute(0, kt);
         __syncthreads();
-        for (int64_t kt = 0; kt < nk; kt += 2) {
-            if (kt + 2 < nk)
-                load_slice<BM, BN, A_KC, B_NC, VEC>(p, m0, n0, (kt + 2) * BK, tid, ra0, rb0);
-            compute(0, kt);
-            if (kt + 1 < nk) store_slice<BM, BN, A_KC, B_NC>(As[1], Bs[1], tid, ra1, rb1);
-            __syncthreads();
-            if (kt + 1 >= nk) break;
-            if (kt + 3 < nk)
-                load_slice<BM, BN, A_KC, B_NC, VEC>(p, m0, n0, (kt + 3) * BK, tid, ra1, rb1);
-            compute(1, kt + 1);
-            if (kt + 2 < nk) store_slice<BM, BN, A_KC, B_NC>(As[0], Bs[0], tid, ra0, rb0);
-            __syncthreads();
-        }
     }
 
     // Epilogue: rows {g*64 + ty*4 + i}, columns {h*64 + tx*4 + j}.
@@ -314,12 +303,13 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
                 const int64_t n = n0 + h * 64 + tx * 4;
                 float* c = part + m * p.N + n;
                 if (pvec && n + 3 < p.N) {
-                    *reinterpret_cast<float4*>(c) = make_float4(outer[i][h * 4], outer[i][h * 4 + 1],
-                                                                outer[i][h * 4 + 2], outer[i][h * 4 + 3]);
+                    *reinterpret_cast<float4*>(c) = make_float4(
+                        outer[i][h][acc_slot(0)], outer[i][h][acc_slot(1)],
+                        outer[i][h][acc_slot(2)], outer[i][h][acc_slot(3)]);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        if (n + j < p.N) c[j] = outer[i][h * 4 + j];
+                        if (n + j < p.N) c[j] = outer[i][h][acc_slot(j)];
                 }
             }
         }
@@ -336,7 +326,7 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
             float* c = p.C + m * p.ldc + n;
             float v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = p.alpha * outer[i][h * 4 + j];
+            for (int j = 0; j < 4; ++j) v[j] = p.alpha * outer[i][h][acc_slot(j)];
             if (cvec && n + 3 < p.N) {
                 float4 o;
                 if (p.beta != 0.f) {
@@ -392,21 +382,30 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(int64_t M, int64_t N
     }
 }
 
-template <int BM, int BN, bool A_KC, bool B_NC>
-void launch_variant(const Args& a, int64_t splits, bool vec, hipStream_t s) {
-    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)splits), block(NT);
-    if (vec)
-        hipLaunchKernelGGL((sgemm_f32_kernel<BM, BN, A_KC, B_NC, true>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((sgemm_f32_kernel<BM, BN, A_KC, B_NC, false>), grid, block, 0, s, a);
+// Whether a tile's loads of an operand lie within 2^32 bytes of a slice's first
+// element: up to `lines` lines of ld floats when k is the unit stride, else the
+// slice's 16 k.
+bool fits32(bool kc, int64_t ld, int64_t lines) {
+    return (kc ? lines : BK) * ld + 128 < (int64_t)1 << 30;
+}
+
+template <int BM, int BN, typename Off>
+void launch_class(const Args& a, bool a_kc, bool b_nc, int64_t splits, hipStream_t s) {
+    const dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)splits);
+    const auto kernel = a_kc ? (b_nc ? sgemm_f32_kernel<BM, BN, true, true, Off>
+                                     : sgemm_f32_kernel<BM, BN, true, false, Off>)
+                             : (b_nc ? sgemm_f32_kernel<BM, BN, false, true, Off>
+                                     : sgemm_f32_kernel<BM, BN, false, false, Off>);
+    hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, s, a);
 }
 
 template <int BM, int BN>
-void launch_class(const Args& a, bool a_kc, bool b_nc, int64_t splits, bool vec, hipStream_t s) {
-    if (a_kc && b_nc) launch_variant<BM, BN, true, true>(a, splits, vec, s);
-    else if (a_kc && !b_nc) launch_variant<BM, BN, true, false>(a, splits, vec, s);
-    else if (!a_kc && b_nc) launch_variant<BM, BN, false, true>(a, splits, vec, s);
-    else launch_variant<BM, BN, false, false>(a, splits, vec, s);
+void launch_class(const Args& a, bool a_kc, bool b_nc, int64_t splits, hipStream_t s) {
+    if (fits32(a_kc, a.lda, std::min<int64_t>(a.M, BM)) &&
+        fits32(!b_nc, a.ldb, std::min<int64_t>(a.N, BN)))
+        launch_class<BM, BN, unsigned>(a, a_kc, b_nc, splits, s);
+    else
+        launch_class<BM, BN, int64_t>(a, a_kc, b_nc, splits, s);
 }
 
 // The plain tile classes: tile shape, workgroups per CU, and the FP32 flop/s
@@ -577,12 +576,9 @@ omb_status launch_sgemm_f32(int64_t M, int64_t N, int64_t K, float alpha,
         }
         a.part = part;
     }
-    const bool vec = ((reinterpret_cast<uintptr_t>(A) & 15) == 0) &&
-                     ((reinterpret_cast<uintptr_t>(B) & 15) == 0) && (lda % 4 == 0) &&
-                     (ldb % 4 == 0);
-    if (cls == 0) launch_class<128, 128>(a, a_kc, b_nc, splits, vec, s);
-    else if (cls == 1) launch_class<128, 64>(a, a_kc, b_nc, splits, vec, s);
-    else launch_class<64, 64>(a, a_kc, b_nc, splits, vec, s);
+    if (cls == 0) launch_class<128, 128>(a, a_kc, b_nc, splits, s);
+    else if (cls == 1) launch_class<128, 64>(a, a_kc, b_nc, splits, s);
+    else launch_class<64, 64>(a, a_kc, b_nc, splits, s);
     OMB_HIP_TRY(hipGetLastError());
     if (splits > 1) return launch_splitk_reduce(M, N, splits, alpha, beta, a.part, C, ldc, s);
     return OMB_OK;
