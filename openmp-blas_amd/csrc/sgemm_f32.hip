@@ -290,61 +290,66 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
         __syncthreads();
     }
 
-    // Epilogue: rows {g*64 + ty*4 + i}, columns {h*64 + tx*4 + j}.
+    // Epilogue: rows {g*64 + ty*4 + i}, columns {h*64 + tx*4 + j}, whole quads
+    // with 128-bit accesses at any alignment, the reads of C in one batch ahead
+    // of the writes.  This bounds products of few k: 5949 x 3823 x 57 with beta
+    // = 1 took 119 us with element accesses on its unaligned rows, 91 with
+    // quads, 78 with the reads ahead; 8192 x 8192 x 64: 228, 225, 171.
+    const int rows = (int)std::min<int64_t>(p.M - m0, BM), cols = (int)std::min<int64_t>(p.N - n0, BN);
     if (p.part) {  // raw partial sums of this split, row-major M x N
-        float* part = p.part + (int64_t)blockIdx.y * p.M * p.N;
-        const bool pvec = p.N % 4 == 0;
+        float* const c0 = p.part + ((int64_t)blockIdx.y * p.M + m0) * p.N + n0;
 #pragma unroll
-        for (int i = 0; i < TR; ++i) {
-            const int64_t m = m0 + (i / 4) * 64 + ty * 4 + (i % 4);
-            if (m >= p.M) continue;
+        for (int i = 0; i < TR; ++i)
 #pragma unroll
             for (int h = 0; h < GC; ++h) {
-                const int64_t n = n0 + h * 64 + tx * 4;
-                float* c = part + m * p.N + n;
-                if (pvec && n + 3 < p.N) {
-                    *reinterpret_cast<float4*>(c) = make_float4(
-                        outer[i][h][acc_slot(0)], outer[i][h][acc_slot(1)],
-                        outer[i][h][acc_slot(2)], outer[i][h][acc_slot(3)]);
-                } else {
+                const int m = (i / 4) * 64 + ty * 4 + (i % 4), n = h * 64 + tx * 4;
+                if (m >= rows) continue;
+                float* c = c0 + m * p.N + n;
+                const acc4 v = outer[i][h];
+                if (n + 3 < cols)
+                    *reinterpret_cast<f32x4_u*>(c) = f32x4_u{v[acc_slot(0)], v[acc_slot(1)],
+                                                             v[acc_slot(2)], v[acc_slot(3)]};
+                else
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        if (n + j < p.N) c[j] = outer[i][h][acc_slot(j)];
-                }
+                        if (n + j < cols) c[j] = v[acc_slot(j)];
             }
-        }
         return;
     }
-    const bool cvec = ((reinterpret_cast<uintptr_t>(p.C) & 15) == 0) && (p.ldc % 4 == 0);
+    const float alpha = p.alpha, beta = p.beta;
+    const int64_t ldo = p.ldc;
+    float* const c0 = p.C + m0 * ldo + n0;
+    float4 old[TR][GC];
+    if (beta != 0.f) {
 #pragma unroll
-    for (int i = 0; i < TR; ++i) {
-        const int64_t m = m0 + (i / 4) * 64 + ty * 4 + (i % 4);
-        if (m >= p.M) continue;
+        for (int i = 0; i < TR; ++i)
+#pragma unroll
+            for (int h = 0; h < GC; ++h) {
+                const int m = (i / 4) * 64 + ty * 4 + (i % 4), n = h * 64 + tx * 4;
+                if (m < rows && n + 3 < cols) old[i][h] = ld4u(c0 + m * ldo + n);
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < TR; ++i)
 #pragma unroll
         for (int h = 0; h < GC; ++h) {
-            const int64_t n = n0 + h * 64 + tx * 4;
-            float* c = p.C + m * p.ldc + n;
-            float v[4];
+            const int m = (i / 4) * 64 + ty * 4 + (i % 4), n = h * 64 + tx * 4;
+            if (m >= rows) continue;
+            float* c = c0 + m * ldo + n;
+            f32x4_u v;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = p.alpha * outer[i][h][acc_slot(j)];
-            if (cvec && n + 3 < p.N) {
-                float4 o;
-                if (p.beta != 0.f) {
-                    float4 c4 = *reinterpret_cast<const float4*>(c);
-                    o = make_float4(v[0] + p.beta * c4.x, v[1] + p.beta * c4.y,
-                                    v[2] + p.beta * c4.z, v[3] + p.beta * c4.w);
-                } else {
-                    o = make_float4(v[0], v[1], v[2], v[3]);
-                }
-                *reinterpret_cast<float4*>(c) = o;
+            for (int j = 0; j < 4; ++j) v[j] = alpha * outer[i][h][acc_slot(j)];
+            if (n + 3 < cols) {
+                if (beta != 0.f)
+                    v = f32x4_u{v[0] + beta * old[i][h].x, v[1] + beta * old[i][h].y,
+                                v[2] + beta * old[i][h].z, v[3] + beta * old[i][h].w};
+                *reinterpret_cast<f32x4_u*>(c) = v;
             } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (n + j < p.N) c[j] = p.beta != 0.f ? v[j] + p.beta * c[j] : v[j];
-                }
+                for (int j = 0; j < 4; ++j)
+                    if (n + j < cols) c[j] = beta != 0.f ? v[j] + beta * c[j] : v[j];
             }
         }
-    }
 }
 
 // C = alpha * (sum of the splits' partials, in split order) + beta * C.
