@@ -93,6 +93,20 @@ constexpr int kLineFloats = 32;  // floats per 128-byte line
 int64_t gemm_k_splits(int64_t M, int64_t N, int64_t K, int64_t align, double rate_full,
                       double rate_alone, int64_t* kchunk);
 int64_t sgemm_f32_splits(int64_t M, int64_t N, int64_t K, int64_t* kchunk);
+// The class of the kernel that divides K among a workgroup's wavefronts whose
+// modelled time is least and below *time (seconds), which it replaces, or -1.
+// Its sums are those of the unsplit tiles, bit for bit, with no partials in memory.
+int sgemm_f32_wave_class(int64_t M, int64_t N, int64_t K, double* time);
+omb_status launch_sgemm_f32_wave(int cls, int64_t M, int64_t N, int64_t K, float alpha,
+                                 const float* A, int64_t lda, bool a_kc, const float* B,
+                                 int64_t ldb, bool b_nc, float beta, float* C, int64_t ldc,
+                                 hipStream_t s);
+// Whether a tile's loads of an operand lie within 2^32 bytes of a 16-k slice's
+// first element: up to `lines` lines of ld floats when k is the unit stride,
+// else the slice's 16 k.
+inline bool offsets_fit32(bool kc, int64_t ld, int64_t lines) {
+    return ld < (int64_t)1 << 30 && (kc ? lines : 16) * ld + 128 < (int64_t)1 << 30;
+}
 int64_t sgemm_split_splits(int64_t M, int64_t N, int64_t K, int64_t* kchunk);
 omb_status launch_splitk_reduce(int64_t M, int64_t N, int64_t splits, float alpha, float beta,
                                 const float* part, float* C, int64_t ldc, hipStream_t s);
@@ -207,6 +221,11 @@ __host__ __device__ inline float rng_uniform(uint64_t key, uint64_t i) {
 // type tells the compiler that only 4-byte alignment is known; gfx950 serves
 // it with one dwordx4 load).  The _nt form does not keep the line in cache.
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+// The accumulators of four adjacent columns.  Column j's lies one place further
+// on: register tuples start on even registers, so with the odd rotation a column
+// of B and its accumulators are never in one register bank.
+typedef float acc4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ constexpr int acc_slot(int j) { return (j + 1) & 3; }
 __device__ inline float4 ld4u_nt(const float* p) {
     f32x4_u v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(p));
     return make_float4(v.x, v.y, v.z, v.w);

@@ -57,6 +57,9 @@ constexpr double kTileRateF32_128x64 = 0.114e12;
 constexpr double kTileRateF32_128x64Alone = 0.158e12;
 constexpr double kTileRateF32_64x64 = 0.079e12;
 constexpr double kTileRateF32_64x64Alone = 0.129e12;
+// A product's time by the tile classes, for the comparison with the classes of
+// sgemm_f32_wave.hip: launch (with a split's second one) and scale of the model.
+constexpr double kTileLaunch = 6.4e-6, kTileScale = 0.78;
 constexpr double kSplitHbm = 4.0e12;      // bytes/s for the partials' traffic
 constexpr double kSplitLaunch = 4.0e-6;   // the reduction kernel's launch and tail
 constexpr double kSplitReduceStep = 1.0e-6;  // one round trip per 8 partials of an element
@@ -75,12 +78,6 @@ struct Args {
     float* part;     // split partial sums [split][M][N], or null (one split)
 };
 
-// The four columns of a quad lie in its accumulator tuple one place further on:
-// register tuples start on even registers, so with the odd rotation a column
-// of B and its accumulators are never in one bank.
-typedef float acc4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ constexpr int acc_slot(int j) { return (j + 1) & 3; }
-
 // One operand's side of a workgroup's tile: E lines (rows of A or columns of
 // B) from line e0 of the operand; KC: k is the unit stride, else the line is.
 // Its 16-k slices are read with 128-bit loads along the unit stride at any
@@ -88,7 +85,7 @@ __device__ __forceinline__ constexpr int acc_slot(int j) { return (j + 1) & 3; }
 // the repeated lines give is never stored, so every full slice of every tile,
 // ragged or not, takes the same unguarded loads.  A thread's loads are byte
 // offsets from the slice's first element, of 32 bits unless the leading
-// dimension is too long for that (fits32).
+// dimension is too long for that (offsets_fit32).
 template <int E, bool KC, typename Off>
 struct Side {
     static constexpr int L = E / 64;  // float4 per thread and slice
@@ -387,13 +384,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(int64_t M, int64_t N
     }
 }
 
-// Whether a tile's loads of an operand lie within 2^32 bytes of a slice's first
-// element: up to `lines` lines of ld floats when k is the unit stride, else the
-// slice's 16 k.
-bool fits32(bool kc, int64_t ld, int64_t lines) {
-    return (kc ? lines : BK) * ld + 128 < (int64_t)1 << 30;
-}
-
 template <int BM, int BN, typename Off>
 void launch_class(const Args& a, bool a_kc, bool b_nc, int64_t splits, hipStream_t s) {
     const dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)splits);
@@ -406,8 +396,8 @@ void launch_class(const Args& a, bool a_kc, bool b_nc, int64_t splits, hipStream
 
 template <int BM, int BN>
 void launch_class(const Args& a, bool a_kc, bool b_nc, int64_t splits, hipStream_t s) {
-    if (fits32(a_kc, a.lda, std::min<int64_t>(a.M, BM)) &&
-        fits32(!b_nc, a.ldb, std::min<int64_t>(a.N, BN)))
+    if (offsets_fit32(a_kc, a.lda, std::min<int64_t>(a.M, BM)) &&
+        offsets_fit32(!b_nc, a.ldb, std::min<int64_t>(a.N, BN)))
         launch_class<BM, BN, unsigned>(a, a_kc, b_nc, splits, s);
     else
         launch_class<BM, BN, int64_t>(a, a_kc, b_nc, splits, s);
@@ -415,11 +405,12 @@ void launch_class(const Args& a, bool a_kc, bool b_nc, int64_t splits, hipStream
 
 // The plain tile classes: tile shape, workgroups per CU, and the FP32 flop/s
 // of one workgroup with the CU full of its class and alone on its CU.
+constexpr int kTileClasses = 3;
 struct F32Class {
     int bm, bn, occ;
     double rate_full, rate_alone;
 };
-constexpr F32Class kF32Classes[3] = {
+constexpr F32Class kF32Classes[kTileClasses] = {
     {128, 128, 2, kTileRateF32, kTileRateF32Alone},
     {128, 64, 3, kTileRateF32_128x64, kTileRateF32_128x64Alone},
     {64, 64, 4, kTileRateF32_64x64, kTileRateF32_64x64Alone},
@@ -511,11 +502,12 @@ int64_t gemm_k_splits(int64_t M, int64_t N, int64_t K, int64_t align, double rat
 // least, a smaller class only when the model finds it 15% faster than the
 // larger one before it (with a 5% margin the model's optimism for partly
 // filled rounds of small tiles cost 3-8% at some sizes from 1216 to 2432).
-// Any class and any exact split give the same bits.
-int sgemm_f32_choose(int64_t M, int64_t N, int64_t K, int64_t* splits, int64_t* kchunk) {
+// Any class and any exact split give the same bits.  *time: what the model gives.
+int choose_tiles(int64_t M, int64_t N, int64_t K, int64_t* splits, int64_t* kchunk,
+                 double* time) {
     int best = 0;
     double best_t = 0.0;
-    for (int c = 0; c < 3; ++c) {
+    for (int c = 0; c < kTileClasses; ++c) {
         const F32Class& k = kF32Classes[c];
         int64_t kc = K;
         double t = 0.0;
@@ -528,7 +520,24 @@ int sgemm_f32_choose(int64_t M, int64_t N, int64_t K, int64_t* splits, int64_t* 
             *kchunk = kc;
         }
     }
+    *time = best_t;
     return best;
+}
+
+// What a product takes: a tile class with its K split, or one of the classes
+// that divide K among a workgroup's wavefronts (numbered after the tiles'),
+// whichever its model finds faster.  The tiles' model leaves out the launch and
+// was fitted before their k loop gained: in this comparison their time is
+// kTileLaunch + kTileScale of it, fitted with the other classes'.
+int sgemm_f32_choose(int64_t M, int64_t N, int64_t K, int64_t* splits, int64_t* kchunk) {
+    double t = 0.0;
+    const int cls = choose_tiles(M, N, K, splits, kchunk, &t);
+    t = kTileLaunch + kTileScale * t;
+    const int wave = sgemm_f32_wave_class(M, N, K, &t);
+    if (wave < 0) return cls;
+    *splits = 1;
+    *kchunk = K;
+    return kTileClasses + wave;
 }
 
 int64_t sgemm_f32_splits(int64_t M, int64_t N, int64_t K, int64_t* kchunk) {
@@ -565,6 +574,9 @@ omb_status launch_sgemm_f32(int64_t M, int64_t N, int64_t K, float alpha,
     // leave CUs idle (the splits' partials are then added in split order).
     int64_t splits = 1, kchunk = K;
     const int cls = sgemm_f32_choose(M, N, K, &splits, &kchunk);
+    if (cls >= kTileClasses)
+        return launch_sgemm_f32_wave(cls - kTileClasses, M, N, K, alpha, A, lda, a_kc, B, ldb, b_nc,
+                                     beta, C, ldc, s);
     const F32Class& fc = kF32Classes[cls];
     Args a{M, N, K, alpha, beta, A, lda, B, ldb, C, ldc, ceil_div(M, fc.bm), ceil_div(N, fc.bn),
            kchunk, nullptr};

@@ -1,0 +1,394 @@
+// Plain FP32 SGEMM for products whose 128x128 tiles leave CUs idle: C =
+// alpha*A*B + beta*C with K divided among the wavefronts of a workgroup.
+//
+// Counterpart of the same code as sgemm_f32.hip (include/mtm.hpp:83-206,
+// include/simd_loop.hpp:80-192), for the small and middle sizes of the
+// reference's sweep (src/mtm.cpp:372-375).  A workgroup of W wavefronts owns
+// one BM x BN tile of C.  Wavefront w sums the 128-k accumulation blocks w,
+// w + W, ... of the whole tile, each from zero, with 4*GR x 4*GC outputs per
+// lane; after every W blocks the wavefronts' block sums meet in LDS and are
+// added to the tile in block order.  That is the unsplit kernel's own fold,
+// outer = ((b0 + b1) + b2) ..., so the bits are those of sgemm_f32_kernel for
+// any W and K, with no partial sums in memory and no second launch, and a
+// wavefront holds one accumulator tile instead of two.
+//
+// Each wavefront stages its own 16-k slices of A and B through its own LDS
+// buffers (LDS operations of a wavefront complete in order, so the k loop has
+// no workgroup barrier), with D slices of global loads in flight.  Rows and
+// columns past C are clamped to valid addresses: what they give is never
+// stored.  Only K's last slice (and the last slice of a tile whose 4-column
+// loads could pass the end of an operand) loads element by element.
+//
+// Bound by FP32 issue once the chip is full; below that by the launch and one
+// memory round trip per D slices.
+#include <algorithm>
+#include <cmath>
+
+#include "common.hpp"
+
+namespace omb {
+namespace {
+
+constexpr int BK = 16;
+constexpr int BLOCK_K = 128;  // k per accumulation block, as sgemm_f32.hip
+constexpr int PAD = 4;
+constexpr int kGroupM = 8;
+
+struct WArgs {
+    int64_t M, N, K;
+    float alpha, beta;
+    const float* A;
+    int64_t lda;
+    const float* B;
+    int64_t ldb;
+    float* C;
+    int64_t ldc;
+    int64_t tiles_m, tiles_n;
+};
+
+// Orders a wavefront's LDS writes before its other lanes' reads (and the
+// reverse): the hardware keeps the order, this keeps the compiler's.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One operand of a wavefront's tile: E rows (of A) or columns (of B^T), called
+// lines, starting at line e0; KC: k is the unit stride.  load() brings a full
+// slice into registers, load_guarded() a partial one, store() puts it into LDS
+// as [k][line].
+template <int E, bool KC, typename Off>
+struct Side {
+    static constexpr int L = E / 16;  // float4 per lane and slice
+    const float* p;  // line e0 (wavefront-uniform, as is the k of a load: the
+                     // loads add a lane's offset to a scalar address)
+    int64_t ld;
+    int n;           // lines of the operand from e0
+    int lane;
+
+    __device__ __forceinline__ void init(const float* X, int64_t ld_, int64_t e0, int64_t extent,
+                                         int lane_) {
+        p = X + (KC ? e0 * ld_ : e0);
+        ld = ld_;
+        n = (int)std::min<int64_t>(extent - e0, E);
+        lane = lane_;
+    }
+    // byte offset of load i: line (KC) or quad of lines, clamped into the operand
+    __device__ __forceinline__ Off offset(int i) const {
+        const int e = lane + 64 * i;
+        return (Off)(4 * (KC ? min(e >> 2, n - 1) * ld + (e & 3) * 4
+                             : (e / (E / 4)) * ld + min(e % (E / 4) * 4, (n - 1) & ~3)));
+    }
+    __device__ __forceinline__ void load(float4 (&v)[L], const Off (&off)[L], int64_t k0) const {
+        const char* q = reinterpret_cast<const char*>(p + (KC ? k0 : k0 * ld));
+#pragma unroll
+        for (int i = 0; i < L; ++i) v[i] = ld4u(reinterpret_cast<const float*>(q + off[i]));
+    }
+    // k steps at the operand's end that a 4-line load could read past: the
+    // last one, or the last three when lines are less than 4 floats apart.
+    __device__ __forceinline__ int tail() const {
+        return KC || n % 4 == 0 ? 0 : (ld < 4 ? 3 : 1);
+    }
+    // k0 .. k1-1 are the valid k of the slice (k1 <= K)
+    __device__ __forceinline__ void load_guarded(float4 (&v)[L], int64_t k0, int64_t k1) const {
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int e = lane + 64 * i;
+            float t[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int64_t line = min(KC ? e >> 2 : e % (E / 4) * 4 + c, n - 1);
+                const int64_t k = k0 + (KC ? (e & 3) * 4 + c : e / (E / 4));
+                const int64_t b = std::min(k, k1 - 1);
+                const float x = p[KC ? line * ld + b : b * ld + line];
+                t[c] = k < k1 ? x : 0.f;
+            }
+            v[i] = make_float4(t[0], t[1], t[2], t[3]);
+        }
+    }
+    __device__ __forceinline__ void store(float (*s)[E + PAD], const float4 (&v)[L]) const {
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int e = lane + 64 * i;
+            if constexpr (KC) {
+                const int line = e >> 2, kq = (e & 3) * 4;
+                s[kq + 0][line] = v[i].x;
+                s[kq + 1][line] = v[i].y;
+                s[kq + 2][line] = v[i].z;
+                s[kq + 3][line] = v[i].w;
+            } else {
+                *reinterpret_cast<float4*>(&s[e / (E / 4)][e % (E / 4) * 4]) = v[i];
+            }
+        }
+    }
+};
+
+// GR, GC: 4-row and 4-column groups per lane (8 x 8 lanes: BM = 32*GR, BN =
+// 32*GC); W wavefronts; D slices of loads in flight.
+template <int GR, int GC, int W, int D, int OCC, bool A_KC, bool B_NC, typename Off>
+__global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
+    constexpr int BM = 32 * GR, BN = 32 * GC, TR = 4 * GR;
+    constexpr int S = TR * GC;            // float4 of the tile per lane
+    constexpr int P = S > 4 ? 2 : 1;      // passes of the LDS sum (bounds its LDS)
+    constexpr int SP = S / P, OWN = (SP + W - 1) / W;  // float4 per pass; of them, added here
+    struct Stage {
+        float a[BK][BM + PAD], b[BK][BN + PAD];
+    };
+    union Shared {
+        Stage stage[W];
+        acc4 sum[W][SP][64];
+    };
+    __shared__ __attribute__((aligned(16))) Shared sh;
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lx = lane & 7, ly = lane >> 3;
+    int64_t tm, tn;
+    group_tile(xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n), p.tiles_m, p.tiles_n, kGroupM, &tm, &tn);
+    const int64_t m0 = tm * BM, n0 = tn * BN;
+    Side<BM, A_KC, Off> sa;
+    Side<BN, !B_NC, Off> sb;
+    sa.init(p.A, p.lda, m0, p.M, lane);
+    sb.init(p.B, p.ldb, n0, p.N, lane);
+    Off oa[sa.L], ob[sb.L];
+#pragma unroll
+    for (int i = 0; i < sa.L; ++i) oa[i] = sa.offset(i);
+#pragma unroll
+    for (int i = 0; i < sb.L; ++i) ob[i] = sb.offset(i);
+    const int tail = max(sa.tail(), sb.tail());
+
+    acc4 inner[TR][GC];
+    Stage& st = sh.stage[wave];
+    float4 fa[2][GR], fb[2][GC];  // fragments of this k and of the next one
+    auto fragment = [&](int k, int set) {
+#pragma unroll
+        for (int g = 0; g < GR; ++g)
+            fa[set][g] = *reinterpret_cast<const float4*>(&st.a[k][g * 32 + ly * 4]);
+#pragma unroll
+        for (int h = 0; h < GC; ++h)
+            fb[set][h] = *reinterpret_cast<const float4*>(&st.b[k][h * 32 + lx * 4]);
+    };
+    auto compute = [&] {  // the staged slice
+        fragment(0, 0);
+#pragma unroll
+        for (int k = 0; k < BK; ++k) {
+            if (k + 1 < BK) fragment(k + 1, (k + 1) & 1);
+            const float* a = reinterpret_cast<const float*>(fa[k & 1]);
+#pragma unroll
+            for (int i = 0; i < TR; ++i)
+#pragma unroll
+                for (int h = 0; h < GC; ++h) {
+                    const float4 v = fb[k & 1][h];
+                    acc4& s = inner[i][h];
+                    s[acc_slot(0)] = fmaf(a[i], v.x, s[acc_slot(0)]);
+                    s[acc_slot(1)] = fmaf(a[i], v.y, s[acc_slot(1)]);
+                    s[acc_slot(2)] = fmaf(a[i], v.z, s[acc_slot(2)]);
+                    s[acc_slot(3)] = fmaf(a[i], v.w, s[acc_slot(3)]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    acc4 outer[P * OWN];
+#pragma unroll
+    for (int o = 0; o < P * OWN; ++o) outer[o] = acc4{0.f, 0.f, 0.f, 0.f};
+    const int64_t nblk = ceil_div(p.K, BLOCK_K);
+    for (int64_t first = 0; first < nblk; first += W) {
+        const int64_t blk = first + wave;
+        if (blk < nblk) {
+#pragma unroll
+            for (int i = 0; i < TR; ++i)
+#pragma unroll
+                for (int h = 0; h < GC; ++h) inner[i][h] = acc4{0.f, 0.f, 0.f, 0.f};
+            const int64_t kb = blk * BLOCK_K, ke = std::min<int64_t>(p.K, kb + BLOCK_K);
+            const int nk = (int)(ke - kb) - (ke == p.K ? tail : 0);
+            const int nfull = nk > 0 ? nk / BK : 0;
+            const int64_t klast = kb + (int64_t)std::max(nfull - 1, 0) * BK;
+            float4 va[D][sa.L], vb[D][sb.L];
+            auto load = [&](int set, int64_t k) {
+                k = k < klast ? k : klast;
+                sa.load(va[set], oa, k);
+                sb.load(vb[set], ob, k);
+            };
+            auto store = [&](int set) {
+                wave_lds_fence();
+                sa.store(st.a, va[set]);
+                sb.store(st.b, vb[set]);
+                wave_lds_fence();
+            };
+            int s = 0;
+            if (nfull >= D) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) load(d, kb + d * BK);
+                store(0);
+                for (; s + D <= nfull; s += D) {
+                    // Keeps each tuple in four consecutive registers through the loop.
+#pragma unroll
+                    for (int i = 0; i < TR; ++i)
+#pragma unroll
+                        for (int h = 0; h < GC; ++h) asm volatile("" : "+v"(inner[i][h]));
+#pragma unroll
+                    for (int d = 0; d < D; ++d) {  // slice s + d is staged, set d free
+                        load(d, kb + (int64_t)(s + D + d) * BK);
+                        __builtin_amdgcn_sched_barrier(0);
+                        compute();
+                        store((d + 1) % D);
+                    }
+                }
+            }
+            // what the last block leaves: fewer than D full slices, K % 16
+#pragma unroll 1
+            for (int64_t k = kb + (int64_t)s * BK; k < ke; k += BK, ++s) {
+                if (s < nfull) {
+                    load(0, k);
+                } else {
+                    sa.load_guarded(va[0], k, std::min<int64_t>(ke, k + BK));
+                    sb.load_guarded(vb[0], k, std::min<int64_t>(ke, k + BK));
+                }
+                store(0);
+                compute();
+            }
+        }
+        // Block sums -> LDS, added in block order by the wavefront that owns
+        // each float4 of the lanes' tiles.
+        const int in_round = (int)std::min<int64_t>(W, nblk - first);
+        if constexpr (W > 1) {
+#pragma unroll
+            for (int q = 0; q < P; ++q) {
+                __syncthreads();  // the staging buffers, or the last pass, are read
+                if (wave < in_round) {
+#pragma unroll
+                    for (int s = 0; s < SP; ++s)
+                        sh.sum[wave][s][lane] = inner[(q * SP + s) / GC][(q * SP + s) % GC];
+                }
+                __syncthreads();
+                for (int w = 0; w < in_round; ++w) {
+#pragma unroll
+                    for (int o = 0; o < OWN; ++o) {
+                        const int slot = wave * OWN + o;
+                        if (slot >= SP) continue;
+                        outer[q * OWN + o] += sh.sum[w][slot][lane];
+                    }
+                }
+            }
+            if (first + W < nblk) __syncthreads();  // before the next round's staging
+        } else {
+#pragma unroll
+            for (int i = 0; i < TR; ++i)
+#pragma unroll
+                for (int h = 0; h < GC; ++h) outer[i * GC + h] += inner[i][h];
+        }
+    }
+
+    // Whole quads at any alignment, the reads of C ahead of the writes.
+    const int rows = (int)std::min<int64_t>(p.M - m0, BM), cols = (int)std::min<int64_t>(p.N - n0, BN);
+    float* const c0 = p.C + m0 * p.ldc + n0;
+    auto place = [&](int o, int* m, int* n) {  // outer[o]'s row and first column
+        const int in_pass = wave * OWN + o % OWN, slot = o / OWN * SP + in_pass;
+        *m = (slot / GC >> 2) * 32 + ly * 4 + (slot / GC & 3);
+        *n = slot % GC * 32 + lx * 4;
+        return in_pass < SP && *m < rows && *n < cols;
+    };
+    float4 old[P * OWN];
+    if (p.beta != 0.f) {
+#pragma unroll
+        for (int o = 0; o < P * OWN; ++o) {
+            int m, n;
+            if (place(o, &m, &n) && n + 3 < cols) old[o] = ld4u(c0 + m * p.ldc + n);
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < P * OWN; ++o) {
+        int m, n;
+        if (!place(o, &m, &n)) continue;
+        float* c = c0 + m * p.ldc + n;
+        f32x4_u v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = p.alpha * outer[o][acc_slot(e)];
+        if (n + 3 < cols) {
+            if (p.beta != 0.f)
+                v = f32x4_u{v[0] + p.beta * old[o].x, v[1] + p.beta * old[o].y,
+                            v[2] + p.beta * old[o].z, v[3] + p.beta * old[o].w};
+            *reinterpret_cast<f32x4_u*>(c) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < cols) c[e] = p.beta != 0.f ? v[e] + p.beta * c[e] : v[e];
+        }
+    }
+}
+
+// The classes: tile, wavefronts, and the measured model of a launch's time (us):
+//   fixed + the rounds of W blocks one after another at `block` us each, or
+//   fixed + the tiles' flop at `rate` TFLOP/s, an idle wavefront of the last
+//   round costing `idle` of a busy one and the last wave of workgroups (per_cu
+//   resident per CU) its square root of unevenness, whichever is longer.
+// Fitted to 1120 products with M, N and K from 32 to 6144 (geometrically drawn, up to 4e10
+// flop): with the choice of sgemm_f32_choose they took 1/1.22 of the tile classes'
+// time, against 1/1.23 if the fastest were always chosen.
+
+struct WaveClass {
+    int gr, gc, w, per_cu;
+    double fixed, rate, block, idle;
+};
+constexpr WaveClass kWaveClasses[4] = {
+    {2, 2, 8, 1, 5.0, 72.0, 15.0, 0.35},
+    {1, 1, 8, 2, 3.1, 49.0, 7.8, 0.46},
+    {1, 1, 4, 5, 3.0, 64.0, 8.4, 0.30},
+    {1, 1, 2, 10, 4.7, 78.0, 9.9, 0.31},
+};
+
+template <int GR, int GC, int W, int OCC>
+void launch_class(const WArgs& p, bool a_kc, bool b_nc, hipStream_t s) {
+    const bool near = offsets_fit32(a_kc, p.lda, std::min<int64_t>(p.M, 32 * GR)) &&
+                      offsets_fit32(!b_nc, p.ldb, std::min<int64_t>(p.N, 32 * GC));
+    auto pick = [&](auto off) {
+        using Off = decltype(off);
+        return a_kc ? (b_nc ? sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, true, true, Off>
+                            : sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, true, false, Off>)
+                    : (b_nc ? sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, false, true, Off>
+                            : sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, false, false, Off>);
+    };
+    hipLaunchKernelGGL(near ? pick(0u) : pick((int64_t)0), dim3((unsigned)(p.tiles_m * p.tiles_n)),
+                       dim3(64 * W), 0, s, p);
+}
+
+}  // namespace
+
+int sgemm_f32_wave_class(int64_t M, int64_t N, int64_t K, double* time) {
+    int best = -1;
+    for (int c = 0; c < 4; ++c) {
+        const WaveClass& k = kWaveClasses[c];
+        const double bm = 32 * k.gr, bn = 32 * k.gc;
+        const int64_t tiles = ceil_div(M, (int64_t)bm) * ceil_div(N, (int64_t)bn);
+        const int64_t blocks = ceil_div(K, BLOCK_K), rounds = ceil_div(blocks, k.w);
+        const double busy = (double)K / BLOCK_K + k.idle * (double)(rounds * k.w - blocks);
+        const double r = (double)tiles / ((double)k.per_cu * device_cu_count());
+        const double full = 2.0 * bm * bn * BLOCK_K * (double)tiles * busy / (k.rate * 1e6) *
+                            (r >= 1.0 && r < 4.0 ? std::sqrt(std::ceil(r) / r) : 1.0);
+        const double chain = (double)rounds * k.block * std::min(1.0, (double)K / BLOCK_K);
+        const double t = (k.fixed + std::max(chain, full)) * 1e-6;
+        if (tiles <= 0x7fffffffLL && t < *time) {
+            best = c;
+            *time = t;
+        }
+    }
+    return best;
+}
+
+omb_status launch_sgemm_f32_wave(int cls, int64_t M, int64_t N, int64_t K, float alpha,
+                                 const float* A, int64_t lda, bool a_kc, const float* B,
+                                 int64_t ldb, bool b_nc, float beta, float* C, int64_t ldc,
+                                 hipStream_t s) {
+    const WaveClass& k = kWaveClasses[cls];
+    const WArgs p{M, N, K, alpha, beta, A, lda, B, ldb, C, ldc,
+                  ceil_div(M, 32 * k.gr), ceil_div(N, 32 * k.gc)};
+    if (cls == 0) launch_class<2, 2, 8, 1>(p, a_kc, b_nc, s);
+    else if (cls == 1) launch_class<1, 1, 8, 2>(p, a_kc, b_nc, s);
+    else if (cls == 2) launch_class<1, 1, 4, 5>(p, a_kc, b_nc, s);
+    else launch_class<1, 1, 2, 5>(p, a_kc, b_nc, s);
+    OMB_HIP_TRY(hipGetLastError());
+    return OMB_OK;
+}
+
+}  // namespace omb

@@ -57,3 +57,38 @@ def test_lines_far_apart(dev, ompblas, ld):
     want = far.double() @ near.double()
     assert torch.equal(product(ompblas, far, near).double(), want)
     assert torch.equal(product(ompblas, near.t(), far.t()).double(), want.t())
+
+
+@pytest.mark.parametrize("a_row", [True, False])
+@pytest.mark.parametrize("b_row", [True, False])
+def test_k_divided_among_wavefronts(dev, ompblas, a_row, b_row):
+    """Sizes where a workgroup's wavefronts share K, in 32 x 32 and 64 x 64
+    tiles: rounds of 2, 4 and 8 blocks of 128, the last one partial or short."""
+    g = torch.Generator(device=dev).manual_seed(23)
+    for m, n in ((32, 32), (33, 31), (1, 70), (200, 150), (515, 513), (1024, 1022), (961, 963)):
+        for k in (5, 112, 128, 130, 256, 257, 500, 1024, 1025, 1160, 2175):
+            a = operand(dev, g, m, k, a_row, 1, 1)
+            b = operand(dev, g, k, n, b_row, 0, 3)
+            want = a.double() @ b.double()
+            assert torch.equal(product(ompblas, a, b).double(), want), (m, n, k)
+            c0 = torch.randint(-8, 9, (m, n), device=dev, generator=g).float()
+            got = product(ompblas, a, b, 0.5, -1.0, c0)
+            assert torch.equal(got.double(), want / 2 - c0), (m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(31, 33, 129), (150, 200, 301), (512, 512, 512), (515, 300, 900),
+                                   (1024, 1024, 1024), (960, 1000, 1900)])
+def test_bits_of_the_unsplit_sum(dev, ompblas, m, n, k):
+    """The wavefronts' block sums meet in block order: the bits of a grouped
+    launch, whose tiles run through all of K."""
+    g = torch.Generator(device=dev).manual_seed(k)
+    a = torch.rand((m, k), device=dev, generator=g) * 2 - 1
+    b = torch.rand((k, n), device=dev, generator=g) * 2 - 1
+    c0 = torch.rand((m, n), device=dev, generator=g)
+    for alpha, beta in ((1.0, 0.0), (1.5, -0.5)):
+        c = c0.clone()
+        plan = ompblas.GroupPlan([(m, n, k, a.data_ptr(), k, b.data_ptr(), n, c.data_ptr(), n,
+                                   alpha, beta)], [])
+        plan.launch()
+        torch.cuda.synchronize()
+        assert torch.equal(product(ompblas, a, b, alpha, beta, c0), c)
