@@ -33,7 +33,8 @@
 
 #include "gemv_row.hpp"
 #include "host_util.hpp"
-#include "split_common.hpp"
+#include "sgemm_wave.hpp"
+#include "split_tile.hpp"
 
 namespace omb {
 namespace {
@@ -82,8 +83,6 @@ struct PArgs {
     const DGemm* gemms;
     const DGemv* gemvs;
     unsigned* counters;  // [0] next dynamic chunk, [1] workgroups done
-    int nprod;
-    int f16;      // split tiles take the scaled FP16 pieces (3 products)
     int chunk;    // consecutive items per chunk
     int nchunks;  // ceil(nitems / chunk)
 };
@@ -111,17 +110,6 @@ __device__ __forceinline__ int item_tid() {
 // register sets; LDS fragments for k+1 are read while k's FMAs run.  Every
 // element sums k in order and folds the running sum every 128 k, as
 // sgemm_f32_kernel does, so the results are the same bits.
-template <int N>
-struct FragT;
-template <>
-struct FragT<2> {
-    typedef float2 type;
-};
-template <>
-struct FragT<4> {
-    typedef float4 type;
-};
-
 template <typename P>
 __device__ __forceinline__ float4 load4_guard(P p, int n) {
     if (n == 4) return ld4u(p);
@@ -145,8 +133,9 @@ __device__ __forceinline__ void tile_f32(const DGemm& g, int tm, int tn, float* 
     constexpr int PA = BM + 4, PB = BN + 4;  // padded LDS rows, 16-byte aligned
     constexpr int NA4 = BM * BK / 4, NB4 = BN * BK / 4;  // float4 per slice
     constexpr int LA = (NA4 + NT - 1) / NT, LB = (NB4 + NT - 1) / NT;
-    typedef typename FragT<FR>::type FragA;
-    typedef typename FragT<FC>::type FragB;
+    static_assert(FR == 4 && FC == 4, "fragments are float4");
+    typedef float4 FragA;
+    typedef float4 FragB;
     // Two LDS buffers of [BK][PA] A and [BK][PB] B: slice k+1 is stored into
     // one while slice k is read from the other (one barrier per slice).
     constexpr int SZ = BK * (PA + PB);
@@ -284,89 +273,237 @@ __device__ __forceinline__ void tile_f32(const DGemm& g, int tm, int tn, float* 
     }
 }
 
-// ------------------------------------------------------------ split tile --
-// 64x64 tile on the MFMA cores: each 16-k slice of A (row-major) and B^T
-// (B row-major) is read as FP32, split into the three BF16 planes and
-// written into the swizzled LDS slice; 4 wavefronts own 32x32 each.
-// The 4 consecutive-k values of A (row m, from k ka) and of B (column n,
-// from k kb) that one loader thread stages per 16-k slice; elements out of
-// range read as 0.  Edge loads read a clamped in-range address and select,
-// so every load of the slice is in flight at once (A and B are non-null
-// whenever a tile has K > 0).
-template <typename P>
-__device__ __forceinline__ void load_split_slice(P A, int64_t lda, int64_t M,
-                                                 P B, int64_t ldb, int64_t N,
-                                                 int64_t K, int64_t m, int64_t ka, int64_t n,
-                                                 int64_t kb, float (&va)[4], float (&vb)[4]) {
-    if (m < M && ka + 3 < K) {
-        const float4 t = ld4u(A + m * lda + ka);
-        va[0] = t.x; va[1] = t.y; va[2] = t.z; va[3] = t.w;
-    } else {
+// -------------------------------------------------- wavefront-private tiles --
+// One wavefront's 32 x 32 of C = alpha*A*B + beta*C at (m0, n0) (row-major):
+// the row and column quads of a lane, as sgemm_wave.hpp lays them out.
+typedef wave::WaveSide<32, true, int64_t, gcfloat*> SideA;
+typedef wave::WaveSide<32, false, int64_t, gcfloat*> SideB;
+
+// C's rows i0 .. i0 + R - 1 of each lane's four, whole quads at any alignment, the
+// reads of C ahead of the writes.
+template <int R>
+__device__ __forceinline__ void store_quads(const DGemm& g, int64_t m0, int64_t n0, int lane, int i0,
+                                            const acc4 (&v)[R]) {
+    typedef OMB_GLOBAL f32x4_u gf32x4_u;
+    const int rows = (int)std::min<int64_t>(g.M - m0, 32), cols = (int)std::min<int64_t>(g.N - n0, 32);
+    const int m = (lane >> 3) * 4 + i0, n = (lane & 7) * 4;
+    if (n >= cols) return;
+    gfloat* const c = as_global(g.C) + (m0 + m) * g.ldc + n0 + n;
+    float4 old[R];
+    if (g.beta != 0.f) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const bool ok = m < M && ka + e < K;
-            const float t = A[ok ? m * lda + ka + e : 0];
-            va[e] = ok ? t : 0.f;
-        }
+        for (int i = 0; i < R; ++i)
+            if (m + i < rows && n + 3 < cols) old[i] = ld4u((gcfloat*)(c + i * g.ldc));
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const bool ok = n < N && kb + e < K;
-        const float t = B[ok ? (kb + e) * ldb + n : 0];
-        vb[e] = ok ? t : 0.f;
+    for (int i = 0; i < R; ++i) {
+        if (m + i >= rows) continue;
+        f32x4_u x;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = g.alpha * v[i][acc_slot(j)];
+        if (n + 3 < cols) {
+            if (g.beta != 0.f)
+                x = f32x4_u{x[0] + g.beta * old[i].x, x[1] + g.beta * old[i].y,
+                            x[2] + g.beta * old[i].z, x[3] + g.beta * old[i].w};
+            *reinterpret_cast<gf32x4_u*>(c + i * g.ldc) = x;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (n + j < cols) {
+                    gfloat* e = c + i * g.ldc + j;
+                    *e = g.beta != 0.f ? x[j] + g.beta * *e : x[j];
+                }
+        }
     }
 }
 
-template <int NPROD>
-__device__ __forceinline__ void tile_split(const DGemm& g, int tm, int tn, uint4* smem) {
-    using namespace split;
-    constexpr int P = 64;  // rows per plane for A and for B^T
-    const int tid = item_tid(), lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int frow = lane & 31, fh = lane >> 5;
-    const int64_t m0 = (int64_t)tm * P, n0 = (int64_t)tn * P;
-    const int64_t M = g.M, N = g.N, K = g.K;
-    gcfloat* const A = as_global(g.A);
-    gcfloat* const B = as_global(g.B);
-    const int64_t lda = g.lda, ldb = g.ldb;
-    // loader roles: A row ra, k quarter qa; B^T row rb (= column of B), k quarter qb
-    const int ra = tid >> 2, qa = tid & 3;
-    const int rb = tid & 63, qb = tid >> 6;
-    uint2* l2 = reinterpret_cast<uint2*>(smem);
+// 64 x 64 as four 32 x 32 quadrants, one per wavefront, each through all of K with
+// slices of its own: no barrier in the k loop, and a quadrant past C costs nothing.
+// Two slices of loads are in flight; the running sum folds every 128 k, as in
+// sgemm_f32_kernel, so the results are the same bits.  Bound by the LDS reads (two
+// 128-bit reads per 16 FMAs) and, for few k, by each slice's latency; 4096 GEMMs of
+// 16 to 512 took 784 us as 64 x 64 tiles of the whole workgroup, 613 so.
+__device__ __forceinline__ void tile_quads(const DGemm& g, int tm, int tn, float* smem) {
+    using namespace wave;
+    const int tid = item_tid(), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t m0 = (int64_t)tm * 64 + (w >> 1) * 32, n0 = (int64_t)tn * 64 + (w & 1) * 32;
+    if (m0 >= g.M || n0 >= g.N) return;
+    WaveStage<1, 1>& st = reinterpret_cast<WaveStage<1, 1>*>(smem)[w];
+    SideA sa;
+    SideB sb;
+    sa.init(as_global(g.A), g.lda, m0, g.M, lane);
+    sb.init(as_global(g.B), g.ldb, n0, g.N, lane);
+    int64_t oa[sa.L], ob[sb.L];
+#pragma unroll
+    for (int i = 0; i < sa.L; ++i) oa[i] = sa.offset(i);
+#pragma unroll
+    for (int i = 0; i < sb.L; ++i) ob[i] = sb.offset(i);
+    acc4 inner[4][1], outer[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) inner[i][0] = outer[i] = acc4{0.f, 0.f, 0.f, 0.f};
+    auto fold = [&] {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            outer[i] += inner[i][0];
+            inner[i][0] = acc4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    const int64_t K = g.K, tail = std::max(sa.tail(), sb.tail());
+    const int64_t nfull = K > tail ? (K - tail) / BK : 0;
+    float4 va[2][sa.L], vb[2][sb.L];
+    auto load = [&](int set, int64_t s) {
+        const int64_t k0 = std::min(s, nfull - 1) * BK;
+        sa.load(va[set], oa, k0);
+        sb.load(vb[set], ob, k0);
+    };
+    auto store = [&](int set) {
+        wave_lds_fence();
+        sa.store(st.a, va[set]);
+        sb.store(st.b, vb[set]);
+        wave_lds_fence();
+    };
+    int64_t s = 0;
+    if (nfull > 0) {
+        load(0, 0);
+        load(1, 1);
+        // whole pairs, with the slice index of the loads clamped to the last one
+        for (; s + 1 < nfull; s += 2) {
+            pin(inner);
+            store(0);
+            load(0, s + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            wave_compute<1, 1>(st, lane, inner);
+            store(1);
+            load(1, s + 3);
+            __builtin_amdgcn_sched_barrier(0);
+            wave_compute<1, 1>(st, lane, inner);
+            if ((s + 2) % (BLOCK_K / BK) == 0) fold();
+        }
+        if (s < nfull) {
+            store(0);
+            wave_compute<1, 1>(st, lane, inner);
+            if (++s % (BLOCK_K / BK) == 0) fold();
+        }
+    }
+    for (int64_t k = s * BK; k < K; k += BK) {
+        sa.load_guarded(va[0], k, std::min<int64_t>(K, k + BK));
+        sb.load_guarded(vb[0], k, std::min<int64_t>(K, k + BK));
+        store(0);
+        wave_compute<1, 1>(st, lane, inner);
+        if ((k + BK) % BLOCK_K == 0) fold();
+    }
+    if (K % BLOCK_K || K == 0) fold();
+    store_quads<4>(g, m0, n0, lane, 0, outer);
+}
 
-    f32x16 inner[1][1], outer[1][1];
-    inner[0][0] = outer[0][0] = f32x16{};
-    const int64_t nkt = ceil_div(K, TK);
-    for (int64_t kt = 0; kt < nkt; ++kt) {
-        const int64_t k0 = kt * TK;
-        float va[4], vb[4];
-        load_split_slice(A, lda, M, B, ldb, N, K, m0 + ra, k0 + 4 * qa, n0 + rb, k0 + 4 * qb, va, vb);
-        __syncthreads();  // previous slice consumed
-        {
-            typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-            bf16x4 pa[3], pb[3];
+// 32 x 32 with K divided among the workgroup's wavefronts by 128-k blocks, whose
+// sums meet in LDS in block order (the fold, and the bits, of the other tiles).
+// For products with a short side and several blocks, whose few tiles would each
+// take all of K in one chain.
+__device__ __forceinline__ void tile_shared_k(const DGemm& g, int tm, int tn, float* smem) {
+    using namespace wave;
+    constexpr int W = NT / 64;
+    const int tid = item_tid(), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t m0 = (int64_t)tm * 32, n0 = (int64_t)tn * 32, K = g.K;
+    WaveStage<1, 1>& st = reinterpret_cast<WaveStage<1, 1>*>(smem)[w];
+    acc4* sum = reinterpret_cast<acc4*>(smem);  // [W][4][64], after a round's staging
+    SideA sa;
+    SideB sb;
+    sa.init(as_global(g.A), g.lda, m0, g.M, lane);
+    sb.init(as_global(g.B), g.ldb, n0, g.N, lane);
+    int64_t oa[sa.L], ob[sb.L];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                __bf16 t0, t1, t2;
-                split3(va[e], t0, t1, t2);
-                pa[0][e] = t0; pa[1][e] = t1; pa[2][e] = t2;
-                split3(vb[e], t0, t1, t2);
-                pb[0][e] = t0; pb[1][e] = t1; pb[2][e] = t2;
+    for (int i = 0; i < sa.L; ++i) oa[i] = sa.offset(i);
+#pragma unroll
+    for (int i = 0; i < sb.L; ++i) ob[i] = sb.offset(i);
+    const int tail = std::max(sa.tail(), sb.tail());
+    acc4 outer[1] = {acc4{0.f, 0.f, 0.f, 0.f}};  // row w of each lane's four
+    const int64_t nblk = ceil_div(K, (int64_t)BLOCK_K);
+    for (int64_t first = 0; first < nblk; first += W) {
+        acc4 inner[4][1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) inner[i][0] = acc4{0.f, 0.f, 0.f, 0.f};
+        const int64_t kb = (first + w) * BLOCK_K, ke = std::min<int64_t>(K, kb + BLOCK_K);
+        if (kb < K) {
+            const int nk = (int)(ke - kb) - (ke == K ? tail : 0);
+            const int nfull = nk > 0 ? nk / BK : 0;
+            float4 va[2][sa.L], vb[2][sb.L];
+            auto load = [&](int set, int s) {
+                const int64_t k0 = kb + std::min(s, nfull - 1) * BK;
+                sa.load(va[set], oa, k0);
+                sb.load(vb[set], ob, k0);
+            };
+            auto store = [&](int set) {
+                wave_lds_fence();
+                sa.store(st.a, va[set]);
+                sb.store(st.b, vb[set]);
+                wave_lds_fence();
+            };
+            int s = 0;
+            if (nfull > 0) {
+                load(0, 0);
+                load(1, 1);
+                for (; s + 1 < nfull; s += 2) {
+                    pin(inner);
+                    store(0);
+                    load(0, s + 2);
+                    __builtin_amdgcn_sched_barrier(0);
+                    wave_compute<1, 1>(st, lane, inner);
+                    store(1);
+                    load(1, s + 3);
+                    __builtin_amdgcn_sched_barrier(0);
+                    wave_compute<1, 1>(st, lane, inner);
+                }
+                if (s < nfull) {
+                    store(0);
+                    wave_compute<1, 1>(st, lane, inner);
+                    ++s;
+                }
             }
-#pragma unroll
-            for (int pl = 0; pl < 3; ++pl) {
-                l2[2 * (pl * 2 * P + lds_chunk(ra, qa >> 1)) + (qa & 1)] =
-                    *reinterpret_cast<const uint2*>(&pa[pl]);
-                l2[2 * (3 * 2 * P + pl * 2 * P + lds_chunk(rb, qb >> 1)) + (qb & 1)] =
-                    *reinterpret_cast<const uint2*>(&pb[pl]);
+            for (int64_t k = kb + s * BK; k < ke; k += BK) {
+                sa.load_guarded(va[0], k, std::min<int64_t>(ke, k + BK));
+                sb.load_guarded(vb[0], k, std::min<int64_t>(ke, k + BK));
+                store(0);
+                wave_compute<1, 1>(st, lane, inner);
             }
         }
+        const int in_round = (int)std::min<int64_t>(W, nblk - first);
+        __syncthreads();  // the staging buffers are read
+        if (w < in_round) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[(w * 4 + i) * 64 + lane] = inner[i][0];
+        }
         __syncthreads();
-        mfma_slice<NPROD, 1, 1, P, P>(smem, wm * 32, wn * 32, frow, fh, inner);
-        if ((kt + 1) % kFoldSlices == 0 || kt + 1 == nkt) fold(inner, outer);
+        for (int b = 0; b < in_round; ++b) outer[0] += sum[(b * 4 + w) * 64 + lane];
+        __syncthreads();  // before the next round's staging
     }
-    store_tile(outer, m0 + wm * 32, n0 + wn * 32, lane, as_global(g.C), g.ldc, M, N, g.alpha,
-               g.beta);
+    store_quads<1>(g, m0, n0, lane, w, outer);
+}
+
+// ------------------------------------------------------------ split tile --
+// 64x64 tile on the MFMA cores of a row-major A and B (split_tile.hpp): the BF16
+// pieces, or (F16) the FP16 pieces of every element scaled by its row's (A) or
+// column's (B) exponent, with the sums scaled back when stored.
+template <int NPROD, bool F16>
+__device__ __forceinline__ void tile_split(const DGemm& g, int tm, int tn, float* smem) {
+    using namespace split;
+    const int tid = item_tid(), wave = tid >> 6;
+    const int64_t m0 = (int64_t)tm * kLines, n0 = (int64_t)tn * kLines;
+    Quad<true, gcfloat*> qa;
+    Quad<false, gcfloat*> qb;
+    qa.init(as_global(g.A), g.lda, m0, g.M, tid);
+    qb.init(as_global(g.B), g.ldb, n0, g.N, tid);
+    const int rows = (int)std::min<int64_t>(g.M - m0, kLines);
+    const int cols = (int)std::min<int64_t>(g.N - n0, kLines);
+    gcint* const em = F16 ? as_global(static_cast<const int*>(g.ea)) + m0 : nullptr;
+    gcint* const en = F16 ? as_global(static_cast<const int*>(g.eb)) + n0 : nullptr;
+    const int ea = F16 ? em[std::min(qa.line, rows - 1)] : 0;
+    const int eb = F16 ? en[std::min(qb.line, cols - 1)] : 0;
+    float out[16];
+    tile_sums<NPROD, F16, 1>(qa, qb, ea, eb, g.K, 0, tid,
+                             reinterpret_cast<Staged<NPROD, F16>*>(smem), nullptr, out);
+    store_sums(out, 0, wave >> 1, wave & 1, tid & 63, as_global(g.C) + m0 * g.ldc + n0, g.ldc, rows,
+               cols, g.alpha, g.beta, em, en);
 }
 
 // --------------------------------------------------- scaled FP16 split --
@@ -424,65 +561,6 @@ __global__ __launch_bounds__(NT) void grouped_exps_kernel(const ExpItem* __restr
     }
 }
 
-// The split tile with the scaled FP16 pieces: every element is scaled by
-// its row (A) or column (B) exponent and split into two FP16 pieces as
-// omb_sgemm's packing pass does; the 3 leading products (a0 b1, a1 b0,
-// a0 b0) run on the FP16 MFMA, and the sums are scaled back when stored.
-__device__ __forceinline__ void tile_split16(const DGemm& g, int tm, int tn, uint4* smem) {
-    using namespace split;
-    constexpr int P = 64;
-    const int tid = item_tid(), lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int frow = lane & 31, fh = lane >> 5;
-    const int64_t m0 = (int64_t)tm * P, n0 = (int64_t)tn * P;
-    const int64_t M = g.M, N = g.N, K = g.K;
-    gcfloat* const A = as_global(g.A);
-    gcfloat* const B = as_global(g.B);
-    const int64_t lda = g.lda, ldb = g.ldb;
-    const int ra = tid >> 2, qa = tid & 3;
-    const int rb = tid & 63, qb = tid >> 6;
-    uint2* l2 = reinterpret_cast<uint2*>(smem);
-    const int ex_a = m0 + ra < M ? g.ea[m0 + ra] : 0;
-    const int ex_b = n0 + rb < N ? g.eb[n0 + rb] : 0;
-
-    f32x16 inner[1][1], outer[1][1];
-    inner[0][0] = outer[0][0] = f32x16{};
-    const int64_t nkt = ceil_div(K, TK);
-    for (int64_t kt = 0; kt < nkt; ++kt) {
-        const int64_t k0 = kt * TK;
-        float va[4], vb[4];
-        load_split_slice(A, lda, M, B, ldb, N, K, m0 + ra, k0 + 4 * qa, n0 + rb, k0 + 4 * qb, va, vb);
-        __syncthreads();  // previous slice consumed
-        {
-            typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
-            u16x4 pa[2], pb[2];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                _Float16 h0, h1;
-                split2_f16(ldexpf(va[e], ex_a), h0, h1);
-                pa[0][e] = __builtin_bit_cast(unsigned short, h0);
-                pa[1][e] = __builtin_bit_cast(unsigned short, h1);
-                split2_f16(ldexpf(vb[e], ex_b), h0, h1);
-                pb[0][e] = __builtin_bit_cast(unsigned short, h0);
-                pb[1][e] = __builtin_bit_cast(unsigned short, h1);
-            }
-#pragma unroll
-            for (int pl = 0; pl < 2; ++pl) {
-                l2[2 * (pl * 2 * P + lds_chunk(ra, qa >> 1)) + (qa & 1)] =
-                    __builtin_bit_cast(uint2, pa[pl]);
-                l2[2 * (2 * 2 * P + pl * 2 * P + lds_chunk(rb, qb >> 1)) + (qb & 1)] =
-                    __builtin_bit_cast(uint2, pb[pl]);
-            }
-        }
-        __syncthreads();
-        mfma_slice<3, 1, 1, P, P, f16x8, 2>(smem, wm * 32, wn * 32, frow, fh, inner);
-        if ((kt + 1) % kFoldSlices == 0 || kt + 1 == nkt) fold(inner, outer);
-    }
-    store_tile(outer, m0 + wm * 32, n0 + wn * 32, lane, as_global(g.C), g.ldc, M, N, g.alpha,
-               g.beta, as_global(static_cast<const int*>(g.ea)),
-               as_global(static_cast<const int*>(g.eb)));
-}
-
 // ------------------------------------------------------------- GEMV item --
 __device__ __forceinline__ void gemv_item(const DGemv& v, int chunk) {
     const int tid = item_tid();
@@ -503,19 +581,19 @@ __device__ __forceinline__ void gemv_item(const DGemv& v, int chunk) {
 
 // ------------------------------------------------------- persistent kernel --
 // LDS: the largest plain class footprint (128x64: two buffers of
-// 16 x (132 + 68) floats); the split tile uses 12 KB.
+// 16 x (132 + 68) floats); the split tiles use at most 24 KB.
 constexpr int kSmemFloats = 2 * (16 * (128 + 4) + 16 * (64 + 4)) + 16;
 
-// Slices of global loads in flight for the 32x32 and 64x64 plain tiles (8
-// VGPRs each).
-constexpr int kPrefetch = 4;
+// One build per kind of GEMM item, so that none holds registers for another's
+// (with all in one, the pipelined split tiles cost the plain plan of 4096 GEMMs
+// 860 us instead of 783).  All but KBIG are bounded to 4 workgroups per CU (at
+// most 128 VGPRs): the plain plan of 4096 GEMMs and 4096 GEMVs measured 3.48 ms
+// so, against 3.55-3.63 ms for builds of 129 and 165 VGPRs (3 per CU).  KBIG (128x64
+// tiles too) is bounded to 2.
+enum Kind { KPLAIN, KBIG, KSPLIT6, KSPLIT3, KSPLIT16, NKIND };
 
-// The lite build is bounded to 4 workgroups per CU (at most 128 VGPRs): the
-// C4 plain plan measured 3.48 ms so, against 3.55-3.63 ms for builds of 129
-// and 165 VGPRs (3 per CU) that spent the registers on deeper split-tile
-// prefetch.  The big build (128x64 tiles) is bounded to 2.
-template <bool BIG>
-__global__ __launch_bounds__(NT, BIG ? 2 : 4) void grouped_kernel(PArgs p) {
+template <int KIND>
+__global__ __launch_bounds__(NT, KIND == KBIG ? 2 : 4) void grouped_kernel(PArgs p) {
     __shared__ __attribute__((aligned(16))) float smem[kSmemFloats];
     __shared__ int s_chunk;
     // Chunks of consecutive (cost-sorted) items: workgroup b starts with
@@ -536,21 +614,21 @@ __global__ __launch_bounds__(NT, BIG ? 2 : 4) void grouped_kernel(PArgs p) {
             w.tn = __builtin_amdgcn_readfirstlane(w.tn);
             switch (w.cls) {
                 case C32:
-                    tile_f32<32, 32, 2, 2, kPrefetch>(p.gemms[w.inst], w.tm, w.tn, smem);
+                    if constexpr (KIND <= KBIG)
+                        tile_shared_k(p.gemms[w.inst], w.tm, w.tn, smem);
                     break;
                 case C64:
-                    tile_f32<64, 64, 4, 4, kPrefetch>(p.gemms[w.inst], w.tm, w.tn, smem);
+                    if constexpr (KIND <= KBIG)
+                        tile_quads(p.gemms[w.inst], w.tm, w.tn, smem);
                     break;
                 case C128x64:
-                    if (BIG) tile_f32<128, 64, 8, 4, 1>(p.gemms[w.inst], w.tm, w.tn, smem);
+                    if constexpr (KIND == KBIG)
+                        tile_f32<128, 64, 8, 4, 1>(p.gemms[w.inst], w.tm, w.tn, smem);
                     break;
                 case CSPLIT:
-                    if (p.f16)
-                        tile_split16(p.gemms[w.inst], w.tm, w.tn, reinterpret_cast<uint4*>(smem));
-                    else if (p.nprod == 3)
-                        tile_split<3>(p.gemms[w.inst], w.tm, w.tn, reinterpret_cast<uint4*>(smem));
-                    else
-                        tile_split<6>(p.gemms[w.inst], w.tm, w.tn, reinterpret_cast<uint4*>(smem));
+                    if constexpr (KIND >= KSPLIT6)
+                        tile_split<KIND == KSPLIT6 ? 6 : 3, KIND == KSPLIT16>(p.gemms[w.inst], w.tm,
+                                                                             w.tn, smem);
                     break;
                 case CGEMV: gemv_item(p.gemvs[w.inst], w.tm); break;
                 default: break;
@@ -566,6 +644,24 @@ __global__ __launch_bounds__(NT, BIG ? 2 : 4) void grouped_kernel(PArgs p) {
         atomicExch(&p.counters[0], 0u);
         atomicExch(&p.counters[1], 0u);
     }
+}
+
+typedef void (*GroupedKernel)(PArgs);
+GroupedKernel grouped_kernel_of(Kind k) {
+    switch (k) {
+        case KBIG: return grouped_kernel<KBIG>;
+        case KSPLIT6: return grouped_kernel<KSPLIT6>;
+        case KSPLIT3: return grouped_kernel<KSPLIT3>;
+        case KSPLIT16: return grouped_kernel<KSPLIT16>;
+        default: return grouped_kernel<KPLAIN>;
+    }
+}
+Kind kind_of(int mode, bool big) {
+    return mode == OMB_MODE_SPLIT_FP16      ? KSPLIT16
+           : mode == OMB_MODE_SPLIT_BF16_P3 ? KSPLIT3
+           : mode == OMB_MODE_SPLIT_BF16    ? KSPLIT6
+           : big                            ? KBIG
+                                            : KPLAIN;
 }
 
 // ---------------------------------------------------------- tuning table --
@@ -587,15 +683,16 @@ int lg(int64_t x) {
 
 Key key_of(int mode, const omb_gemm_desc& d) { return Key{mode, lg(d.M), lg(d.N), lg(d.K)}; }
 
-// Class without a tuning entry: split mode has one class; plain takes 32x32
-// tiles when the smaller output dimension is under 48, else 64x64.  (The
+// Class without a tuning entry: split mode has one class; plain takes 64x64, or
+// 32x32 with K shared by the wavefronts when the smaller output dimension is under
+// 48 and K has three accumulation blocks or more (4096 GEMMs: 621 us so, 648 with
+// every short side in 32x32, 613 with none, 684 with every such K).  (The
 // 128x64 class needs the larger-register kernel, 2 workgroups per CU instead
-// of 3, which slows every other item of a mixed plan; at C4's shapes 64x64
-// gives the same total rate, so 128x64 is used only when a loaded tuning
-// table names it.)
+// of 4, which slows every other item of a mixed plan, so it is used only when a
+// loaded tuning table names it.)
 int default_class(int mode, const omb_gemm_desc& d) {
     if (mode != OMB_MODE_PLAIN_F32) return CSPLIT;
-    return std::min(d.M, d.N) < 48 ? C32 : C64;
+    return d.K > 2 * kFoldK && std::min(d.M, d.N) < 48 ? C32 : C64;
 }
 
 // The table's class for the bucket, if it computes this mode (the loader
@@ -660,11 +757,9 @@ omb_status validate(const omb_gemm_desc* gemms, int32_t n_gemm, const omb_gemv_d
     return OMB_OK;
 }
 
-// Estimated seconds of one workgroup on one CU (for longest-first order).
 // Estimated seconds one workgroup spends on an item (for the longest-first
-// order): per-workgroup rates measured on MI355X with 3 workgroups per CU --
-// 32x32 16 GFLOP/s, 64x64 40, 128x64 59, split 64x64 54 (FP32-equivalent),
-// GEMV 8 GB/s -- plus about 2 us of fixed cost per item.
+// order): per-workgroup rates -- 32x32 16 GFLOP/s, 64x64 40, 128x64 59, split
+// 64x64 54 (FP32-equivalent), GEMV 8 GB/s -- plus about 2 us of fixed cost per item.
 double item_cost(const Item& it, const std::vector<DGemm>& g, const std::vector<DGemv>& v) {
     constexpr double kFixed = 2.0e-6;
     if (it.cls == CGEMV) return kFixed + 64.0 * (double)v[it.inst].N * 4.0 / 8.0e9;
@@ -702,14 +797,9 @@ omb_status launch_plan(omb_group_plan* p, hipStream_t s) {
                            p->d_gemms);
         OMB_HIP_TRY(hipGetLastError());
     }
-    const bool f16 = p->mode == OMB_MODE_SPLIT_FP16;
-    PArgs a{p->d_items, p->nitems, p->d_gemms, p->d_gemvs, p->d_counters,
-            p->mode == OMB_MODE_SPLIT_BF16_P3 || f16 ? 3 : 6, f16 ? 1 : 0, p->chunk,
+    PArgs a{p->d_items, p->nitems, p->d_gemms, p->d_gemvs, p->d_counters, p->chunk,
             (int)ceil_div(p->nitems, p->chunk)};
-    if (p->big)
-        hipLaunchKernelGGL(grouped_kernel<true>, dim3(p->grid), dim3(NT), 0, s, a);
-    else
-        hipLaunchKernelGGL(grouped_kernel<false>, dim3(p->grid), dim3(NT), 0, s, a);
+    hipLaunchKernelGGL(grouped_kernel_of(kind_of(p->mode, p->big)), dim3(p->grid), dim3(NT), 0, s, a);
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
@@ -820,8 +910,8 @@ omb_status build_plan(const omb_gemm_desc* gemms, int32_t n_gemm, const omb_gemv
         return OMB_EDEVICE;
     }
     cus = prop.multiProcessorCount;
-    hipError_t e = p->big ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, grouped_kernel<true>, NT, 0)
-                          : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, grouped_kernel<false>, NT, 0);
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per_cu, grouped_kernel_of(kind_of(p->mode, p->big)), NT, 0);
     if (e != hipSuccess || per_cu < 1) per_cu = 1;
     p->dev = dev;
     p->grid = std::max(1, std::min(p->nitems, cus * per_cu));
@@ -1097,21 +1187,22 @@ size_t batch_block_bytes() {
            round_up(sizeof(DGemv) * kBatchMaxGemvs, 256) + sizeof(Item) * kBatchMaxItems;
 }
 
-int lite_per_cu() {
-    static int per_cu = -1;
+// Resident workgroups per CU of a kind's kernel.
+int kind_per_cu(Kind k) {
+    static int per_cu[NKIND] = {};
     static std::mutex mu;
     std::lock_guard<std::mutex> lock(mu);
-    if (per_cu < 0) {
+    if (per_cu[k] == 0) {
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, grouped_kernel<false>, NT, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, grouped_kernel_of(k), NT, 0) !=
                 hipSuccess ||
             v < 1) {
             (void)hipGetLastError();
             v = 1;
         }
-        per_cu = v;
+        per_cu[k] = v;
     }
-    return per_cu;
+    return per_cu[k];
 }
 }  // namespace
 
@@ -1204,29 +1295,32 @@ omb_status batch_launch(GroupBatch* b, const omb_gemm_desc* gemms, int n_gemm,
     // travel too; the block is at most a few hundred KB).
     const size_t used = ioff + sizeof(Item) * (size_t)nitems;
     OMB_HIP_TRY(hipMemcpyAsync(b->dev, b->host, used, hipMemcpyHostToDevice, s));
-    const int grid = std::max(1, std::min(nitems, device_cu_count() * lite_per_cu()));
+    const Kind kind = kind_of(mode, false);
+    const int grid = std::max(1, std::min(nitems, device_cu_count() * kind_per_cu(kind)));
     const int chunk = std::max(1, std::min(4, nitems / (8 * grid)));
     PArgs a{reinterpret_cast<const Item*>(b->dev + ioff), nitems,
             reinterpret_cast<const DGemm*>(b->dev), reinterpret_cast<const DGemv*>(b->dev + voff),
-            b->counters, mode == OMB_MODE_SPLIT_BF16_P3 ? 3 : 6, 0, chunk,
-            (int)ceil_div(nitems, chunk)};
-    hipLaunchKernelGGL(grouped_kernel<false>, dim3(grid), dim3(NT), 0, s, a);
+            b->counters, chunk, (int)ceil_div(nitems, chunk)};
+    hipLaunchKernelGGL(grouped_kernel_of(kind), dim3(grid), dim3(NT), 0, s, a);
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
 
 // The steps of batch_launch over no items: the occupancy query (cached for
 // the process), a copy of the whole pinned block (copies this size run as a
-// runtime kernel, whose first launch is the cost), and the launch, in which one
+// runtime kernel, whose first launch is the cost), and each kind's launch, in which one
 // workgroup finds no chunk (nchunks = 0), reads no item and, as the last
 // workgroup to finish, leaves both counters at zero.
 omb_status batch_warm(GroupBatch* b, hipStream_t s) {
-    (void)lite_per_cu();
     OMB_HIP_TRY(hipMemcpyAsync(b->dev, b->host, b->bytes, hipMemcpyHostToDevice, s));
     PArgs a{reinterpret_cast<const Item*>(b->dev), 0, reinterpret_cast<const DGemm*>(b->dev),
-            reinterpret_cast<const DGemv*>(b->dev), b->counters, 6, 0, 1, 0};
-    hipLaunchKernelGGL(grouped_kernel<false>, dim3(1), dim3(NT), 0, s, a);
-    OMB_HIP_TRY(hipGetLastError());
+            reinterpret_cast<const DGemv*>(b->dev), b->counters, 1, 0};
+    for (int mode : {OMB_MODE_PLAIN_F32, OMB_MODE_SPLIT_BF16, OMB_MODE_SPLIT_BF16_P3}) {
+        const Kind kind = kind_of(mode, false);  // the modes batch_launch takes
+        (void)kind_per_cu(kind);
+        hipLaunchKernelGGL(grouped_kernel_of(kind), dim3(1), dim3(NT), 0, s, a);
+        OMB_HIP_TRY(hipGetLastError());
+    }
     return OMB_OK;
 }
 

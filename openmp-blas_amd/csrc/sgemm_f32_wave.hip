@@ -24,14 +24,13 @@
 #include <algorithm>
 #include <cmath>
 
-#include "common.hpp"
+#include "sgemm_wave.hpp"
 
 namespace omb {
 namespace {
 
-constexpr int BK = 16;
-constexpr int BLOCK_K = 128;  // k per accumulation block, as sgemm_f32.hip
-constexpr int PAD = 4;
+using namespace wave;
+
 constexpr int kGroupM = 8;
 
 struct WArgs {
@@ -46,84 +45,6 @@ struct WArgs {
     int64_t tiles_m, tiles_n;
 };
 
-// Orders a wavefront's LDS writes before its other lanes' reads (and the
-// reverse): the hardware keeps the order, this keeps the compiler's.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// One operand of a wavefront's tile: E rows (of A) or columns (of B^T), called
-// lines, starting at line e0; KC: k is the unit stride.  load() brings a full
-// slice into registers, load_guarded() a partial one, store() puts it into LDS
-// as [k][line].
-template <int E, bool KC, typename Off>
-struct Side {
-    static constexpr int L = E / 16;  // float4 per lane and slice
-    const float* p;  // line e0 (wavefront-uniform, as is the k of a load: the
-                     // loads add a lane's offset to a scalar address)
-    int64_t ld;
-    int n;           // lines of the operand from e0
-    int lane;
-
-    __device__ __forceinline__ void init(const float* X, int64_t ld_, int64_t e0, int64_t extent,
-                                         int lane_) {
-        p = X + (KC ? e0 * ld_ : e0);
-        ld = ld_;
-        n = (int)std::min<int64_t>(extent - e0, E);
-        lane = lane_;
-    }
-    // byte offset of load i: line (KC) or quad of lines, clamped into the operand
-    __device__ __forceinline__ Off offset(int i) const {
-        const int e = lane + 64 * i;
-        return (Off)(4 * (KC ? min(e >> 2, n - 1) * ld + (e & 3) * 4
-                             : (e / (E / 4)) * ld + min(e % (E / 4) * 4, (n - 1) & ~3)));
-    }
-    __device__ __forceinline__ void load(float4 (&v)[L], const Off (&off)[L], int64_t k0) const {
-        const char* q = reinterpret_cast<const char*>(p + (KC ? k0 : k0 * ld));
-#pragma unroll
-        for (int i = 0; i < L; ++i) v[i] = ld4u(reinterpret_cast<const float*>(q + off[i]));
-    }
-    // k steps at the operand's end that a 4-line load could read past: the
-    // last one, or the last three when lines are less than 4 floats apart.
-    __device__ __forceinline__ int tail() const {
-        return KC || n % 4 == 0 ? 0 : (ld < 4 ? 3 : 1);
-    }
-    // k0 .. k1-1 are the valid k of the slice (k1 <= K)
-    __device__ __forceinline__ void load_guarded(float4 (&v)[L], int64_t k0, int64_t k1) const {
-#pragma unroll
-        for (int i = 0; i < L; ++i) {
-            const int e = lane + 64 * i;
-            float t[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int64_t line = min(KC ? e >> 2 : e % (E / 4) * 4 + c, n - 1);
-                const int64_t k = k0 + (KC ? (e & 3) * 4 + c : e / (E / 4));
-                const int64_t b = std::min(k, k1 - 1);
-                const float x = p[KC ? line * ld + b : b * ld + line];
-                t[c] = k < k1 ? x : 0.f;
-            }
-            v[i] = make_float4(t[0], t[1], t[2], t[3]);
-        }
-    }
-    __device__ __forceinline__ void store(float (*s)[E + PAD], const float4 (&v)[L]) const {
-#pragma unroll
-        for (int i = 0; i < L; ++i) {
-            const int e = lane + 64 * i;
-            if constexpr (KC) {
-                const int line = e >> 2, kq = (e & 3) * 4;
-                s[kq + 0][line] = v[i].x;
-                s[kq + 1][line] = v[i].y;
-                s[kq + 2][line] = v[i].z;
-                s[kq + 3][line] = v[i].w;
-            } else {
-                *reinterpret_cast<float4*>(&s[e / (E / 4)][e % (E / 4) * 4]) = v[i];
-            }
-        }
-    }
-};
-
 // GR, GC: 4-row and 4-column groups per lane (8 x 8 lanes: BM = 32*GR, BN =
 // 32*GC); W wavefronts; D slices of loads in flight.
 template <int GR, int GC, int W, int D, int OCC, bool A_KC, bool B_NC, typename Off>
@@ -132,11 +53,8 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
     constexpr int S = TR * GC;            // float4 of the tile per lane
     constexpr int P = S > 4 ? 2 : 1;      // passes of the LDS sum (bounds its LDS)
     constexpr int SP = S / P, OWN = (SP + W - 1) / W;  // float4 per pass; of them, added here
-    struct Stage {
-        float a[BK][BM + PAD], b[BK][BN + PAD];
-    };
     union Shared {
-        Stage stage[W];
+        WaveStage<GR, GC> stage[W];
         acc4 sum[W][SP][64];
     };
     __shared__ __attribute__((aligned(16))) Shared sh;
@@ -146,8 +64,8 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
     int64_t tm, tn;
     group_tile(xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n), p.tiles_m, p.tiles_n, kGroupM, &tm, &tn);
     const int64_t m0 = tm * BM, n0 = tn * BN;
-    Side<BM, A_KC, Off> sa;
-    Side<BN, !B_NC, Off> sb;
+    WaveSide<BM, A_KC, Off, const float*> sa;
+    WaveSide<BN, !B_NC, Off, const float*> sb;
     sa.init(p.A, p.lda, m0, p.M, lane);
     sb.init(p.B, p.ldb, n0, p.N, lane);
     Off oa[sa.L], ob[sb.L];
@@ -158,36 +76,8 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
     const int tail = max(sa.tail(), sb.tail());
 
     acc4 inner[TR][GC];
-    Stage& st = sh.stage[wave];
-    float4 fa[2][GR], fb[2][GC];  // fragments of this k and of the next one
-    auto fragment = [&](int k, int set) {
-#pragma unroll
-        for (int g = 0; g < GR; ++g)
-            fa[set][g] = *reinterpret_cast<const float4*>(&st.a[k][g * 32 + ly * 4]);
-#pragma unroll
-        for (int h = 0; h < GC; ++h)
-            fb[set][h] = *reinterpret_cast<const float4*>(&st.b[k][h * 32 + lx * 4]);
-    };
-    auto compute = [&] {  // the staged slice
-        fragment(0, 0);
-#pragma unroll
-        for (int k = 0; k < BK; ++k) {
-            if (k + 1 < BK) fragment(k + 1, (k + 1) & 1);
-            const float* a = reinterpret_cast<const float*>(fa[k & 1]);
-#pragma unroll
-            for (int i = 0; i < TR; ++i)
-#pragma unroll
-                for (int h = 0; h < GC; ++h) {
-                    const float4 v = fb[k & 1][h];
-                    acc4& s = inner[i][h];
-                    s[acc_slot(0)] = fmaf(a[i], v.x, s[acc_slot(0)]);
-                    s[acc_slot(1)] = fmaf(a[i], v.y, s[acc_slot(1)]);
-                    s[acc_slot(2)] = fmaf(a[i], v.z, s[acc_slot(2)]);
-                    s[acc_slot(3)] = fmaf(a[i], v.w, s[acc_slot(3)]);
-                }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
+    WaveStage<GR, GC>& st = sh.stage[wave];
+    auto compute = [&] { wave_compute<GR, GC>(st, lane, inner); };
 
     acc4 outer[P * OWN];
 #pragma unroll
@@ -222,11 +112,7 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
                 for (int d = 0; d < D; ++d) load(d, kb + d * BK);
                 store(0);
                 for (; s + D <= nfull; s += D) {
-                    // Keeps each tuple in four consecutive registers through the loop.
-#pragma unroll
-                    for (int i = 0; i < TR; ++i)
-#pragma unroll
-                        for (int h = 0; h < GC; ++h) asm volatile("" : "+v"(inner[i][h]));
+                    pin(inner);
 #pragma unroll
                     for (int d = 0; d < D; ++d) {  // slice s + d is staged, set d free
                         load(d, kb + (int64_t)(s + D + d) * BK);

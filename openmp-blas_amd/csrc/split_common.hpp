@@ -48,6 +48,38 @@ __device__ inline void split3(float x, __bf16& h0, __bf16& h1, __bf16& h2) {
     h2 = (__bf16)(r1 - (float)h1);
 }
 
+// The same for four values into PL planes, without a branch: with the value limited
+// to BF16's finite range h0 is split3's (rounded within the range, truncated past
+// it).  An infinite x then leaves an infinite rest, whose own rest is NaN; with two
+// planes 0 * x makes the first rest NaN.
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+template <int PL>
+__device__ __forceinline__ void split3x4(const float (&v)[4], u16x4 (&h)[PL]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        float r0 = v[i], r1 = v[i + 1];
+#pragma unroll
+        for (int pl = 0; pl < PL; ++pl) {
+            const f32x2 x = pl == 0 ? f32x2{__builtin_amdgcn_fmed3f(r0, -0x1.fep127f, 0x1.fep127f),
+                                            __builtin_amdgcn_fmed3f(r1, -0x1.fep127f, 0x1.fep127f)}
+                                    : f32x2{r0, r1};
+            const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector(x, bf16x2));
+            h[pl][i] = (unsigned short)u;
+            h[pl][i + 1] = (unsigned short)(u >> 16);
+            if (pl + 1 < PL) {
+                r0 -= __uint_as_float(u << 16);
+                r1 -= __uint_as_float(u & 0xffff0000u);
+            }
+            if (PL == 2 && pl == 0) {
+                r0 = fmaf(0.f, v[i], r0);
+                r1 = fmaf(0.f, v[i + 1], r1);
+            }
+        }
+    }
+}
+
 // Scaled FP16 split (two planes per packed slice): the power-of-two exponent
 // that brings a line whose largest magnitude is amax into [2^14, 2^15) (0
 // for a zero, infinite or NaN amax), and x * 2^e = h0 + h1 + r with
