@@ -760,12 +760,17 @@ omb_status validate(const omb_gemm_desc* gemms, int32_t n_gemm, const omb_gemv_d
 // Estimated seconds one workgroup spends on an item (for the longest-first
 // order): per-workgroup rates -- 32x32 16 GFLOP/s, 64x64 40, 128x64 59, split
 // 64x64 54 (FP32-equivalent), GEMV 8 GB/s -- plus about 2 us of fixed cost per item.
+// GEMM items count a quarter, so that most follow the GEMV items: the two kinds
+// side by side are slower than one after the other (4096 GEMMs alone 613 us, 4096
+// GEMVs alone 2608; mixed by equal weights 3356, GEMMs first 3212, GEMVs first 3187,
+// at a quarter 3180; 300 of each 314, 329, 321, 314).
+constexpr double kGemmOrder = 0.25;
 double item_cost(const Item& it, const std::vector<DGemm>& g, const std::vector<DGemv>& v) {
     constexpr double kFixed = 2.0e-6;
     if (it.cls == CGEMV) return kFixed + 64.0 * (double)v[it.inst].N * 4.0 / 8.0e9;
     static const double rate[NCLS] = {16e9, 40e9, 59e9, 54e9, 0.0};
-    return kFixed + 2.0 * kTileM[it.cls] * kTileN[it.cls] *
-                        (double)std::max<int64_t>(g[it.inst].K, 1) / rate[it.cls];
+    return kGemmOrder * (kFixed + 2.0 * kTileM[it.cls] * kTileN[it.cls] *
+                                      (double)std::max<int64_t>(g[it.inst].K, 1) / rate[it.cls]);
 }
 
 template <typename T>
