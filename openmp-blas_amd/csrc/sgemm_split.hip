@@ -165,22 +165,25 @@ __global__ __launch_bounds__(NT) void split_pack_kernel(const float* __restrict_
 }
 
 // Both operands of one product in one launch (same K): row tiles of the
-// first, then of the second, along blockIdx.x.
+// first, then of the second, along blockIdx.x.  amax, exps: the row maxima's bits
+// and where the exponents go (scaled FP16 split only).
 struct PackOperand {
     const float* X;
     int64_t R, rs, cs;
     int k_major;
     __bf16* out;
     int64_t rtiles;
+    unsigned* amax;
+    int* exps;
 };
-template <int PLN>
+template <bool F16, int PLN>
 __global__ __launch_bounds__(NT) void split_pack_pair_kernel(PackOperand a, PackOperand b,
                                                              int64_t K, int64_t nkt) {
     const bool first = (int64_t)blockIdx.x < a.rtiles;
     const PackOperand& o = first ? a : b;
     const int64_t rt = first ? (int64_t)blockIdx.x : (int64_t)blockIdx.x - a.rtiles;
-    pack_tile<false, PLN>(o.X, o.R, K, o.rs, o.cs, nkt, o.k_major, o.out, nullptr, nullptr, rt,
-                          blockIdx.y);
+    pack_tile<F16, PLN>(o.X, o.R, K, o.rs, o.cs, nkt, o.k_major, o.out, o.amax, o.exps, rt,
+                        blockIdx.y);
 }
 
 // ----------------------------------------------------------------- pass 2 --
@@ -355,50 +358,76 @@ __global__ __launch_bounds__(NT, 2) void sgemm_bf16x3_kernel(MArgs p) {
 }
 
 // ------------------------------------------------- scaled FP16 split --
-// Largest magnitude of every row of an R x K operand (element (r, k) at
+// Largest magnitude of every row of both operands (element (r, k) at
 // X[r*rs + k*cs]), as the bits of |x| (for non-negative floats the unsigned
 // order is the numeric order, and NaN's bits exceed infinity's, so a NaN
 // row max is NaN).  The order of a max does not matter: deterministic.
-// k-contiguous rows (cs == 1): one wavefront per row, written directly.
-__global__ __launch_bounds__(NT) void amax_rows_kc_kernel(const float* __restrict__ X,
-                                                          int64_t R, int64_t K, int64_t rs,
-                                                          unsigned* __restrict__ amax) {
-    const int lane = threadIdx.x & 63;
-    const int64_t r = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    if (r >= R) return;
-    const float* row = X + r * rs;
-    unsigned m = 0;
-    const int64_t n4 = K >> 2;
-    for (int64_t j = lane; j < n4; j += 64) {
-        const float4 v = ld4u_nt(row + 4 * j);
-        m = max(m, max(max(__float_as_uint(fabsf(v.x)), __float_as_uint(fabsf(v.y))),
-                       max(__float_as_uint(fabsf(v.z)), __float_as_uint(fabsf(v.w)))));
-    }
-    const int64_t t = (n4 << 2) + lane;
-    if (t < K) m = max(m, __float_as_uint(fabsf(row[t])));
+//
+// One launch for the pair, 32 rows per 1024-thread workgroup through all of K
+// (few long rows: through a k range per blockIdx.y, combined by atomics into zeroed
+// maxima), so that they need no zeroing and no second pass; a thread keeps eight 128-bit
+// loads in flight along the unit stride (a wavefront per two rows where that is
+// k, 128 bytes of each of 128 k where it is the rows).  A product of 1024^3 took 48 us
+// (k contiguous in both) to 89 (rows contiguous in both) with maxima and pack
+// launches per operand, and for adjacent rows one that zeroes and one of 256-k chunks
+// combined by atomics; 41 to 43 so.  2600 x 2400 x 1700: 141-182, 135-140;
+// 64 x 64 x 60000: 137-276, 70-77; 8192^3: 3763-3777, 3746-3768.
+constexpr int kAmaxRows = 32, kAmaxThreads = 1024;
+constexpr int64_t kAmaxRange = 4096;  // least k of a range
+__global__ __launch_bounds__(kAmaxThreads) void amax_pair_kernel(PackOperand a, PackOperand b,
+                                                                 int64_t K, int64_t groups_a,
+                                                                 int64_t range) {
+    __shared__ unsigned top[kAmaxRows];
+    const bool first = (int64_t)blockIdx.x < groups_a;
+    const PackOperand& o = first ? a : b;
+    const int64_t kb = (int64_t)blockIdx.y * range;
+    const float* const X = o.X + kb * o.cs;
+    K = std::min(K - kb, range);
+    const int64_t r0 = ((int64_t)blockIdx.x - (first ? 0 : groups_a)) * kAmaxRows;
+    const int rows = (int)std::min<int64_t>(o.R - r0, kAmaxRows), tid = threadIdx.x;
+    auto most = [](unsigned m, float4 v) {
+        return max(m, max(max(__float_as_uint(fabsf(v.x)), __float_as_uint(fabsf(v.y))),
+                          max(__float_as_uint(fabsf(v.z)), __float_as_uint(fabsf(v.w)))));
+    };
+    if (tid < kAmaxRows) top[tid] = 0u;
+    __syncthreads();
+    if (o.cs == 1) {
+        // loads past a row's last whole quad repeat it
+        const int lane = tid & 63, w = tid >> 6;
+        const int64_t n4 = K >> 2;
+        const float* row[2] = {X + (r0 + min(w, rows - 1)) * o.rs,
+                               X + (r0 + min(w + 16, rows - 1)) * o.rs};
+        unsigned m[2] = {0u, 0u};
+        for (int64_t j = lane; j - lane < n4; j += 4 * 64) {
+            float4 v[4][2];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off, 64));
-    if (lane == 0) amax[r] = m;
-}
-
-// Other layouts, over 256-k chunks combined with atomicMax into a zeroed
-// `amax`.  rs == 1 (consecutive rows adjacent in memory): one thread per 4
-// rows, one 128-bit load per k (1 KB per wavefront), 8 k in flight.
-constexpr int kAmaxChunk = 256;
-__global__ __launch_bounds__(NT) void amax_rows4_kernel(const float* __restrict__ X, int64_t R,
-                                                        int64_t K, int64_t cs,
-                                                        unsigned* __restrict__ amax) {
-    const int64_t r = ((int64_t)blockIdx.x * NT + threadIdx.x) * 4;
-    if (r >= R) return;
-    const int64_t k0 = (int64_t)blockIdx.y * kAmaxChunk;
-    const int64_t k1 = k0 + kAmaxChunk < K ? k0 + kAmaxChunk : K;
-    unsigned m[4] = {0u, 0u, 0u, 0u};
-    int64_t k = k0;
-    if (r + 3 < R) {
-        for (; k + 8 <= k1; k += 8) {
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    v[u][q] = ld4u_nt(row[q] + 4 * std::min(j + u * 64, n4 - 1));
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) m[q] = most(m[q], v[u][q]);
+        }
+        const int64_t t = (n4 << 2) + lane;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            if (t < K) m[q] = max(m[q], __float_as_uint(fabsf(row[q][t])));
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1)
+                m[q] = max(m[q], (unsigned)__shfl_xor((int)m[q], off, 64));
+            if (lane == 0) top[w + 16 * q] = m[q];
+        }
+    } else if (o.rs == 1 && o.R >= 4) {
+        // quads past the last row repeat the last four
+        const int c = std::min<int64_t>(r0 + (tid & 7) * 4, o.R - 4) - r0;
+        const float* p = X + r0 + c;
+        unsigned m[4] = {0u, 0u, 0u, 0u};
+        for (int64_t k = tid >> 3; k - (tid >> 3) < K; k += 8 * 128) {
             float4 v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = ld4u_nt(X + r + (k + u) * cs);
+            for (int u = 0; u < 8; ++u) v[u] = ld4u_nt(p + std::min(k + u * 128, K - 1) * o.cs);
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 m[0] = max(m[0], __float_as_uint(fabsf(v[u].x)));
@@ -407,28 +436,22 @@ __global__ __launch_bounds__(NT) void amax_rows4_kernel(const float* __restrict_
                 m[3] = max(m[3], __float_as_uint(fabsf(v[u].w)));
             }
         }
-    }
-    for (; k < k1; ++k)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            if (r + e < R) m[e] = max(m[e], __float_as_uint(fabsf(X[r + e + k * cs])));
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (r + e < R) atomicMax(&amax[r + e], m[e]);
-}
-
-// Any strides: one thread per row.
-__global__ __launch_bounds__(NT) void amax_rows_any_kernel(const float* __restrict__ X,
-                                                           int64_t R, int64_t K, int64_t rs,
-                                                           int64_t cs,
-                                                           unsigned* __restrict__ amax) {
-    const int64_t r = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (r >= R) return;
-    const int64_t k0 = (int64_t)blockIdx.y * kAmaxChunk;
-    const int64_t k1 = k0 + kAmaxChunk < K ? k0 + kAmaxChunk : K;
-    unsigned m = 0;
-    for (int64_t k = k0; k < k1; ++k) m = max(m, __float_as_uint(fabsf(X[r * rs + k * cs])));
-    atomicMax(&amax[r], m);
+            if (c + e >= 0) atomicMax(&top[c + e], m[e]);
+    } else {
+        const int r = tid & (kAmaxRows - 1);
+        unsigned m = 0u;
+        if (r < rows)
+            for (int64_t k = tid / kAmaxRows; k < K; k += kAmaxThreads / kAmaxRows)
+                m = max(m, __float_as_uint(fabsf(X[(r0 + r) * o.rs + k * o.cs])));
+        atomicMax(&top[r], m);
+    }
+    __syncthreads();
+    if (tid < rows) {
+        if (gridDim.y > 1) atomicMax(&o.amax[r0 + tid], top[tid]);
+        else o.amax[r0 + tid] = top[tid];
+    }
 }
 
 __global__ __launch_bounds__(NT) void zero_u32_kernel(unsigned* p, int64_t n) {
@@ -475,50 +498,50 @@ omb_status launch_split_pack_pair(int64_t M, int64_t N, int64_t K, const float* 
                                   int64_t csB, __bf16* bp, hipStream_t s, int planes) {
     if (K <= 0 || (M <= 0 && N <= 0)) return OMB_OK;
     const int64_t nkt = ceil_div(K, TK), kgroups = ceil_div(nkt, SPLIT_SL);
-    const PackOperand a{A, M, rsA, csA, csA == 1 ? 1 : 0, ap, M > 0 ? ceil_div(M, TM) : 0};
-    const PackOperand b{Bt, N, rsB, csB, csB == 1 ? 1 : 0, bp, N > 0 ? ceil_div(N, TM) : 0};
+    const PackOperand a{A, M, rsA, csA, csA == 1 ? 1 : 0, ap, M > 0 ? ceil_div(M, TM) : 0,
+                        nullptr, nullptr};
+    const PackOperand b{Bt, N, rsB, csB, csB == 1 ? 1 : 0, bp, N > 0 ? ceil_div(N, TM) : 0,
+                        nullptr, nullptr};
     if (a.rtiles + b.rtiles > 0x7fffffffLL || kgroups > 65535) {
         set_error("split pack: operands too large for one launch");
         return OMB_EUNSUPPORTED;
     }
     const dim3 grid((unsigned)(a.rtiles + b.rtiles), (unsigned)kgroups);
     if (planes == 2)
-        hipLaunchKernelGGL(split_pack_pair_kernel<2>, grid, dim3(NT), 0, s, a, b, K, nkt);
+        hipLaunchKernelGGL((split_pack_pair_kernel<false, 2>), grid, dim3(NT), 0, s, a, b, K, nkt);
     else
-        hipLaunchKernelGGL(split_pack_pair_kernel<3>, grid, dim3(NT), 0, s, a, b, K, nkt);
+        hipLaunchKernelGGL((split_pack_pair_kernel<false, 3>), grid, dim3(NT), 0, s, a, b, K, nkt);
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
 
-omb_status launch_split16_pack(int64_t R, int64_t K, const float* X, int64_t rs, int64_t cs,
-                               __bf16* out, unsigned* amax, int* exps, hipStream_t s) {
-    if (R <= 0 || K <= 0) return OMB_OK;
-    const int64_t rtiles = ceil_div(R, TM), nkt = ceil_div(K, TK);
-    const int64_t kgroups = ceil_div(nkt, SPLIT_SL);
-    const int64_t achunks = ceil_div(K, kAmaxChunk);
-    if (rtiles > 0x7fffffffLL || kgroups > 65535 || achunks > 65535) {
-        set_error("split pack: operand too large for one launch");
+// Row maxima of A and B^T (amax_b follows amax_a), then both packed in their scaled
+// FP16 pieces.
+omb_status launch_split16_pack_pair(int64_t M, int64_t N, int64_t K, const float* A, int64_t rsA,
+                                    int64_t csA, __bf16* ap, unsigned* amax_a, int* ea,
+                                    const float* Bt, int64_t rsB, int64_t csB, __bf16* bp,
+                                    unsigned* amax_b, int* eb, hipStream_t s) {
+    if (K <= 0 || M <= 0 || N <= 0) return OMB_OK;
+    const int64_t nkt = ceil_div(K, TK), kgroups = ceil_div(nkt, SPLIT_SL);
+    const PackOperand a{A, M, rsA, csA, csA == 1 ? 1 : 0, ap, ceil_div(M, TM), amax_a, ea};
+    const PackOperand b{Bt, N, rsB, csB, csB == 1 ? 1 : 0, bp, ceil_div(N, TM), amax_b, eb};
+    const int64_t ga = ceil_div(M, (int64_t)kAmaxRows), gb = ceil_div(N, (int64_t)kAmaxRows);
+    if (ga + gb > 0x7fffffffLL || kgroups > 65535) {
+        set_error("split pack: operands too large for one launch");
         return OMB_EUNSUPPORTED;
     }
-    if (cs == 1) {
-        hipLaunchKernelGGL(amax_rows_kc_kernel, dim3((unsigned)ceil_div(R, NT / 64)), dim3(NT), 0,
-                           s, X, R, K, rs, amax);
-    } else {
-        hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(R, NT), 1024)),
-                           dim3(NT), 0, s, amax, R);
-        if (rs == 1)
-            hipLaunchKernelGGL(amax_rows4_kernel,
-                               dim3((unsigned)ceil_div(R, 4 * NT), (unsigned)achunks), dim3(NT), 0,
-                               s, X, R, K, cs, amax);
-        else
-            hipLaunchKernelGGL(amax_rows_any_kernel,
-                               dim3((unsigned)ceil_div(R, NT), (unsigned)achunks), dim3(NT), 0, s,
-                               X, R, K, rs, cs, amax);
-    }
-    OMB_HIP_TRY(hipGetLastError());
-    const int k_major = cs == 1 ? 1 : 0;
-    hipLaunchKernelGGL((split_pack_kernel<true, 2>), dim3((unsigned)rtiles, (unsigned)kgroups),
-                       dim3(NT), 0, s, X, R, K, rs, cs, nkt, k_major, out, amax, exps);
+    // k ranges of whole 128-byte lines when the row groups alone leave CUs idle
+    const int64_t ranges = std::max<int64_t>(
+        1, std::min<int64_t>(2 * device_cu_count() / (ga + gb), K / kAmaxRange));
+    const int64_t range = round_up(ceil_div(K, ranges), kLineFloats);
+    if (ranges > 1)
+        hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(M + N, NT), 1024)),
+                           dim3(NT), 0, s, amax_a, M + N);
+    hipLaunchKernelGGL(amax_pair_kernel, dim3((unsigned)(ga + gb), (unsigned)ceil_div(K, range)),
+                       dim3(kAmaxThreads), 0, s, a, b, K, ga, range);
+    hipLaunchKernelGGL((split_pack_pair_kernel<true, 2>),
+                       dim3((unsigned)(a.rtiles + b.rtiles), (unsigned)kgroups), dim3(NT), 0, s, a, b,
+                       K, nkt);
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
@@ -636,8 +659,8 @@ omb_status launch_sgemm_split16_ws(int64_t M, int64_t N, int64_t K, float alpha,
     float* part =
         splits > 1 ? reinterpret_cast<float*>(ws + packed + split16_extra_bytes(M, N)) : nullptr;
     // A scaled by rows, B^T (rows n) by rows, i.e. B by columns.
-    OMB_TRY(launch_split16_pack(M, K, A, rsA, csA, ap, amax_a, ea, s));
-    OMB_TRY(launch_split16_pack(N, K, B, csB, rsB, bp, amax_b, eb, s));
+    OMB_TRY(launch_split16_pack_pair(M, N, K, A, rsA, csA, ap, amax_a, ea, B, csB, rsB, bp, amax_b, eb,
+                                     s));
     return launch_sgemm_packed(M, N, K, alpha, ap, bp, beta, C, ldc, 3, s, part, ea, eb, 2);
 }
 
