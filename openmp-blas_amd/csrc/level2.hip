@@ -219,8 +219,8 @@ __device__ inline void tile_put(float (*tile)[TPAD], const float4 (&v)[TT / 16])
 // without, 99 us with it, 16384^2 462 and 412 us; other strides lose 2-9%
 // by it (8000 x 12032: 144 and 158 us).
 template <int RT, int CT>
-__global__ __launch_bounds__(NT) void transpose_lines_kernel(int64_t R, int64_t Cc, int64_t GR,
-                                                             int64_t GC,
+__global__ __launch_bounds__(NT) void transpose_lines_kernel(int64_t R, int64_t Cc, unsigned GR,
+                                                             unsigned GC,
                                                              const float* __restrict__ S,
                                                              int64_t lds, float* __restrict__ D,
                                                              int64_t ldd, int on_lines, int diag) {
@@ -231,12 +231,14 @@ __global__ __launch_bounds__(NT) void transpose_lines_kernel(int64_t R, int64_t 
     __shared__ float tile[LR][CT + 1];
     const int cq = threadIdx.x % CQ, rr = threadIdx.x / CQ;
     const int g = threadIdx.x % RQ, cc = threadIdx.x / RQ;
-    const int64_t ntiles = GR * GC;
+    const uint64_t ntiles = (uint64_t)GR * GC;
     // XCD x (workgroups x mod 8) takes tiles [x, x+1) * ntiles / 8, r fastest.
-    const int64_t x = blockIdx.x & 7, end = ntiles * (x + 1) / 8;
-    for (int64_t t = ntiles * x / 8 + (blockIdx.x >> 3); t < end; t += gridDim.x >> 3) {
-        const int64_t gr = t % GR, gc = diag ? (t / GR + gr) % GC : t / GR;
-        const int64_t r0 = gr * RT, c0 = gc * CT;
+    const unsigned x = blockIdx.x & 7;
+    const uint64_t end = ntiles * (x + 1) / 8;
+    for (uint64_t t = ntiles * x / 8 + (blockIdx.x >> 3); t < end; t += gridDim.x >> 3) {
+        // t < 2^32: a matrix of that many tiles is 32 TB
+        const unsigned q = (unsigned)t / GR, gr = (unsigned)t % GR, gc = diag ? (q + gr) % GC : q;
+        const int64_t r0 = (int64_t)gr * RT, c0 = (int64_t)gc * CT;
         const bool full = (on_lines || r0 >= kLine) && r0 + RT <= R && c0 + CT <= Cc;
         float4 v[LR / RPI];
         if (full) {
@@ -417,7 +419,7 @@ extern "C" omb_status omb_stranspose(int64_t M, int64_t N, const float* A, int64
         const int64_t GR = ceil_div(R + (on_lines ? 0 : kLine - 1), rt), GC = ceil_div(Cc, ct);
         const dim3 grid((unsigned)std::min<int64_t>(round_up(GR * GC, 8), 1 << 24));
         const auto kernel = big ? transpose_lines_kernel<128, 64> : transpose_lines_kernel<64, 32>;
-        hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, s, R, Cc, GR, GC, A, lda, C, ldc,
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, s, R, Cc, (unsigned)GR, (unsigned)GC, A, lda, C, ldc,
                            on_lines ? 1 : 0, diag ? 1 : 0);
     } else {
         // whole-line groups of C are whole-line groups of A on every row

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
 
     const int tid = threadIdx.x;
     const int64_t ntiles = p.tiles_m * p.tiles_n;
-    int64_t t = xcd_remap(blockIdx.x, ntiles);
+    const unsigned t = xcd_remap(blockIdx.x, (unsigned)ntiles);
     int64_t tm, tn;
     group_tile(t, p.tiles_m, p.tiles_n, kGroupM, &tm, &tn);
     const int64_t m0 = tm * BM, n0 = tn * BN;

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lx = lane & 7, ly = lane >> 3;
     int64_t tm, tn;
-    group_tile(xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n), p.tiles_m, p.tiles_n, kGroupM, &tm, &tn);
+    group_tile(xcd_remap(blockIdx.x, (unsigned)(p.tiles_m * p.tiles_n)), p.tiles_m, p.tiles_n, kGroupM, &tm, &tn);
     const int64_t m0 = tm * BM, n0 = tn * BN;
     WaveSide<BM, A_KC, Off, const float*> sa;
     WaveSide<BN, !B_NC, Off, const float*> sb;

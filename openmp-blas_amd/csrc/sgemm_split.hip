@@ -246,7 +246,7 @@ __global__ __launch_bounds__(NT, 2) void sgemm_bf16x3_kernel(MArgs p) {
     const int lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int64_t ntiles = p.tiles_m * p.tiles_n;
-    int64_t t = xcd_remap(blockIdx.x, ntiles);
+    const unsigned t = xcd_remap(blockIdx.x, (unsigned)ntiles);
     int64_t tm, tn;
     group_tile(t, p.tiles_m, p.tiles_n, kGroupM, &tm, &tn);
 

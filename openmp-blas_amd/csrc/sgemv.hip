@@ -104,8 +104,8 @@ __global__ __launch_bounds__(NT) void sgemv_col_kernel(int64_t M, int64_t N, flo
                                                        int64_t mpad, int nrb, int nchunks,
                                                        int64_t cols_per_chunk, unsigned* count) {
     constexpr int CG = 64 / LR, STEP = 4 * CG, RB = 4 * LR;
-    const int64_t b = xcd_remap(blockIdx.x, (int64_t)gridDim.x);
-    const int rb = (int)(b % nrb), ch = (int)(b / nrb);
+    const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
+    const int rb = (int)(b % (unsigned)nrb), ch = (int)(b / (unsigned)nrb);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int cg = lane / LR;
     const int64_t r0 = (int64_t)rb * RB;
