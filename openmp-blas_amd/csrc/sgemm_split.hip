@@ -348,13 +348,14 @@ __global__ __launch_bounds__(NT, 2) void sgemm_bf16x3_kernel(MArgs p) {
 
     // (The exponents scale a split's partial sums before they are stored:
     // a power-of-two scale commutes with the in-order sum of the partials.)
+    constexpr bool kExps = std::is_same<V, f16x8>::value;
     if (p.part)  // partial sums of this split (alpha 1, beta 0 store them unchanged)
-        store_tile(outer, tm * TM + wm * 64, tn * TN + wn * 64, lane,
-                   p.part + (int64_t)blockIdx.y * p.M * p.N, p.N, p.M, p.N, 1.f, 0.f, p.ea,
-                   p.eb);
+        store_tile<kExps>(outer, tm * TM + wm * 64, tn * TN + wn * 64, lane,
+                          p.part + (int64_t)blockIdx.y * p.M * p.N, p.N, p.M, p.N, 1.f, 0.f, p.ea,
+                          p.eb);
     else
-        store_tile(outer, tm * TM + wm * 64, tn * TN + wn * 64, lane, p.C, p.ldc, p.M, p.N,
-                   p.alpha, p.beta, p.ea, p.eb);
+        store_tile<kExps>(outer, tm * TM + wm * 64, tn * TN + wn * 64, lane, p.C, p.ldc, p.M, p.N,
+                          p.alpha, p.beta, p.ea, p.eb);
 }
 
 // ------------------------------------------------- scaled FP16 split --
