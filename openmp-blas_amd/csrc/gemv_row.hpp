@@ -31,9 +31,7 @@ __device__ inline P wave_uniform_ptr(P p) {
 constexpr int64_t kGemvOff32Cols = (int64_t)1 << 29;
 
 // (PA / PX / PY: generic or global-address-space pointers.  STREAM: rows of A
-// are loaded with the non-temporal hint; the grouped kernel, whose items
-// are short and share cache lines across item boundaries, loads them
-// normally -- measured 3.5% faster there.  OFF32, for N < kGemvOff32Cols and
+// are loaded with the non-temporal hint.  OFF32, for N < kGemvOff32Cols and
 // a wavefront-uniform r0: the row bases are scalar and every load adds one
 // 32-bit lane offset, which frees about 90 VGPRs of per-row addresses and
 // measured 1.5% more bandwidth in the standalone row kernel, 0.8% in the
@@ -43,9 +41,11 @@ constexpr int64_t kGemvOff32Cols = (int64_t)1 << 29;
 // without it the compiler consumes loads as they come and the last groups
 // are one round trip each (9003 x 6001 with 2 x 8: 34.7 us, 4 x 4 without
 // BATCH: 43.1).  The 16 x 1 form is the exception: its rounds overlap without
-// a barrier.)
-template <int ROWS, int UNROLL, bool STREAM, bool OFF32 = false, bool BATCH = false, typename PA,
-          typename PX, typename PY>
+// a barrier.  EXACT: the last round has only the loads that its row needs, all
+// with STREAM's hint, for callers whose rows are mostly one to three rounds; on
+// long rows it measured the same.)
+template <int ROWS, int UNROLL, bool STREAM, bool OFF32 = false, bool BATCH = false,
+          bool EXACT = false, typename PA, typename PX, typename PY>
 __device__ __forceinline__ void gemv_rows_wave(int64_t r0, int nr, int64_t N, float alpha,
                                                PA __restrict__ A, int64_t lda,
                                                PX __restrict__ x, float beta,
@@ -87,23 +87,36 @@ __device__ __forceinline__ void gemv_rows_wave(int64_t r0, int nr, int64_t N, fl
             for (int r = 0; r < ROWS; ++r) acc[r] = dot4(av[r][u], xv[u], acc[r]);
     }
     if constexpr (BATCH) {
-        if (j - lane < n4) {
-            float4 xv[UNROLL];
-            float4 av[ROWS][UNROLL];
+        auto last = [&](auto loads) {
+            constexpr int U = decltype(loads)::value;
+            float4 xv[U];
+            float4 av[ROWS][U];
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
+            for (int u = 0; u < U; ++u)
                 xv[u] = ld4u(at(x, std::min<Idx>(j + 64 * u, n4 - 1)));
 #pragma unroll
             for (int r = 0; r < ROWS; ++r)
 #pragma unroll
-                for (int u = 0; u < UNROLL; ++u)
-                    av[r][u] = ld4u(at(ar[r], std::min<Idx>(j + 64 * u, n4 - 1)));
+                for (int u = 0; u < U; ++u) {
+                    const auto p = at(ar[r], std::min<Idx>(j + 64 * u, n4 - 1));
+                    av[r][u] = STREAM && EXACT ? ld4u_nt(p) : ld4u(p);
+                }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
+            for (int u = 0; u < U; ++u)
 #pragma unroll
                 for (int r = 0; r < ROWS; ++r)
                     if (j + 64 * u < n4) acc[r] = dot4(av[r][u], xv[u], acc[r]);
+        };
+        const Idx left = n4 - (j - lane);
+        if constexpr (EXACT) {
+            static_assert(UNROLL <= 4, "a form for each number of loads");
+            if (left > 192) last(std::integral_constant<int, UNROLL>{});
+            else if (left > 128) last(std::integral_constant<int, std::min(UNROLL, 3)>{});
+            else if (left > 64) last(std::integral_constant<int, std::min(UNROLL, 2)>{});
+            else if (left > 0) last(std::integral_constant<int, 1>{});
+        } else if (left > 0) {
+            last(std::integral_constant<int, UNROLL>{});
         }
     } else {
         for (; j < n4; j += 64) {

@@ -565,15 +565,28 @@ __global__ __launch_bounds__(NT) void grouped_exps_kernel(const ExpItem* __restr
 __device__ __forceinline__ void gemv_item(const DGemv& v, int chunk) {
     const int tid = item_tid();
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // wavefront w takes rows chunk*64 + 16w .. +15 in one pass (16 rows of
-    // 128-bit loads in flight per lane); rows under 2^29 columns use scalar
-    // row bases and 32-bit lane offsets (GEMV-only C4 2.63 -> 2.61 ms)
+    // Wavefront w takes rows chunk*64 + 16w .. +15, as many at a time as keep 16
+    // loads per lane in flight (16 rows x 1 load, 8 x 2, 4 x 4) with no load past a
+    // short row, and with the non-temporal hint: bound by HBM, whose rate the hint
+    // raises from 6.3 to 6.8 TB/s for rows of 4096, if the loads of a row come
+    // together so that lines at their borders are read once.  4096 GEMVs of 64 to
+    // 4096: 2622 us as 16 x 1 without the hint, 2599 with it, 2460 so (6.3 TB/s).
     const int64_t r0 = (int64_t)chunk * 64 + wave * 16;
     if (r0 >= v.M) return;
     const int nr = (int)(v.M - r0 < 16 ? v.M - r0 : 16);
-    if (v.N < kGemvOff32Cols)
-        gemv_rows_wave<16, 1, false, true>(r0, nr, v.N, v.alpha, as_global(v.A), v.lda,
-                                           as_global(v.x), v.beta, as_global(v.y), lane);
+    auto rows = [&](auto rows_at_once, auto loads) {
+        constexpr int R = decltype(rows_at_once)::value, U = decltype(loads)::value;
+        for (int q = 0; q < nr; q += R)
+            gemv_rows_wave<R, U, true, true, true, true>(
+                r0 + q, std::min(nr - q, R), v.N, v.alpha, as_global(v.A), v.lda, as_global(v.x),
+                v.beta, as_global(v.y), lane);
+    };
+    typedef std::integral_constant<int, 1> I1;
+    typedef std::integral_constant<int, 2> I2;
+    typedef std::integral_constant<int, 4> I4;
+    if (v.N < 4 * 65) rows(std::integral_constant<int, 16>{}, I1{});
+    else if (v.N < 4 * 129) rows(std::integral_constant<int, 8>{}, I2{});
+    else if (v.N < kGemvOff32Cols) rows(I4{}, I4{});
     else
         gemv_rows_wave<16, 1, false>(r0, nr, v.N, v.alpha, as_global(v.A), v.lda, as_global(v.x), v.beta,
                                      as_global(v.y), lane);
