@@ -116,13 +116,18 @@ omb_status launch_sgemm_f32(int64_t M, int64_t N, int64_t K, float alpha,
                             float beta, float* C, int64_t ldc, hipStream_t s,
                             float* part = nullptr);
 
-// The split product of mode `f16` / `nprod` in one launch of 64 x 64 tiles, K shared
-// by `groups` (1, 2 or 4) groups of 256 threads; a_kc, b_kc: k is A's, B's unit
-// stride, lda, ldb the other one.  The bits are the packed path's (no or exact split).
+// A split product in one launch of 64 x 64 tiles, K shared by `groups` (1, 2 or 4)
+// groups of 256 threads; a_kc, b_kc: k is A's, B's unit stride, lda, ldb the other
+// one.  amax_a, amax_b: the lines' maxima for the scaled FP16 form, else null.  The
+// bits are the packed path's with no or an exact split of K.
+// sgemm_split_tile_groups: the number of groups with the least modelled time, or 0
+// where the packed path's is less (or it splits K in coarse blocks).
+int sgemm_split_tile_groups(int64_t M, int64_t N, int64_t K, int nprod, bool f16);
 omb_status launch_sgemm_split_tile(int groups, int64_t M, int64_t N, int64_t K, float alpha,
                                    const float* A, int64_t lda, bool a_kc, const float* B,
                                    int64_t ldb, bool b_kc, float beta, float* C, int64_t ldc,
-                                   int nprod, bool f16, hipStream_t s);
+                                   int nprod, const unsigned* amax_a, const unsigned* amax_b,
+                                   hipStream_t s);
 
 // Split-BF16 SGEMM (row-major C after layout folding); operands as strided
 // views: both are split into the packed form in the stream's workspace, then

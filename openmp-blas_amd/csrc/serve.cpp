@@ -149,6 +149,10 @@ omb_status launch_request(const omb_request& r, char* ws, hipStream_t s) {
                 return launch_sgemm_split16_ws(r.m, r.n, r.k, 1.f, r.a, r.k, 1, r.b, r.n, 1, 0.f,
                                                r.c, r.n, ws, s);
             const int planes = split_planes(r);
+            if (const int groups = sgemm_split_tile_groups(r.m, r.n, r.k, planes == 2 ? 3 : 6, false))
+                return launch_sgemm_split_tile(groups, r.m, r.n, r.k, 1.f, r.a, r.k, true, r.b, r.n,
+                                               false, 0.f, r.c, r.n, planes == 2 ? 3 : 6, nullptr,
+                                               nullptr, s);
             __bf16* ap = reinterpret_cast<__bf16*>(ws);
             __bf16* bp = ap + packed_elems(r, r.m);
             // A, and B^T of row-major B, in one launch

@@ -519,33 +519,18 @@ omb_status launch_split_pack_pair(int64_t M, int64_t N, int64_t K, const float* 
     return OMB_OK;
 }
 
-// Row maxima of A and B^T (amax_b follows amax_a), then both packed in their scaled
-// FP16 pieces.
-omb_status launch_split16_pack_pair(int64_t M, int64_t N, int64_t K, const float* A, int64_t rsA,
-                                    int64_t csA, __bf16* ap, unsigned* amax_a, int* ea,
-                                    const float* Bt, int64_t rsB, int64_t csB, __bf16* bp,
-                                    unsigned* amax_b, int* eb, hipStream_t s) {
-    if (K <= 0 || M <= 0 || N <= 0) return OMB_OK;
-    const int64_t nkt = ceil_div(K, TK), kgroups = ceil_div(nkt, SPLIT_SL);
-    const PackOperand a{A, M, rsA, csA, csA == 1 ? 1 : 0, ap, ceil_div(M, TM), amax_a, ea};
-    const PackOperand b{Bt, N, rsB, csB, csB == 1 ? 1 : 0, bp, ceil_div(N, TM), amax_b, eb};
-    const int64_t ga = ceil_div(M, (int64_t)kAmaxRows), gb = ceil_div(N, (int64_t)kAmaxRows);
-    if (ga + gb > 0x7fffffffLL || kgroups > 65535) {
-        set_error("split pack: operands too large for one launch");
-        return OMB_EUNSUPPORTED;
-    }
+// Row maxima of both operands (b's follow a's in memory).
+omb_status launch_amax_pair(const PackOperand& a, const PackOperand& b, int64_t K, hipStream_t s) {
+    const int64_t ga = ceil_div(a.R, (int64_t)kAmaxRows), gb = ceil_div(b.R, (int64_t)kAmaxRows);
     // k ranges of whole 128-byte lines when the row groups alone leave CUs idle
     const int64_t ranges = std::max<int64_t>(
         1, std::min<int64_t>(2 * device_cu_count() / (ga + gb), K / kAmaxRange));
     const int64_t range = round_up(ceil_div(K, ranges), kLineFloats);
     if (ranges > 1)
-        hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(M + N, NT), 1024)),
-                           dim3(NT), 0, s, amax_a, M + N);
+        hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(a.R + b.R, NT), 1024)),
+                           dim3(NT), 0, s, a.amax, a.R + b.R);
     hipLaunchKernelGGL(amax_pair_kernel, dim3((unsigned)(ga + gb), (unsigned)ceil_div(K, range)),
                        dim3(kAmaxThreads), 0, s, a, b, K, ga, range);
-    hipLaunchKernelGGL((split_pack_pair_kernel<true, 2>),
-                       dim3((unsigned)(a.rtiles + b.rtiles), (unsigned)kgroups), dim3(NT), 0, s, a, b,
-                       K, nkt);
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
@@ -606,6 +591,10 @@ omb_status launch_sgemm_split(int64_t M, int64_t N, int64_t K, float alpha,
                               const float* A, int64_t rsA, int64_t csA,
                               const float* B, int64_t rsB, int64_t csB,
                               float beta, float* C, int64_t ldc, int nprod, hipStream_t s) {
+    if (const int groups = sgemm_split_tile_groups(M, N, K, nprod, false))
+        return launch_sgemm_split_tile(groups, M, N, K, alpha, A, csA == 1 ? rsA : csA, csA == 1, B,
+                                       rsB == 1 ? csB : rsB, rsB == 1, beta, C, ldc, nprod, nullptr,
+                                       nullptr, s);
     // the 3-product form packs only the two planes it reads
     const int planes = nprod == 3 ? 2 : 3;
     const size_t a_elems = (size_t)(planes == 2 ? split16_packed_elems(M, K)
@@ -663,8 +652,23 @@ omb_status launch_sgemm_split16_ws(int64_t M, int64_t N, int64_t K, float alpha,
     float* part =
         splits > 1 ? reinterpret_cast<float*>(ws + packed + split16_extra_bytes(M, N)) : nullptr;
     // A scaled by rows, B^T (rows n) by rows, i.e. B by columns.
-    OMB_TRY(launch_split16_pack_pair(M, N, K, A, rsA, csA, ap, amax_a, ea, B, csB, rsB, bp, amax_b, eb,
-                                     s));
+    const int64_t kgroups = ceil_div(ceil_div(K, TK), SPLIT_SL);
+    const PackOperand oa{A, M, rsA, csA, csA == 1 ? 1 : 0, ap, ceil_div(M, TM), amax_a, ea};
+    const PackOperand ob{B, N, csB, rsB, rsB == 1 ? 1 : 0, bp, ceil_div(N, TM), amax_b, eb};
+    if (ceil_div(M, (int64_t)kAmaxRows) + ceil_div(N, (int64_t)kAmaxRows) > 0x7fffffffLL ||
+        kgroups > 65535) {
+        set_error("split pack: operands too large for one launch");
+        return OMB_EUNSUPPORTED;
+    }
+    OMB_TRY(launch_amax_pair(oa, ob, K, s));
+    if (const int groups = sgemm_split_tile_groups(M, N, K, 3, true))
+        return launch_sgemm_split_tile(groups, M, N, K, alpha, A, csA == 1 ? rsA : csA, csA == 1, B,
+                                       rsB == 1 ? csB : rsB, rsB == 1, beta, C, ldc, 3, amax_a, amax_b,
+                                       s);
+    hipLaunchKernelGGL((split_pack_pair_kernel<true, 2>),
+                       dim3((unsigned)(oa.rtiles + ob.rtiles), (unsigned)kgroups), dim3(NT), 0, s, oa,
+                       ob, K, ceil_div(K, TK));
+    OMB_HIP_TRY(hipGetLastError());
     return launch_sgemm_packed(M, N, K, alpha, ap, bp, beta, C, ldc, 3, s, part, ea, eb, 2);
 }
 
