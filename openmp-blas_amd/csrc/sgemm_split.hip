@@ -99,48 +99,67 @@ __device__ __forceinline__ void pack_tile(const float* __restrict__ X, int64_t R
     if (F16 && kg == 0 && tid < TM && r0 + tid < R)
         exps[r0 + tid] = row_exp<true>(amax, r0 + tid, R);
     // 128-bit loads (any alignment) need a unit stride along the loaded
-    // index; other strides take the element path.  The values are the same.
-    const bool vec = k_major ? cs == 1 : rs == 1;
+    // index; other strides take the element path, as do the last k of a
+    // partial group and, along rows, a partial tile.  The values are the same.
+    const bool vec = (k_major ? cs == 1 : rs == 1) && k0 + SPLIT_SL * TK <= K;
     if (k_major) {
-        // 128 rows x (4 * SPLIT_SL) float4 along k: thread -> (row, k4)
+        // 128 rows x (4 * SPLIT_SL) float4 along k: thread -> (row, k4); every
+        // load is issued before the first is converted, rows past the last
+        // repeat it and are zeroed.  Rows that do not start on lines share
+        // them with the next group, so they are loaded without the hint.
+        const bool lines = rs % kLineFloats == 0;
+        constexpr int Q = 2 * SPLIT_SL;
+        float4 t[Q];
+        int e[Q];
+        auto place = [&](int j, int* kk4) {
+            const int f = tid + NT * j;
+            *kk4 = (f % (4 * SPLIT_SL)) * 4;
+            return f / (4 * SPLIT_SL);
+        };
 #pragma unroll
-        for (int j = 0; j < 2 * SPLIT_SL; ++j) {
-            const int f = tid + NT * j, row = f / (4 * SPLIT_SL), kk4 = (f % (4 * SPLIT_SL)) * 4;
-            const int64_t r = r0 + row, k = k0 + kk4;
-            float v[4];
-            if (vec && r < R && k + 3 < K) {
-                const float4 t = ld4u_nt(X + r * rs + k);
-                v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+        for (int j = 0; j < Q; ++j) {
+            int kk4;
+            const int64_t r = r0 + place(j, &kk4), rc = std::min(r, R - 1), k = k0 + kk4;
+            e[j] = F16 ? (int)amax[rc] : 0;
+            if (vec) {
+                t[j] = lines ? ld4u_nt(X + rc * rs + k) : ld4u(X + rc * rs + k);
             } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = ld(X, R, K, rs, cs, r, k + e);
+                t[j] = make_float4(ld(X, R, K, rs, cs, rc, k), ld(X, R, K, rs, cs, rc, k + 1),
+                                   ld(X, R, K, rs, cs, rc, k + 2), ld(X, R, K, rs, cs, rc, k + 3));
             }
-            put4<F16, PLN>(lds, row, kk4, v, row_exp<F16>(amax, r, R));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < Q; ++j) {
+            int kk4;
+            const int row = place(j, &kk4);
+            const bool in = r0 + row < R;
+            const float v[4] = {in ? t[j].x : 0.f, in ? t[j].y : 0.f, in ? t[j].z : 0.f,
+                                in ? t[j].w : 0.f};
+            put4<F16, PLN>(lds, row, kk4, v, F16 ? line_exp(__uint_as_float((unsigned)e[j])) : 0);
         }
     } else {
         // (16 * SPLIT_SL) k-columns x 32 float4 along rows: thread -> (4 columns, 4 rows)
-        static_assert(SPLIT_SL * 128 % NT == 0, "whole passes of the workgroup");
+        static_assert(SPLIT_SL * 128 == NT, "one pass of the workgroup");
+        const int kq = tid >> 5, row4 = (tid & 31) * 4;
+        const int64_t r = r0 + row4;
+        float m[4][4];  // [k][row]
+        if (vec && r0 + TM <= R) {
+            float4 t[4];
 #pragma unroll
-        for (int j = 0; j < SPLIT_SL * 128 / NT; ++j) {
-            const int f = tid + NT * j, kq = f >> 5, row4 = (f & 31) * 4;
-            const int64_t r = r0 + row4;
-            float m[4][4];  // [k][row]
+            for (int c = 0; c < 4; ++c) t[c] = ld4u_nt(X + (k0 + kq * 4 + c) * cs + r);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int64_t k = k0 + kq * 4 + c;
-                if (vec && k < K && r + 3 < R) {
-                    const float4 t = ld4u_nt(X + k * cs + r);
-                    m[c][0] = t.x; m[c][1] = t.y; m[c][2] = t.z; m[c][3] = t.w;
-                } else {
+            for (int c = 0; c < 4; ++c) m[c][0] = t[c].x, m[c][1] = t[c].y, m[c][2] = t[c].z, m[c][3] = t[c].w;
+        } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) m[c][e] = ld(X, R, K, rs, cs, r + e, k);
-                }
-            }
+            for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float v[4] = {m[0][e], m[1][e], m[2][e], m[3][e]};
-                put4<F16, PLN>(lds, row4 + e, kq * 4, v, row_exp<F16>(amax, r + e, R));
-            }
+                for (int e = 0; e < 4; ++e) m[c][e] = ld(X, R, K, rs, cs, r + e, k0 + kq * 4 + c);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v[4] = {m[0][e], m[1][e], m[2][e], m[3][e]};
+            put4<F16, PLN>(lds, row4 + e, kq * 4, v, row_exp<F16>(amax, r + e, R));
         }
     }
     __syncthreads();
@@ -165,8 +184,12 @@ __global__ __launch_bounds__(NT) void split_pack_kernel(const float* __restrict_
 }
 
 // Both operands of one product in one launch (same K): row tiles of the
-// first, then of the second, along blockIdx.x.  amax, exps: the row maxima's bits
-// and where the exponents go (scaled FP16 split only).
+// first, then of the second.  The workgroups of one XCD take neighbouring pieces
+// of the unit stride, which share lines where rows do not start on them.  Bound by
+// HBM; with the k groups along blockIdx.y and each load converted as it came, scaled
+// FP16 of 2500 x 3001 x 1777 (both operands k-contiguous) took 119 us, 111 so, split
+// BF16 162 and 152; 4001 x 500 x 6001 164 and 145, 192 and 181; whole lines the same.
+// amax, exps: the row maxima's bits and where the exponents go (scaled FP16 split only).
 struct PackOperand {
     const float* X;
     int64_t R, rs, cs;
@@ -179,11 +202,15 @@ struct PackOperand {
 template <bool F16, int PLN>
 __global__ __launch_bounds__(NT) void split_pack_pair_kernel(PackOperand a, PackOperand b,
                                                              int64_t K, int64_t nkt) {
-    const bool first = (int64_t)blockIdx.x < a.rtiles;
+    const unsigned groups = (unsigned)((nkt + SPLIT_SL - 1) / SPLIT_SL);
+    unsigned t = xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned ta = (unsigned)a.rtiles * groups;
+    const bool first = t < ta;
     const PackOperand& o = first ? a : b;
-    const int64_t rt = first ? (int64_t)blockIdx.x : (int64_t)blockIdx.x - a.rtiles;
-    pack_tile<F16, PLN>(o.X, o.R, K, o.rs, o.cs, nkt, o.k_major, o.out, o.amax, o.exps, rt,
-                        blockIdx.y);
+    if (!first) t -= ta;
+    const unsigned inner = o.k_major ? groups : (unsigned)o.rtiles, q = t / inner, r = t - q * inner;
+    const int64_t rt = o.k_major ? q : r, kg = o.k_major ? r : q;
+    pack_tile<F16, PLN>(o.X, o.R, K, o.rs, o.cs, nkt, o.k_major, o.out, o.amax, o.exps, rt, kg);
 }
 
 // ----------------------------------------------------------------- pass 2 --
@@ -506,11 +533,11 @@ omb_status launch_split_pack_pair(int64_t M, int64_t N, int64_t K, const float* 
                         nullptr, nullptr};
     const PackOperand b{Bt, N, rsB, csB, csB == 1 ? 1 : 0, bp, N > 0 ? ceil_div(N, TM) : 0,
                         nullptr, nullptr};
-    if (a.rtiles + b.rtiles > 0x7fffffffLL || kgroups > 65535) {
+    if ((a.rtiles + b.rtiles) * kgroups > 0x7fffffffLL || kgroups > 65535) {
         set_error("split pack: operands too large for one launch");
         return OMB_EUNSUPPORTED;
     }
-    const dim3 grid((unsigned)(a.rtiles + b.rtiles), (unsigned)kgroups);
+    const dim3 grid((unsigned)((a.rtiles + b.rtiles) * kgroups));
     if (planes == 2)
         hipLaunchKernelGGL((split_pack_pair_kernel<false, 2>), grid, dim3(NT), 0, s, a, b, K, nkt);
     else
@@ -656,7 +683,7 @@ omb_status launch_sgemm_split16_ws(int64_t M, int64_t N, int64_t K, float alpha,
     const PackOperand oa{A, M, rsA, csA, csA == 1 ? 1 : 0, ap, ceil_div(M, TM), amax_a, ea};
     const PackOperand ob{B, N, csB, rsB, rsB == 1 ? 1 : 0, bp, ceil_div(N, TM), amax_b, eb};
     if (ceil_div(M, (int64_t)kAmaxRows) + ceil_div(N, (int64_t)kAmaxRows) > 0x7fffffffLL ||
-        kgroups > 65535) {
+        kgroups > 65535 || (oa.rtiles + ob.rtiles) * kgroups > 0x7fffffffLL) {
         set_error("split pack: operands too large for one launch");
         return OMB_EUNSUPPORTED;
     }
@@ -666,7 +693,7 @@ omb_status launch_sgemm_split16_ws(int64_t M, int64_t N, int64_t K, float alpha,
                                        rsB == 1 ? csB : rsB, rsB == 1, beta, C, ldc, 3, amax_a, amax_b,
                                        s);
     hipLaunchKernelGGL((split_pack_pair_kernel<true, 2>),
-                       dim3((unsigned)(oa.rtiles + ob.rtiles), (unsigned)kgroups), dim3(NT), 0, s, oa,
+dim3((unsigned)((oa.rtiles + ob.rtiles) * kgroups)), dim3(NT), 0, s, oa,
                        ob, K, ceil_div(K, TK));
     OMB_HIP_TRY(hipGetLastError());
     return launch_sgemm_packed(M, N, K, alpha, ap, bp, beta, C, ldc, 3, s, part, ea, eb, 2);
