@@ -183,16 +183,17 @@ struct Slot {
     bool busy() const { return req >= 0 || !batch.empty(); }
 };
 
-// Requests small enough to share a grouped launch: at most 1e8 FLOP per
-// GEMM and 4 MiB of A per GEMV (launch-bound on their own), at most 32 per
-// launch.  Measured on the C5 trace (3000 requests, split-BF16): larger
-// limits (3e8-4e9 FLOP, 8-32 MiB, 512 per launch) put mid-size GEMMs on
-// the grouped 64x64 tiles, which are slower than their direct kernels, and
-// made p99 worse at 48k-64k requests/s.  A GEMM joins only if its direct
-// call keeps the unsplit fold (no K split, or one 128-k / 256-k
-// accumulation block per split), since a grouped tile never splits K.
-constexpr double kBatchGemmFlop = 1e8;
-constexpr double kBatchGemvBytes = 4.0 * (1 << 20);
+// Requests small enough to share a grouped launch: at most 1e9 FLOP per GEMM and
+// 16 MiB of A per GEMV, at most 32 per launch.  Up to there a GEMM's direct kernel
+// works on tiles like the grouped one, and a launch of its own on a shared chip
+// waits 30 to 90 us in its queue.  A burst of 192 requests (split BF16): 1e8 and 4 MiB
+// 1724 to 1790 us, 1e9 and 4 MiB 1573 to 1593, these 1512 to 1524; 64 per launch the
+// same.  3000 requests at once 31.5 ms -> 28.1 (plain 40.8 -> 38.1); at 32,000 and
+// 64,000 per second p99 0.26 to 0.29 and 0.40 to 0.44 ms with either.  A GEMM
+// joins only if its direct call keeps the unsplit fold (no K split, or one 128-k /
+// 256-k accumulation block per split), since a grouped tile never splits K.
+constexpr double kBatchGemmFlop = 1e9;
+constexpr double kBatchGemvBytes = 16.0 * (1 << 20);
 constexpr int kBatchMax = 32;
 constexpr int64_t kBatchMaxItems = 65536;  // the descriptor block's item capacity
 
