@@ -93,6 +93,8 @@ constexpr int kLineFloats = 32;  // floats per 128-byte line
 int64_t gemm_k_splits(int64_t M, int64_t N, int64_t K, int64_t align, double rate_full,
                       double rate_alone, int64_t* kchunk);
 int64_t sgemm_f32_splits(int64_t M, int64_t N, int64_t K, int64_t* kchunk);
+// The K split of the tile classes alone: at least what any choice needs in partials.
+int64_t sgemm_f32_tile_splits(int64_t M, int64_t N, int64_t K);
 // The class of the kernel that divides K among a workgroup's wavefronts whose
 // modelled time is least and below *time (seconds), which it replaces, or -1.
 // Its sums are those of the unsplit tiles, bit for bit, with no partials in memory.

@@ -546,6 +546,13 @@ int64_t sgemm_f32_splits(int64_t M, int64_t N, int64_t K, int64_t* kchunk) {
     return splits;
 }
 
+int64_t sgemm_f32_tile_splits(int64_t M, int64_t N, int64_t K) {
+    int64_t splits = 1, kchunk = K;
+    double t = 0.0;
+    choose_tiles(M, N, K, &splits, &kchunk, &t);
+    return splits;
+}
+
 omb_status launch_splitk_reduce(int64_t M, int64_t N, int64_t splits, float alpha, float beta,
                                 const float* part, float* C, int64_t ldc, hipStream_t s) {
     if (M <= 0 || N <= 0) return OMB_OK;
