@@ -194,6 +194,7 @@ struct Slot {
 // joins only if its direct call keeps the unsplit fold (no K split, or one 128-k /
 // 256-k accumulation block per split), since a grouped tile never splits K.
 constexpr double kBatchGemmFlop = 1e9;
+constexpr double kBatchUnfitFlop = 1e8;  // the most of a GEMM whose own workspace never fits
 constexpr double kBatchGemvBytes = 16.0 * (1 << 20);
 constexpr int kBatchMax = 32;
 constexpr int64_t kBatchMaxItems = 65536;  // the descriptor block's item capacity
@@ -427,6 +428,8 @@ class Engine {
             const omb_request& q = st.req(r);
             if (!batchable(q)) continue;
             if (q.kind == OMB_REQ_GEMM) {
+                // (a larger one is refused in its turn, as without a backlog)
+                if ((size_t)q.ws_bytes > arena_.capacity() && flop_of(q) > kBatchUnfitFlop) continue;
                 if (bmode < 0) bmode = q.mode;
                 if (q.mode != bmode) continue;
             }
