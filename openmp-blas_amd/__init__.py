@@ -241,7 +241,8 @@ def is_matrix(t) -> bool:
 
 
 def is_vector(t) -> bool:
-    return t.dim() == 1 or (t.dim() == 2 and (t.shape[0] == 1 or t.shape[1] == 1))
+    shape = t.shape
+    return len(shape) == 1 or (len(shape) == 2 and (shape[0] == 1 or shape[1] == 1))
 
 
 def mtm(c, a, b, num_threads=None, mode: int = PLAIN_F32, stream=None):
@@ -249,46 +250,49 @@ def mtm(c, a, b, num_threads=None, mode: int = PLAIN_F32, stream=None):
 
     ``num_threads`` is accepted for signature parity and ignored (the GPU
     decides its own parallelism)."""
-    if not (is_matrix(a) and is_matrix(b) and is_matrix(c)):
+    sa, sb, sc = a.shape, b.shape, c.shape
+    if len(sa) != 2 or len(sb) != 2 or len(sc) != 2:
         raise RuntimeError("amt::mtm: a, b, and c must be the matrices")
-    if not (a.shape[0] == c.shape[0] and a.shape[1] == b.shape[0] and c.shape[1] == b.shape[1]):
+    (M, K), N = sa, sb[1]
+    if sc[0] != M or sb[0] != K or sc[1] != N:
         raise RuntimeError("amt::mtm: dimension mismatch")
-    M, K = a.shape
-    N = b.shape[1]
-    (rsa, csa), (rsb, csb), (rsc, csc) = _strides(a), _strides(b), _strides(c)
+    (rsa, csa), (rsb, csb), (rsc, csc) = a.stride(), b.stride(), c.stride()
 
     def run():
-        check(sgemm(M, N, K, 1.0, _ptr(a), rsa, csa, _ptr(b), rsb, csb, 1.0, _ptr(c), rsc, csc,
-                    mode, stream))
+        _done(lib().omb_sgemm(M, N, K, 1.0, a.data_ptr(), rsa, csa, b.data_ptr(), rsb, csb, 1.0,
+                              c.data_ptr(), rsc, csc, mode, _stream(stream)))
 
     return run
 
 
-def _vec_len(t) -> int:
-    return t.numel()
+def _done(status: int) -> None:
+    """check() of a closure's call, without a call of its own where it succeeded."""
+    if status:
+        check(status)
 
 
-def _is_first_order(a) -> bool:
+def _first_order(rs: int, cs: int, cols: int) -> bool:
     """Column-major (uBLAS first_order) when the row stride is 1."""
-    rs, cs = _strides(a)
     if cs == 1 and rs == 1:
-        return a.shape[1] <= 1
+        return cols <= 1
     return rs == 1
 
 
 def mtv(c, a, b, num_threads=None, stream=None):
     """amt::mtv (include/mtv.hpp:100-162): c += A*b for column-major A
     (first_order helper, :15-70), c = A*b for row-major A (last_order, :72-98)."""
-    if not (is_matrix(a) and is_vector(b) and is_vector(c)):
+    shape = a.shape
+    if not (len(shape) == 2 and is_vector(b) and is_vector(c)):
         raise RuntimeError("amt::mtv: c and b must be vector, and a must be a matrix")
-    if a.shape[1] != _vec_len(b) or a.shape[0] != _vec_len(c):
+    M, N = shape
+    if N != b.numel() or M != c.numel():
         raise RuntimeError("amt::mtv: dimension mismatch")
-    M, N = a.shape
-    rs, cs = _strides(a)
-    beta = 1.0 if _is_first_order(a) else 0.0
+    rs, cs = a.stride()
+    beta = 1.0 if _first_order(rs, cs, N) else 0.0
 
     def run():
-        check(sgemv(M, N, 1.0, _ptr(a), rs, cs, _ptr(b), beta, _ptr(c), stream))
+        _done(lib().omb_sgemv(M, N, 1.0, a.data_ptr(), rs, cs, b.data_ptr(), beta, c.data_ptr(),
+                              _stream(stream)))
 
     return run
 
@@ -297,17 +301,19 @@ def vtm(c, a, b, num_threads=None, stream=None):
     """amt::vtm (include/mtv.hpp:164-236): c = A^T b.  The reference runs the
     helper of the other layout, so a column-major A overwrites c and a
     row-major A accumulates into c; the product itself is the true A^T b."""
-    if not (is_matrix(a) and is_vector(b) and is_vector(c)):
+    shape = a.shape
+    if not (len(shape) == 2 and is_vector(b) and is_vector(c)):
         raise RuntimeError("amt::vtm: c and b must be vector, and a must be a matrix")
-    if a.shape[1] != _vec_len(c) or a.shape[0] != _vec_len(b):
+    M, N = shape
+    if N != c.numel() or M != b.numel():
         raise RuntimeError("amt::vtm: dimension mismatch")
-    M, N = a.shape
-    rs, cs = _strides(a)
-    beta = 0.0 if _is_first_order(a) else 1.0
+    rs, cs = a.stride()
+    beta = 0.0 if _first_order(rs, cs, N) else 1.0
 
     def run():
         # A^T is N x M with strides (cs, rs).
-        check(sgemv(N, M, 1.0, _ptr(a), cs, rs, _ptr(b), beta, _ptr(c), stream))
+        _done(lib().omb_sgemv(N, M, 1.0, a.data_ptr(), cs, rs, b.data_ptr(), beta, c.data_ptr(),
+                              _stream(stream)))
 
     return run
 
@@ -316,12 +322,12 @@ def dot_prod(c, a, b, num_threads=None, stream=None):
     """amt::dot_prod (include/dot.hpp:176-224): c[0] = sum a*b (overwrite)."""
     if not (is_vector(a) and is_vector(b)):
         raise RuntimeError("amt::dot_prod: both tensor must be vector")
-    if _vec_len(a) != _vec_len(b):
+    n = a.numel()
+    if n != b.numel():
         raise RuntimeError("amt::dot_prod: both vector must be of same size")
-    n = _vec_len(a)
 
     def run():
-        check(sdot(n, _ptr(a), _ptr(b), _ptr(c), stream))
+        _done(lib().omb_sdot(n, a.data_ptr(), b.data_ptr(), c.data_ptr(), _stream(stream)))
 
     return run
 
@@ -338,13 +344,14 @@ def outer_prod(c, a, b, num_threads=None, stream=None):
     (length M) and b (length N) and an M x N matrix C of either layout."""
     if not (is_vector(a) and is_vector(b)):
         raise RuntimeError("amt::outer_prod: both tensor must be vector")
-    M, N = _vec_len(a), _vec_len(b)
-    if not is_matrix(c) or c.shape[0] != M or c.shape[1] != N:
+    M, N = a.numel(), b.numel()
+    if c.shape != (M, N):
         raise RuntimeError("amt::outer_prod: dimension mismatch")
-    rs, cs = _strides(c)
+    rs, cs = c.stride()
 
     def run():
-        check(sger(M, N, 1.0, _ptr(a), _ptr(b), _ptr(c), rs, cs, stream))
+        _done(lib().omb_sger(M, N, 1.0, a.data_ptr(), b.data_ptr(), c.data_ptr(), rs, cs,
+                             _stream(stream)))
 
     return run
 
@@ -368,15 +375,17 @@ def transpose(c, a=None, num_threads=None, stream=None):
             check(stranspose_inplace(n, _ptr(a), ld, stream))
 
         return run_inplace
-    if not (is_matrix(a) and is_matrix(c)):
+    sa, sc = a.shape, c.shape
+    if len(sa) != 2 or len(sc) != 2:
         raise RuntimeError("amt::transpose: a and c must be the matrices")
-    if a.shape[0] != c.shape[1] or a.shape[1] != c.shape[0]:
+    M, N = sa
+    if sc[0] != N or sc[1] != M:
         raise RuntimeError("amt::transpose: dimension mismatch")
-    M, N = a.shape
-    (rsA, csA), (rsC, csC) = _strides(a), _strides(c)
+    (rsA, csA), (rsC, csC) = a.stride(), c.stride()
 
     def run():
-        check(stranspose(M, N, _ptr(a), rsA, csA, _ptr(c), rsC, csC, stream))
+        _done(lib().omb_stranspose(M, N, a.data_ptr(), rsA, csA, c.data_ptr(), rsC, csC,
+                                   _stream(stream)))
 
     return run
 
