@@ -424,7 +424,7 @@ def main():
                                         "frac_of_hbm_peak": nbytes / t_i / PEAK_HBM,
                                         "bytes": nbytes}
         kernels["ger_kernel (16384^2, row-major C)"] = level2["sger_row"]
-        kernels["transpose_tiles_kernel (16384^2)"] = level2["transpose_out_of_place"]
+        kernels["transpose_lines_kernel (16384^2)"] = level2["transpose_out_of_place"]
         kernels["transpose_inplace_kernel (16384^2)"] = level2["transpose_in_place"]
         del LA, LC
         sync()
