@@ -30,12 +30,12 @@
 //
 // Row-major C only: a column-major C is handled by the caller through
 // C^T = B^T A^T (swap operands and their strides).
-#include "common.hpp"
+#include "slice_bounds.hpp"
 
 namespace omb {
 namespace {
 
-constexpr int BK = 16;
+constexpr int BK = kSliceK;
 constexpr int NT = 256;         // threads per workgroup (a 16 x 16 thread grid)
 constexpr int INNER_K = 128;    // k steps per inner accumulation block
 constexpr int PAD = 4;          // LDS row padding (floats), keeps float4 alignment
@@ -100,17 +100,9 @@ struct Side {
         p = X + (KC ? e0 * ld + kbeg : e0 + kbeg * ld);
         n = (int)std::min<int64_t>(lines - e0, E);
 #pragma unroll
-        for (int i = 0; i < L; ++i) {
-            const int e = tid + i * NT;
-            off[i] = (Off)(4 * (KC ? min(e >> 2, n - 1) * ld + (e & 3) * 4
-                                   : (e / (E / 4)) * ld + min(e % (E / 4) * 4, (n - 1) & ~3)));
-        }
+        for (int i = 0; i < L; ++i) off[i] = (Off)(4 * slice_load<E, KC>(tid + i * NT, n, ld));
     }
-    // k steps at the operand's end that a 4-line load could read past: the
-    // last one, or the last three when lines are less than 4 floats apart.
-    __device__ __forceinline__ int tail() const {
-        return KC || n % 4 == 0 ? 0 : (ld < 4 ? 3 : 1);
-    }
+    __device__ __forceinline__ int tail() const { return slice_tail<KC>(n, ld); }
     __device__ __forceinline__ void load(float4 (&v)[L], int64_t k0) const {
         const char* q = reinterpret_cast<const char*>(p + (KC ? k0 : k0 * ld));
 #pragma unroll
@@ -235,8 +227,7 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
     Side<BN, !B_NC, Off> sb;
     sa.init(p.A, p.lda, m0, p.M, kbeg, tid);
     sb.init(p.B, p.ldb, n0, p.N, kbeg, tid);
-    const int tail = kbeg + p.K == q.K ? max(sa.tail(), sb.tail()) : 0;
-    const int64_t nfull = p.K > tail ? (p.K - tail) / BK : 0;
+    const int64_t nfull = full_slices(kbeg, kbeg + p.K, q.K, max(sa.tail(), sb.tail()));
     int64_t kt = 0;
     if (nfull > 0) {
         // Slices kt and kt+1 in LDS buffers 0 and 1, loads two slices ahead in

@@ -5,12 +5,12 @@
 
 #include <algorithm>
 
-#include "common.hpp"
+#include "slice_bounds.hpp"
 
 namespace omb {
 namespace wave {
 
-constexpr int BK = 16;
+constexpr int BK = kSliceK;
 constexpr int BLOCK_K = 128;  // k per accumulation block, as sgemm_f32.hip
 constexpr int PAD = 4;
 
@@ -54,20 +54,14 @@ struct WaveSide {
     }
     // byte offset of load i: line (KC) or quad of lines, clamped into the operand
     __device__ __forceinline__ Off offset(int i) const {
-        const int e = lane + 64 * i;
-        return (Off)(4 * (KC ? min(e >> 2, n - 1) * ld + (e & 3) * 4
-                             : (e / (E / 4)) * ld + min(e % (E / 4) * 4, (n - 1) & ~3)));
+        return (Off)(4 * slice_load<E, KC>(lane + 64 * i, n, ld));
     }
     __device__ __forceinline__ void load(float4 (&v)[L], const Off (&off)[L], int64_t k0) const {
         const P q = p + (KC ? k0 : k0 * ld);
 #pragma unroll
         for (int i = 0; i < L; ++i) v[i] = ld4u(at_bytes(q, off[i]));
     }
-    // k steps at the operand's end that a 4-line load could read past: the
-    // last one, or the last three when lines are less than 4 floats apart.
-    __device__ __forceinline__ int tail() const {
-        return KC || n % 4 == 0 ? 0 : (ld < 4 ? 3 : 1);
-    }
+    __device__ __forceinline__ int tail() const { return slice_tail<KC>(n, ld); }
     // k0 .. k1-1 are the valid k of the slice (k1 <= K)
     __device__ __forceinline__ void load_guarded(float4 (&v)[L], int64_t k0, int64_t k1) const {
 #pragma unroll
