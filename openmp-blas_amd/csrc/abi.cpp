@@ -63,6 +63,17 @@ omb_status get_workspace(hipStream_t stream, size_t bytes, Workspace** out) {
     return OMB_OK;
 }
 
+unsigned* eager_arrivals(hipStream_t stream, const Workspace& ws) {
+    if (!ws.arrivals || stream == hipStreamPerThread) return nullptr;
+    if (!stream) return ws.arrivals;  // the null stream cannot be captured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return status == hipStreamCaptureStatusNone ? ws.arrivals : nullptr;
+}
+
 int device_cu_count() {
     static std::mutex mu;
     static std::map<int, int> cache;

@@ -35,8 +35,10 @@ __host__ __device__ inline int64_t round_up(int64_t a, int64_t b) { return ceil_
 
 // --------------------------------------------------------------- workspace --
 // Per-stream scratch memory: one grow-only device buffer, and the stream's
-// own arrival counters (zero between launches; null for streams past the
-// first kArrivalSlots, whose calls add their partials in a second launch).
+// own arrival counters (null for streams past the first kArrivalSlots).  A
+// launch that uses counters needs them zero and leaves them zero, so two that
+// overlap could leave them wrong for every later one; launches take them from
+// eager_arrivals, which keeps them to one stream's calls in order.
 struct Workspace {
     void* buf = nullptr;
     size_t bytes = 0;
@@ -47,6 +49,11 @@ constexpr int kArrivalCounters = 256;  // per stream
 constexpr int kArrivalStride = 16;     // counters lie 64 bytes apart
 // Counters of workspace `slot` on the current device, or null.
 unsigned* arrival_counters(int slot);
+// The workspace's counters for a launch on its stream, or null, upon which the
+// partials are added by a second launch (in the same order): while the stream
+// is captured, since the graph may be replayed on another stream beside this
+// one's calls, and for hipStreamPerThread, one handle for many streams.
+unsigned* eager_arrivals(hipStream_t stream, const Workspace& ws);
 
 // Compute units of the current device (cached per device).
 int device_cu_count();

@@ -216,7 +216,7 @@ omb_status launch_sdot(int64_t n, const float* x, const float* y, float* result,
     Workspace* ws = nullptr;
     OMB_TRY(get_workspace(s, n > 0 ? (size_t)sdot_blocks(n) * sizeof(double) : 0, &ws));
     return launch_sdot_ws(n, x, y, result, reinterpret_cast<double*>(ws->buf), s,
-                          ws->arrivals);
+                          n <= kArrivalMost ? eager_arrivals(s, *ws) : nullptr);
 }
 
 unsigned* arrival_counters(int slot) {

@@ -285,7 +285,7 @@ omb_status launch_col(int64_t M, int64_t N, float alpha, const float* A, int64_t
     Workspace* ws = nullptr;
     OMB_TRY(get_workspace(s, nchunks > 1 ? (size_t)(nchunks * mpad) * sizeof(float) : 0, &ws));
     float* part = reinterpret_cast<float*>(ws->buf);
-    unsigned* count = nrb <= kArrivalCounters ? ws->arrivals : nullptr;
+    unsigned* count = nchunks > 1 && nrb <= kArrivalCounters ? eager_arrivals(s, *ws) : nullptr;
     hipLaunchKernelGGL((sgemv_col_kernel<LR, U, STREAM, TINY>), dim3((unsigned)(nrb * nchunks)),
                        dim3(NT), 0, s, M, N, alpha, A, lda, x, beta, y, part, mpad, (int)nrb,
                        (int)nchunks, cpc, count);
