@@ -99,17 +99,18 @@ constexpr int kLineFloats = 32;  // floats per 128-byte line
 // the stream's workspace; launch_splitk_reduce adds them in split order.
 int64_t gemm_k_splits(int64_t M, int64_t N, int64_t K, int64_t align, double rate_full,
                       double rate_alone, int64_t* kchunk);
+// The K split that a plain product's sums follow, whichever kernel takes it: at
+// least what that kernel needs in partials.
 int64_t sgemm_f32_splits(int64_t M, int64_t N, int64_t K, int64_t* kchunk);
-// The K split of the tile classes alone: at least what any choice needs in partials.
-int64_t sgemm_f32_tile_splits(int64_t M, int64_t N, int64_t K);
 // The class of the kernel that divides K among a workgroup's wavefronts whose
 // modelled time is least and below *time (seconds), which it replaces, or -1.
-// Its sums are those of the unsplit tiles, bit for bit, with no partials in memory.
+// Its sums are those of the tile classes with K split by kchunk, bit for bit,
+// with no partials in memory.
 int sgemm_f32_wave_class(int64_t M, int64_t N, int64_t K, double* time);
 omb_status launch_sgemm_f32_wave(int cls, int64_t M, int64_t N, int64_t K, float alpha,
                                  const float* A, int64_t lda, bool a_kc, const float* B,
                                  int64_t ldb, bool b_nc, float beta, float* C, int64_t ldc,
-                                 hipStream_t s);
+                                 int64_t kchunk, hipStream_t s);
 // Whether a tile's loads of an operand lie within 2^32 bytes of a 16-k slice's
 // first element: up to `lines` lines of ld floats when k is the unit stride,
 // else the slice's 16 k.

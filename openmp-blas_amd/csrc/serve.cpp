@@ -90,14 +90,14 @@ size_t need_bytes(const omb_request& r) {
     switch (r.kind) {
         case OMB_REQ_GEMM: {
             if (r.m == 0 || r.n == 0 || r.k == 0) return 0;
+            int64_t kc = 0;
             // partial sums when K is split; what omb_serve_request_bytes answers
             // does not depend on which kernel of one launch takes the product
             if (r.mode == OMB_MODE_PLAIN_F32) {
-                const int64_t splits = sgemm_f32_tile_splits(r.m, r.n, r.k);
+                const int64_t splits = sgemm_f32_splits(r.m, r.n, r.k, &kc);
                 return splits > 1 ? (size_t)(splits * r.m * r.n) * sizeof(float) : 0;
             }
             if (r.mode == OMB_MODE_SPLIT_FP16) return split16_ws_bytes(r.m, r.n, r.k);
-            int64_t kc = 0;
             const int64_t splits = sgemm_split_splits(r.m, r.n, r.k, &kc);
             return packed_bytes(r) +
                    (splits > 1 ? (size_t)(splits * r.m * r.n) * sizeof(float) : 0);

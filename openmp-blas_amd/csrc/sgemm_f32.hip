@@ -516,8 +516,8 @@ int choose_tiles(int64_t M, int64_t N, int64_t K, int64_t* splits, int64_t* kchu
 }
 
 // What a product takes: a tile class with its K split, or one of the classes
-// that divide K among a workgroup's wavefronts (numbered after the tiles'),
-// whichever its model finds faster.  The tiles' model leaves out the launch and
+// that divide K among a workgroup's wavefronts (numbered after the tiles') and
+// fold its sums as that split does, whichever its model finds faster.  The tiles' model leaves out the launch and
 // was fitted before their k loop gained: in this comparison their time is
 // kTileLaunch + kTileScale of it, fitted with the other classes'.
 int sgemm_f32_choose(int64_t M, int64_t N, int64_t K, int64_t* splits, int64_t* kchunk) {
@@ -525,22 +525,13 @@ int sgemm_f32_choose(int64_t M, int64_t N, int64_t K, int64_t* splits, int64_t* 
     const int cls = choose_tiles(M, N, K, splits, kchunk, &t);
     t = kTileLaunch + kTileScale * t;
     const int wave = sgemm_f32_wave_class(M, N, K, &t);
-    if (wave < 0) return cls;
-    *splits = 1;
-    *kchunk = K;
-    return kTileClasses + wave;
+    return wave < 0 ? cls : kTileClasses + wave;
 }
 
 int64_t sgemm_f32_splits(int64_t M, int64_t N, int64_t K, int64_t* kchunk) {
     int64_t splits = 1;
-    sgemm_f32_choose(M, N, K, &splits, kchunk);
-    return splits;
-}
-
-int64_t sgemm_f32_tile_splits(int64_t M, int64_t N, int64_t K) {
-    int64_t splits = 1, kchunk = K;
     double t = 0.0;
-    choose_tiles(M, N, K, &splits, &kchunk, &t);
+    choose_tiles(M, N, K, &splits, kchunk, &t);
     return splits;
 }
 
@@ -574,7 +565,7 @@ omb_status launch_sgemm_f32(int64_t M, int64_t N, int64_t K, float alpha,
     const int cls = sgemm_f32_choose(M, N, K, &splits, &kchunk);
     if (cls >= kTileClasses)
         return launch_sgemm_f32_wave(cls - kTileClasses, M, N, K, alpha, A, lda, a_kc, B, ldb, b_nc,
-                                     beta, C, ldc, s);
+                                     beta, C, ldc, kchunk, s);
     const F32Class& fc = kF32Classes[cls];
     Args a{M, N, K, alpha, beta, A, lda, B, ldb, C, ldc, ceil_div(M, fc.bm), ceil_div(N, fc.bn),
            kchunk, nullptr};

@@ -8,9 +8,12 @@
 // w + W, ... of the whole tile, each from zero, with 4*GR x 4*GC outputs per
 // lane; after every W blocks the wavefronts' block sums meet in LDS and are
 // added to the tile in block order.  That is the unsplit kernel's own fold,
-// outer = ((b0 + b1) + b2) ..., so the bits are those of sgemm_f32_kernel for
-// any W and K, with no partial sums in memory and no second launch, and a
-// wavefront holds one accumulator tile instead of two.
+// outer = ((b0 + b1) + b2) ..., and where the tile classes would split K in
+// coarser pieces, whose sums are shorter and err less, the fold starts anew at
+// every piece and the pieces' sums (kept in LDS) are added in order.  So the
+// bits are those of sgemm_f32_kernel with that split for any W and K, with no
+// partial sums in memory and no second launch, and a wavefront holds one
+// accumulator tile instead of two.
 //
 // Each wavefront stages its own 16-k slices of A and B through its own LDS
 // buffers (LDS operations of a wavefront complete in order, so the k loop has
@@ -32,6 +35,7 @@ namespace {
 using namespace wave;
 
 constexpr int kGroupM = 8;
+constexpr int kOneSegment = 1 << 30;  // more blocks than an operand that fits in memory has
 
 struct WArgs {
     int64_t M, N, K;
@@ -43,12 +47,14 @@ struct WArgs {
     float* C;
     int64_t ldc;
     int64_t tiles_m, tiles_n;
+    int seg;  // accumulation blocks per segment of the fold (kOneSegment: all of K)
 };
 
 // GR, GC: 4-row and 4-column groups per lane (8 x 8 lanes: BM = 32*GR, BN =
 // 32*GC); W wavefronts; D slices of loads in flight.
 template <int GR, int GC, int W, int D, int OCC, bool A_KC, bool B_NC, typename Off>
 __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
+    static_assert(W > 1, "the wavefronts share K");
     constexpr int BM = 32 * GR, BN = 32 * GC, TR = 4 * GR;
     constexpr int S = TR * GC;            // float4 of the tile per lane
     constexpr int P = S > 4 ? 2 : 1;      // passes of the LDS sum (bounds its LDS)
@@ -58,6 +64,7 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
         acc4 sum[W][SP][64];
     };
     __shared__ __attribute__((aligned(16))) Shared sh;
+    __shared__ acc4 total[P * OWN][64 * W];  // the segments' sums, each thread's own
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lx = lane & 7, ly = lane >> 3;
@@ -83,6 +90,7 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
 #pragma unroll
     for (int o = 0; o < P * OWN; ++o) outer[o] = acc4{0.f, 0.f, 0.f, 0.f};
     const int64_t nblk = ceil_div(p.K, BLOCK_K);
+    int left = p.seg, left_now = 0;  // blocks until the segment ends
     for (int64_t first = 0; first < nblk; first += W) {
         const int64_t blk = first + wave;
         if (blk < nblk) {
@@ -137,34 +145,45 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
         // Block sums -> LDS, added in block order by the wavefront that owns
         // each float4 of the lanes' tiles.
         const int in_round = (int)std::min<int64_t>(W, nblk - first);
-        if constexpr (W > 1) {
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
-                __syncthreads();  // the staging buffers, or the last pass, are read
-                if (wave < in_round) {
+        for (int q = 0; q < P; ++q) {
+            __syncthreads();  // the staging buffers, or the last pass, are read
+            if (wave < in_round) {
 #pragma unroll
-                    for (int s = 0; s < SP; ++s)
-                        sh.sum[wave][s][lane] = inner[(q * SP + s) / GC][(q * SP + s) % GC];
-                }
-                __syncthreads();
-                for (int w = 0; w < in_round; ++w) {
+                for (int s = 0; s < SP; ++s)
+                    sh.sum[wave][s][lane] = inner[(q * SP + s) / GC][(q * SP + s) % GC];
+            }
+            __syncthreads();
+            left_now = left;
+            for (int w = 0, e; w < in_round; w = e) {
+                e = std::min(in_round, w + left_now);
+                for (int b = w; b < e; ++b) {
 #pragma unroll
                     for (int o = 0; o < OWN; ++o) {
                         const int slot = wave * OWN + o;
                         if (slot >= SP) continue;
-                        outer[q * OWN + o] += sh.sum[w][slot][lane];
+                        outer[q * OWN + o] += sh.sum[b][slot][lane];
                     }
                 }
+                left_now -= e - w;
+                if (left_now > 0) continue;
+                left_now = p.seg;
+#pragma unroll
+                for (int o = 0; o < OWN; ++o) {
+                    acc4& t = total[q * OWN + o][threadIdx.x];
+                    t = first + e == p.seg ? outer[q * OWN + o] : t + outer[q * OWN + o];
+                    outer[q * OWN + o] = acc4{0.f, 0.f, 0.f, 0.f};
+                }
             }
-            if (first + W < nblk) __syncthreads();  // before the next round's staging
-        } else {
-#pragma unroll
-            for (int i = 0; i < TR; ++i)
-#pragma unroll
-                for (int h = 0; h < GC; ++h) outer[i * GC + h] += inner[i][h];
         }
+        left = left_now;
+        if (first + W < nblk) __syncthreads();  // before the next round's staging
     }
 
+    if (nblk >= p.seg) {
+#pragma unroll
+        for (int o = 0; o < P * OWN; ++o) outer[o] += total[o][threadIdx.x];
+    }
     // Whole quads at any alignment, the reads of C ahead of the writes.
     const int rows = (int)std::min<int64_t>(p.M - m0, BM), cols = (int)std::min<int64_t>(p.N - n0, BN);
     float* const c0 = p.C + m0 * p.ldc + n0;
@@ -264,10 +283,11 @@ int sgemm_f32_wave_class(int64_t M, int64_t N, int64_t K, double* time) {
 omb_status launch_sgemm_f32_wave(int cls, int64_t M, int64_t N, int64_t K, float alpha,
                                  const float* A, int64_t lda, bool a_kc, const float* B,
                                  int64_t ldb, bool b_nc, float beta, float* C, int64_t ldc,
-                                 hipStream_t s) {
+                                 int64_t kchunk, hipStream_t s) {
     const WaveClass& k = kWaveClasses[cls];
     const WArgs p{M, N, K, alpha, beta, A, lda, B, ldb, C, ldc,
-                  ceil_div(M, 32 * k.gr), ceil_div(N, 32 * k.gc)};
+                  ceil_div(M, 32 * k.gr), ceil_div(N, 32 * k.gc),
+                  kchunk < K && kchunk > BLOCK_K ? (int)(kchunk / BLOCK_K) : kOneSegment};
     if (cls == 0) launch_class<2, 2, 8, 1>(p, a_kc, b_nc, s);
     else if (cls == 1) launch_class<1, 1, 8, 2>(p, a_kc, b_nc, s);
     else if (cls == 2) launch_class<1, 1, 4, 5>(p, a_kc, b_nc, s);
