@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
 #pragma unroll
                 for (int h = 0; h < GC; ++h) inner[i][h] = acc4{0.f, 0.f, 0.f, 0.f};
             const int64_t kb = blk * BLOCK_K, ke = std::min<int64_t>(p.K, kb + BLOCK_K);
-            const int nfull = (int)full_slices(kb, ke, p.K, tail);
+            const int nfull = full_slices((int)std::min<int64_t>(p.K - kb, 2 * BLOCK_K), BLOCK_K, tail);
             const int64_t klast = kb + (int64_t)std::max(nfull - 1, 0) * BK;
             float4 va[D][sa.L], vb[D][sb.L];
             auto load = [&](int set, int64_t k) {

@@ -29,14 +29,15 @@ __host__ __device__ __forceinline__ int slice_tail(int n, int64_t ld) {
     return KC || n % 4 == 0 ? 0 : (ld < 4 ? 3 : 1);
 }
 
-// The slices of the range [kb, ke) of a product's K that unguarded loads may
-// take, given the larger tail of its two operands.  The tail counts from the end
-// of K, not of the range: with K = 129 the last three k begin in the block of 128
-// before the last.
-__host__ __device__ __forceinline__ int64_t full_slices(int64_t kb, int64_t ke, int64_t K,
-                                                        int tail) {
-    const int64_t n = std::min(ke, K - tail) - kb;
-    return n > 0 ? (int64_t)((uint64_t)n / kSliceK) : 0;
+// The slices that unguarded loads may take of a range of `len` k, from whose first
+// k on the product has `left` (any value of at least len + 3 stands for a larger
+// one), given the larger tail of its two operands.  The tail counts from the end of
+// K, not of the range: with K = 129 the last three k begin in the block of 128
+// before the last.  Blocks count in 32 bits, 0.1 us of a small product.
+template <typename T>
+__host__ __device__ __forceinline__ T full_slices(T left, T len, int tail) {
+    const T n = std::min(left - tail, len);
+    return n > 0 ? n / kSliceK : 0;
 }
 
 }  // namespace omb
