@@ -81,6 +81,9 @@ omb_status resolve_layout(const char* name, int64_t rows, int64_t cols, int64_t 
 // against 7.3); an update of 120 MB: equal.
 constexpr int64_t kStreamBytes = (int64_t)96 << 20;
 constexpr int kLineFloats = 32;  // floats per 128-byte line
+// Work-items (workgroups times threads) along one dimension of a launch stay
+// below this.
+constexpr int64_t kLaunchItems = (int64_t)1 << 32;
 
 // ------------------------------------------------------------ kernels -----
 // Plain FP32 SGEMM, row-major C (ldc), A K-contiguous iff a_kc, B N-contiguous

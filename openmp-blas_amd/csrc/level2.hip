@@ -417,7 +417,8 @@ extern "C" omb_status omb_stranspose(int64_t M, int64_t N, const float* A, int64
         const int64_t rt = big ? 128 : 64, ct = big ? 64 : 32;
         // rows of D moved back by up to 31 floats can need one tile more
         const int64_t GR = ceil_div(R + (on_lines ? 0 : kLine - 1), rt), GC = ceil_div(Cc, ct);
-        const dim3 grid((unsigned)std::min<int64_t>(round_up(GR * GC, 8), 1 << 24));
+        // (the kernel strides over the tiles; 2 x 2^30 has as many as exceed a launch)
+        const dim3 grid((unsigned)std::min<int64_t>(round_up(GR * GC, 8), kLaunchItems / NT / 4));
         const auto kernel = big ? transpose_lines_kernel<128, 64> : transpose_lines_kernel<64, 32>;
         hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, s, R, Cc, (unsigned)GR, (unsigned)GC, A, lda, C, ldc,
                            on_lines ? 1 : 0, diag ? 1 : 0);
