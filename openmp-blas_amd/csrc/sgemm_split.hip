@@ -405,16 +405,18 @@ __global__ __launch_bounds__(NT, 2) void sgemm_bf16x3_kernel(MArgs p) {
 // 64 x 64 x 60000: 137-276, 70-77; 8192^3: 3763-3777, 3746-3768.
 constexpr int kAmaxRows = 32, kAmaxThreads = 1024;
 constexpr int64_t kAmaxRange = 4096;  // least k of a range
+// g0: the launch's first group of rows.
 __global__ __launch_bounds__(kAmaxThreads) void amax_pair_kernel(PackOperand a, PackOperand b,
                                                                  int64_t K, int64_t groups_a,
-                                                                 int64_t range) {
+                                                                 int64_t range, int64_t g0) {
     __shared__ unsigned top[kAmaxRows];
-    const bool first = (int64_t)blockIdx.x < groups_a;
+    const int64_t group = g0 + blockIdx.x;
+    const bool first = group < groups_a;
     const PackOperand& o = first ? a : b;
     const int64_t kb = (int64_t)blockIdx.y * range;
     const float* const X = o.X + kb * o.cs;
     K = std::min(K - kb, range);
-    const int64_t r0 = ((int64_t)blockIdx.x - (first ? 0 : groups_a)) * kAmaxRows;
+    const int64_t r0 = (group - (first ? 0 : groups_a)) * kAmaxRows;
     const int rows = (int)std::min<int64_t>(o.R - r0, kAmaxRows), tid = threadIdx.x;
     auto most = [](unsigned m, float4 v) {
         return max(m, max(max(__float_as_uint(fabsf(v.x)), __float_as_uint(fabsf(v.y))),
@@ -533,7 +535,7 @@ omb_status launch_split_pack_pair(int64_t M, int64_t N, int64_t K, const float* 
                         nullptr, nullptr};
     const PackOperand b{Bt, N, rsB, csB, csB == 1 ? 1 : 0, bp, N > 0 ? ceil_div(N, TM) : 0,
                         nullptr, nullptr};
-    if ((a.rtiles + b.rtiles) * kgroups > 0x7fffffffLL || kgroups > 65535) {
+    if ((a.rtiles + b.rtiles) * kgroups * NT >= kLaunchItems || kgroups > 65535) {
         set_error("split pack: operands too large for one launch");
         return OMB_EUNSUPPORTED;
     }
@@ -556,8 +558,11 @@ omb_status launch_amax_pair(const PackOperand& a, const PackOperand& b, int64_t 
     if (ranges > 1)
         hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(a.R + b.R, NT), 1024)),
                            dim3(NT), 0, s, a.amax, a.R + b.R);
-    hipLaunchKernelGGL(amax_pair_kernel, dim3((unsigned)(ga + gb), (unsigned)ceil_div(K, range)),
-                       dim3(kAmaxThreads), 0, s, a, b, K, ga, range);
+    constexpr int64_t kMost = kLaunchItems / kAmaxThreads - 1;  // groups of one launch
+    for (int64_t g0 = 0; g0 < ga + gb; g0 += kMost)
+        hipLaunchKernelGGL(amax_pair_kernel,
+                           dim3((unsigned)std::min(ga + gb - g0, kMost), (unsigned)ceil_div(K, range)),
+                           dim3(kAmaxThreads), 0, s, a, b, K, ga, range, g0);
     OMB_HIP_TRY(hipGetLastError());
     return OMB_OK;
 }
@@ -682,8 +687,7 @@ omb_status launch_sgemm_split16_ws(int64_t M, int64_t N, int64_t K, float alpha,
     const int64_t kgroups = ceil_div(ceil_div(K, TK), SPLIT_SL);
     const PackOperand oa{A, M, rsA, csA, csA == 1 ? 1 : 0, ap, ceil_div(M, TM), amax_a, ea};
     const PackOperand ob{B, N, csB, rsB, rsB == 1 ? 1 : 0, bp, ceil_div(N, TM), amax_b, eb};
-    if (ceil_div(M, (int64_t)kAmaxRows) + ceil_div(N, (int64_t)kAmaxRows) > 0x7fffffffLL ||
-        kgroups > 65535 || (oa.rtiles + ob.rtiles) * kgroups > 0x7fffffffLL) {
+    if (kgroups > 65535 || (oa.rtiles + ob.rtiles) * kgroups * NT >= kLaunchItems) {
         set_error("split pack: operands too large for one launch");
         return OMB_EUNSUPPORTED;
     }
