@@ -272,7 +272,7 @@ int sgemm_f32_wave_class(int64_t M, int64_t N, int64_t K, double* time) {
                             (r >= 1.0 && r < 4.0 ? std::sqrt(std::ceil(r) / r) : 1.0);
         const double chain = (double)rounds * k.block * std::min(1.0, (double)K / BLOCK_K);
         const double t = (k.fixed + std::max(chain, full)) * 1e-6;
-        if (tiles <= 0x7fffffffLL && t < *time) {
+        if (tiles * 64 * k.w < kLaunchItems && t < *time) {
             best = c;
             *time = t;
         }

@@ -17,7 +17,6 @@ namespace {
 
 using namespace split;
 
-constexpr int NT = 256;  // threads of a group
 
 struct TArgs {
     int64_t M, N, K;
@@ -134,7 +133,6 @@ int sgemm_split_tile_groups(int64_t M, int64_t N, int64_t K, int nprod, bool f16
     // tell them from those that it made slower (3698 x 53 x 2062: 48 us packed, 57).
     if (f16 && K > 2000) return 0;
     const int64_t tiles = ceil_div(M, (int64_t)kLines) * ceil_div(N, (int64_t)kLines);
-    if (tiles > 0x7fffffffLL) return 0;
     const FormModel& f = kForms[f16 ? 2 : nprod == 3 ? 1 : 0];
     const double cus = (double)device_cu_count(), slices = (double)ceil_div(K, (int64_t)TK);
     const double blocks = (double)ceil_div(K, (int64_t)TK * kFoldSlices);
@@ -146,7 +144,7 @@ int sgemm_split_tile_groups(int64_t M, int64_t N, int64_t K, int nprod, bool f16
                   (splits > 1.0 ? q.part * 1e-6 * (double)M * (double)N * splits : 0.0);
     int groups = 0;
     for (const TileModel& t : f.tile) {
-        if (!t.groups) continue;
+        if (!t.groups || tiles * split::NT * t.groups >= kLaunchItems) continue;
         const double rounds = std::ceil(blocks / t.groups);
         const double chain = t.groups == 1 ? slices * t.step
                                            : rounds * (std::min(16.0, slices) * t.step + t.fold);
@@ -168,7 +166,7 @@ omb_status launch_sgemm_split_tile(int groups, int64_t M, int64_t N, int64_t K, 
                                    int nprod, const unsigned* amax_a, const unsigned* amax_b,
                                    hipStream_t s) {
     const int64_t tiles_m = ceil_div(M, (int64_t)kLines), tiles_n = ceil_div(N, (int64_t)kLines);
-    if (tiles_m * tiles_n > 0x7fffffffLL) {
+    if (tiles_m * tiles_n * split::NT * groups >= kLaunchItems) {
         set_error("sgemm split: too many tiles for one launch");
         return OMB_EUNSUPPORTED;
     }
