@@ -348,7 +348,7 @@ __device__ __forceinline__ void tile_quads(const DGemm& g, int tm, int tn, float
             inner[i][0] = acc4{0.f, 0.f, 0.f, 0.f};
         }
     };
-    const int64_t K = g.K, nfull = full_slices(K, K, std::max(sa.tail(), sb.tail()));
+    const int64_t K = g.K, nfull = full_slices(K, 0, std::max(sa.tail(), sb.tail()));
     float4 va[2][sa.L], vb[2][sb.L];
     auto load = [&](int set, int64_t s) {
         const int64_t k0 = std::min(s, nfull - 1) * BK;
@@ -424,7 +424,7 @@ __device__ __forceinline__ void tile_shared_k(const DGemm& g, int tm, int tn, fl
         for (int i = 0; i < 4; ++i) inner[i][0] = acc4{0.f, 0.f, 0.f, 0.f};
         const int64_t kb = (first + w) * BLOCK_K, ke = std::min<int64_t>(K, kb + BLOCK_K);
         if (kb < K) {
-            const int nfull = full_slices((int)std::min<int64_t>(K - kb, 2 * BLOCK_K), BLOCK_K, tail);
+            const int nfull = full_slices((int)(ke - kb), K - ke, tail);
             float4 va[2][sa.L], vb[2][sb.L];
             auto load = [&](int set, int s) {
                 const int64_t k0 = kb + std::min(s, nfull - 1) * BK;

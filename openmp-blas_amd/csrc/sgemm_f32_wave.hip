@@ -17,15 +17,16 @@
 //
 // Each wavefront stages its own 16-k slices of A and B through its own LDS
 // buffers (LDS operations of a wavefront complete in order, so the k loop has
-// no workgroup barrier), with D slices of global loads in flight.  Rows and
+// no workgroup barrier), with the next slice's global loads in flight.  Rows and
 // columns past C are clamped to valid addresses: what they give is never
 // stored.  Only K's last slice (and the last slice of a tile whose 4-column
 // loads could pass the end of an operand) loads element by element.
 //
 // Bound by FP32 issue once the chip is full; below that by the launch and one
-// memory round trip per D slices.
+// memory round trip per slice.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "sgemm_wave.hpp"
 
@@ -35,7 +36,6 @@ namespace {
 using namespace wave;
 
 constexpr int kGroupM = 8;
-constexpr int kOneSegment = 1 << 30;  // more blocks than an operand that fits in memory has
 
 struct WArgs {
     int64_t M, N, K;
@@ -47,12 +47,14 @@ struct WArgs {
     float* C;
     int64_t ldc;
     int64_t tiles_m, tiles_n;
-    int seg;  // accumulation blocks per segment of the fold (kOneSegment: all of K)
+    int seg;  // accumulation blocks per piece of K, or 0: K is one piece
 };
 
 // GR, GC: 4-row and 4-column groups per lane (8 x 8 lanes: BM = 32*GR, BN =
-// 32*GC); W wavefronts; D slices of loads in flight.
-template <int GR, int GC, int W, int D, int OCC, bool A_KC, bool B_NC, typename Off>
+// 32*GC); W wavefronts.  PIECES: K is folded in pieces of p.seg blocks; a build of
+// its own, since the code for them made products of few k up to 7% slower
+// (1150 x 1310 x 33: 8.2 us, 8.8 with one build for both).
+template <int GR, int GC, int W, int OCC, bool PIECES, bool A_KC, bool B_NC, typename Off>
 __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
     static_assert(W > 1, "the wavefronts share K");
     constexpr int BM = 32 * GR, BN = 32 * GC, TR = 4 * GR;
@@ -64,7 +66,7 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
         acc4 sum[W][SP][64];
     };
     __shared__ __attribute__((aligned(16))) Shared sh;
-    __shared__ acc4 total[P * OWN][64 * W];  // the segments' sums, each thread's own
+    __shared__ acc4 total[PIECES ? P * OWN : 1][PIECES ? 64 * W : 1];  // the pieces' sums, each thread's own
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lx = lane & 7, ly = lane >> 3;
@@ -90,7 +92,7 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
 #pragma unroll
     for (int o = 0; o < P * OWN; ++o) outer[o] = acc4{0.f, 0.f, 0.f, 0.f};
     const int64_t nblk = ceil_div(p.K, BLOCK_K);
-    int left = p.seg, left_now = 0;  // blocks until the segment ends
+    int left = p.seg;  // blocks until the piece ends
     for (int64_t first = 0; first < nblk; first += W) {
         const int64_t blk = first + wave;
         if (blk < nblk) {
@@ -99,46 +101,42 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
 #pragma unroll
                 for (int h = 0; h < GC; ++h) inner[i][h] = acc4{0.f, 0.f, 0.f, 0.f};
             const int64_t kb = blk * BLOCK_K, ke = std::min<int64_t>(p.K, kb + BLOCK_K);
-            const int nfull = full_slices((int)std::min<int64_t>(p.K - kb, 2 * BLOCK_K), BLOCK_K, tail);
+            const int nfull = full_slices((int)(ke - kb), p.K - ke, tail);
             const int64_t klast = kb + (int64_t)std::max(nfull - 1, 0) * BK;
-            float4 va[D][sa.L], vb[D][sb.L];
-            auto load = [&](int set, int64_t k) {
+            float4 va[sa.L], vb[sb.L];
+            auto load = [&](int64_t k) {
                 k = k < klast ? k : klast;
-                sa.load(va[set], oa, k);
-                sb.load(vb[set], ob, k);
+                sa.load(va, oa, k);
+                sb.load(vb, ob, k);
             };
-            auto store = [&](int set) {
+            auto store = [&] {
                 wave_lds_fence();
-                sa.store(st.a, va[set]);
-                sb.store(st.b, vb[set]);
+                sa.store(st.a, va);
+                sb.store(st.b, vb);
                 wave_lds_fence();
             };
             int s = 0;
-            if (nfull >= D) {
-#pragma unroll
-                for (int d = 0; d < D; ++d) load(d, kb + d * BK);
-                store(0);
-                for (; s + D <= nfull; s += D) {
+            if (nfull > 1) {
+                load(kb);
+                store();
+                for (; s < nfull; ++s) {  // slice s is staged
                     pin(inner);
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {  // slice s + d is staged, set d free
-                        load(d, kb + (int64_t)(s + D + d) * BK);
-                        __builtin_amdgcn_sched_barrier(0);
-                        compute();
-                        store((d + 1) % D);
-                    }
+                    load(kb + (int64_t)(s + 1) * BK);
+                    __builtin_amdgcn_sched_barrier(0);
+                    compute();
+                    store();
                 }
             }
-            // what the last block leaves: fewer than D full slices, K % 16
+            // a lone slice, and what unguarded loads leave: K % 16, the end of K
 #pragma unroll 1
             for (int64_t k = kb + (int64_t)s * BK; k < ke; k += BK, ++s) {
                 if (s < nfull) {
-                    load(0, k);
+                    load(k);
                 } else {
-                    sa.load_guarded(va[0], k, std::min<int64_t>(ke, k + BK));
-                    sb.load_guarded(vb[0], k, std::min<int64_t>(ke, k + BK));
+                    sa.load_guarded(va, k, std::min<int64_t>(ke, k + BK));
+                    sb.load_guarded(vb, k, std::min<int64_t>(ke, k + BK));
                 }
-                store(0);
+                store();
                 compute();
             }
         }
@@ -154,9 +152,9 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
                     sh.sum[wave][s][lane] = inner[(q * SP + s) / GC][(q * SP + s) % GC];
             }
             __syncthreads();
-            left_now = left;
+            int until = left;
             for (int w = 0, e; w < in_round; w = e) {
-                e = std::min(in_round, w + left_now);
+                e = PIECES ? std::min(in_round, w + until) : in_round;
                 for (int b = w; b < e; ++b) {
 #pragma unroll
                     for (int o = 0; o < OWN; ++o) {
@@ -165,22 +163,24 @@ __global__ __launch_bounds__(64 * W, OCC) void sgemm_f32_wave_kernel(WArgs p) {
                         outer[q * OWN + o] += sh.sum[b][slot][lane];
                     }
                 }
-                left_now -= e - w;
-                if (left_now > 0) continue;
-                left_now = p.seg;
+                if constexpr (PIECES) {
+                    until -= e - w;
+                    if (until > 0) continue;
+                    until = p.seg;
 #pragma unroll
-                for (int o = 0; o < OWN; ++o) {
-                    acc4& t = total[q * OWN + o][threadIdx.x];
-                    t = first + e == p.seg ? outer[q * OWN + o] : t + outer[q * OWN + o];
-                    outer[q * OWN + o] = acc4{0.f, 0.f, 0.f, 0.f};
+                    for (int o = 0; o < OWN; ++o) {
+                        acc4& t = total[q * OWN + o][threadIdx.x];
+                        t = first + e == p.seg ? outer[q * OWN + o] : t + outer[q * OWN + o];
+                        outer[q * OWN + o] = acc4{0.f, 0.f, 0.f, 0.f};
+                    }
                 }
             }
+            if (q == P - 1) left = until;
         }
-        left = left_now;
         if (first + W < nblk) __syncthreads();  // before the next round's staging
     }
 
-    if (nblk >= p.seg) {
+    if constexpr (PIECES) {  // K has more than one
 #pragma unroll
         for (int o = 0; o < P * OWN; ++o) outer[o] += total[o][threadIdx.x];
     }
@@ -246,15 +246,19 @@ template <int GR, int GC, int W, int OCC>
 void launch_class(const WArgs& p, bool a_kc, bool b_nc, hipStream_t s) {
     const bool near = offsets_fit32(a_kc, p.lda, std::min<int64_t>(p.M, 32 * GR)) &&
                       offsets_fit32(!b_nc, p.ldb, std::min<int64_t>(p.N, 32 * GC));
-    auto pick = [&](auto off) {
+    auto pick = [&](auto off, auto pieces) {
         using Off = decltype(off);
-        return a_kc ? (b_nc ? sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, true, true, Off>
-                            : sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, true, false, Off>)
-                    : (b_nc ? sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, false, true, Off>
-                            : sgemm_f32_wave_kernel<GR, GC, W, 1, OCC, false, false, Off>);
+        constexpr bool P = decltype(pieces)::value;
+        return a_kc ? (b_nc ? sgemm_f32_wave_kernel<GR, GC, W, OCC, P, true, true, Off>
+                            : sgemm_f32_wave_kernel<GR, GC, W, OCC, P, true, false, Off>)
+                    : (b_nc ? sgemm_f32_wave_kernel<GR, GC, W, OCC, P, false, true, Off>
+                            : sgemm_f32_wave_kernel<GR, GC, W, OCC, P, false, false, Off>);
     };
-    hipLaunchKernelGGL(near ? pick(0u) : pick((int64_t)0), dim3((unsigned)(p.tiles_m * p.tiles_n)),
-                       dim3(64 * W), 0, s, p);
+    const std::true_type yes;
+    const std::false_type no;
+    const auto kernel = p.seg ? (near ? pick(0u, yes) : pick((int64_t)0, yes))
+                              : (near ? pick(0u, no) : pick((int64_t)0, no));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(64 * W), 0, s, p);
 }
 
 }  // namespace
@@ -287,7 +291,7 @@ omb_status launch_sgemm_f32_wave(int cls, int64_t M, int64_t N, int64_t K, float
     const WaveClass& k = kWaveClasses[cls];
     const WArgs p{M, N, K, alpha, beta, A, lda, B, ldb, C, ldc,
                   ceil_div(M, 32 * k.gr), ceil_div(N, 32 * k.gc),
-                  kchunk < K && kchunk > BLOCK_K ? (int)(kchunk / BLOCK_K) : kOneSegment};
+                  kchunk < K && kchunk > BLOCK_K ? (int)(kchunk / BLOCK_K) : 0};
     if (cls == 0) launch_class<2, 2, 8, 1>(p, a_kc, b_nc, s);
     else if (cls == 1) launch_class<1, 1, 8, 2>(p, a_kc, b_nc, s);
     else if (cls == 2) launch_class<1, 1, 4, 5>(p, a_kc, b_nc, s);

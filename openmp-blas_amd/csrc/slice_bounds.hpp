@@ -29,14 +29,15 @@ __host__ __device__ __forceinline__ int slice_tail(int n, int64_t ld) {
     return KC || n % 4 == 0 ? 0 : (ld < 4 ? 3 : 1);
 }
 
-// The slices that unguarded loads may take of a range of `len` k, from whose first
-// k on the product has `left` (any value of at least len + 3 stands for a larger
-// one), given the larger tail of its two operands.  The tail counts from the end of
-// K, not of the range: with K = 129 the last three k begin in the block of 128
-// before the last.  Blocks count in 32 bits, 0.1 us of a small product.
+// The slices that unguarded loads may take of a range of `len` k of a product
+// that has `after` more k behind the range, given the larger tail of its two
+// operands.  The tail counts from the end of K, not of the range: with K = 129 the
+// last three k begin in the block of 128 before the last.  (As a lower bound of
+// two ends, min(len, len + after - tail), the same cost products of a partial slice
+// up to 2%: 1000 x 700 x 100 9.44 us, 9.30 so.)
 template <typename T>
-__host__ __device__ __forceinline__ T full_slices(T left, T len, int tail) {
-    const T n = std::min(left - tail, len);
+__host__ __device__ __forceinline__ T full_slices(T len, int64_t after, int tail) {
+    const T n = len - (after < tail ? tail - (int)after : 0);
     return n > 0 ? n / kSliceK : 0;
 }
 

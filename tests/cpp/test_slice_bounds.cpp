@@ -18,12 +18,7 @@ static void walk(int n, int64_t ld, int64_t K, int64_t range) {
     const int tail = slice_tail<KC>(n, ld);
     const int64_t last = KC ? (n - 1) * ld + K - 1 : (K - 1) * ld + n - 1;
     for (int64_t kb = 0; kb < K; kb += range) {
-        const int64_t ke = std::min(K, kb + range), full = full_slices(K - kb, range, tail);
-        // as the kernels count blocks
-        if (range == 128 && full_slices((int)std::min<int64_t>(K - kb, 256), 128, tail) != full) {
-            std::fprintf(stderr, "FAILED: 32 and 64 bits differ at K %ld\n", (long)K);
-            std::exit(1);
-        }
+        const int64_t ke = std::min(K, kb + range), full = full_slices(ke - kb, K - ke, tail);
         bool ok = full >= 0 && kb + full * kSliceK <= ke;
         for (int64_t s = 0; s < full; ++s)
             for (int e = 0; e < 4 * E; ++e) {
