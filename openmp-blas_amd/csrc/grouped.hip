@@ -100,16 +100,13 @@ __device__ __forceinline__ int item_tid() {
 }
 
 // ------------------------------------------------------------ plain tile --
-// BM x BN tile of C = alpha*A*B + beta*C (all row-major); 256 threads on an
-// H x W = (BM/TMR) x (BN/TNR) grid.  Thread (ty, tx) owns GR fragments of FR
-// consecutive rows, at rows g*(BM/GR) + ty*FR + i, and GC fragments of FC
-// consecutive columns (FR = min(TMR, 4), GR = TMR / FR; likewise for
-// columns), so every LDS read is one 64- or 128-bit access.  Slices of 16 k
-// are loaded with 128-bit global loads along the unit-stride index, staged
-// through two LDS buffers, and the next D slices are prefetched into D
-// register sets; LDS fragments for k+1 are read while k's FMAs run.  Every
-// element sums k in order and folds the running sum every 128 k, as
-// sgemm_f32_kernel does, so the results are the same bits.
+// 128 x 64 tile of C = alpha*A*B + beta*C (all row-major); 256 threads on a
+// 16 x 16 grid.  Thread (ty, tx) owns rows g*64 + ty*4 + i (g < 2, i < 4) and
+// columns tx*4 + j (j < 4), so every LDS read is one 128-bit access.  Slices of
+// 16 k are loaded with 128-bit global loads along the unit-stride index one slice
+// ahead and staged through two LDS buffers; LDS fragments for k+1 are read while
+// k's FMAs run.  Every element sums k in order and folds the running sum every
+// 128 k, as sgemm_f32_kernel does, so the results are the same bits.
 template <typename P>
 __device__ __forceinline__ float4 load4_guard(P p, int n) {
     if (n == 4) return ld4u(p);
@@ -122,20 +119,13 @@ __device__ __forceinline__ float4 load4_guard(P p, int n) {
 
 __device__ __forceinline__ int clamp4i(int64_t r) { return r <= 0 ? 0 : (r >= 4 ? 4 : (int)r); }
 
-template <int BM, int BN, int TMR, int TNR, int D>
-__device__ __forceinline__ void tile_f32(const DGemm& g, int tm, int tn, float* smem) {
-    constexpr int BK = 16;
-    constexpr int H = BM / TMR, W = BN / TNR;
-    static_assert(H * W == NT, "thread grid must cover the workgroup");
-    constexpr int FR = TMR < 4 ? TMR : 4, GR = TMR / FR;
-    constexpr int FC = TNR < 4 ? TNR : 4, GC = TNR / FC;
+__device__ __forceinline__ void tile_128x64(const DGemm& g, int tm, int tn, float* smem) {
+    constexpr int BM = 128, BN = 64, BK = 16, W = 16;  // W: threads along a row of the tile
+    constexpr int GR = BM / 64, TMR = 4 * GR, TNR = 4;
     constexpr int kFold = kFoldK / BK;
     constexpr int PA = BM + 4, PB = BN + 4;  // padded LDS rows, 16-byte aligned
-    constexpr int NA4 = BM * BK / 4, NB4 = BN * BK / 4;  // float4 per slice
-    constexpr int LA = (NA4 + NT - 1) / NT, LB = (NB4 + NT - 1) / NT;
-    static_assert(FR == 4 && FC == 4, "fragments are float4");
-    typedef float4 FragA;
-    typedef float4 FragB;
+    constexpr int LA = BM * BK / 4 / NT, LB = BN * BK / 4 / NT;  // float4 per thread and slice
+    static_assert(LA * NT * 4 == BM * BK && LB * NT * 4 == BN * BK, "whole loads");
     // Two LDS buffers of [BK][PA] A and [BK][PB] B: slice k+1 is stored into
     // one while slice k is read from the other (one barrier per slice).
     constexpr int SZ = BK * (PA + PB);
@@ -146,50 +136,42 @@ __device__ __forceinline__ void tile_f32(const DGemm& g, int tm, int tn, float* 
     gcfloat* const gB = as_global(g.B);
     gfloat* const gC = as_global(g.C);
 
-    float4 ra[D][LA], rb[D][LB];  // D slices of loads in flight, one set each
-    auto load = [&](int set, int64_t k0) {
+    float4 ra[LA], rb[LB];  // the slice in flight
+    auto load = [&](int64_t k0) {
 #pragma unroll
-        for (int i = 0; i < LA; ++i) {
+        for (int i = 0; i < LA; ++i) {  // A[m][k]: float4 along k
             const int e = tid + i * NT;
-            if (e < NA4) {  // A[m][k]: float4 along k
-                const int row = e >> 2, kq = (e & 3) * 4;
-                const int64_t m = m0 + row, k = k0 + kq;
-                const int n = m < M ? clamp4i(K - k) : 0;
-                ra[set][i] = load4_guard(gA + (n ? m * g.lda + k : 0), n);
-            }
+            const int row = e >> 2, kq = (e & 3) * 4;
+            const int64_t m = m0 + row, k = k0 + kq;
+            const int n = m < M ? clamp4i(K - k) : 0;
+            ra[i] = load4_guard(gA + (n ? m * g.lda + k : 0), n);
         }
 #pragma unroll
-        for (int i = 0; i < LB; ++i) {
+        for (int i = 0; i < LB; ++i) {  // B[k][n]: float4 along n
             const int e = tid + i * NT;
-            if (e < NB4) {  // B[k][n]: float4 along n
-                const int kk = e / (BN / 4), nq = (e % (BN / 4)) * 4;
-                const int64_t nn = n0 + nq, k = k0 + kk;
-                const int n = k < K ? clamp4i(N - nn) : 0;
-                rb[set][i] = load4_guard(gB + (n ? k * g.ldb + nn : 0), n);
-            }
+            const int kk = e / (BN / 4), nq = (e % (BN / 4)) * 4;
+            const int64_t nn = n0 + nq, k = k0 + kk;
+            const int n = k < K ? clamp4i(N - nn) : 0;
+            rb[i] = load4_guard(gB + (n ? k * g.ldb + nn : 0), n);
         }
     };
-    auto store = [&](int set, int buf) {
+    auto store = [&](int buf) {
         float* As = smem + buf * SZ;
         float* Bs = As + BK * PA;
 #pragma unroll
         for (int i = 0; i < LA; ++i) {
             const int e = tid + i * NT;
-            if (e < NA4) {
-                const int row = e >> 2, kq = (e & 3) * 4;
-                As[(kq + 0) * PA + row] = ra[set][i].x;
-                As[(kq + 1) * PA + row] = ra[set][i].y;
-                As[(kq + 2) * PA + row] = ra[set][i].z;
-                As[(kq + 3) * PA + row] = ra[set][i].w;
-            }
+            const int row = e >> 2, kq = (e & 3) * 4;
+            As[(kq + 0) * PA + row] = ra[i].x;
+            As[(kq + 1) * PA + row] = ra[i].y;
+            As[(kq + 2) * PA + row] = ra[i].z;
+            As[(kq + 3) * PA + row] = ra[i].w;
         }
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
             const int e = tid + i * NT;
-            if (e < NB4) {
-                const int kk = e / (BN / 4), nq = (e % (BN / 4)) * 4;
-                *reinterpret_cast<float4*>(&Bs[kk * PB + nq]) = rb[set][i];
-            }
+            const int kk = e / (BN / 4), nq = (e % (BN / 4)) * 4;
+            *reinterpret_cast<float4*>(&Bs[kk * PB + nq]) = rb[i];
         }
     };
 
@@ -203,22 +185,19 @@ __device__ __forceinline__ void tile_f32(const DGemm& g, int tm, int tn, float* 
     auto compute = [&](int buf, int64_t kt) {
         const float* As = smem + buf * SZ;
         const float* Bs = As + BK * PA;
-        FragA fa[2][GR];
-        FragB fb[2][GC];
+        float4 fa[2][GR], fb[2];
         auto fragment = [&](int k, int set) {
 #pragma unroll
             for (int q = 0; q < GR; ++q)
-                fa[set][q] = *reinterpret_cast<const FragA*>(&As[k * PA + q * (BM / GR) + ty * FR]);
-#pragma unroll
-            for (int q = 0; q < GC; ++q)
-                fb[set][q] = *reinterpret_cast<const FragB*>(&Bs[k * PB + q * (BN / GC) + tx * FC]);
+                fa[set][q] = *reinterpret_cast<const float4*>(&As[k * PA + q * 64 + ty * 4]);
+            fb[set] = *reinterpret_cast<const float4*>(&Bs[k * PB + tx * 4]);
         };
         fragment(0, 0);
 #pragma unroll
         for (int k = 0; k < BK; ++k) {
             if (k + 1 < BK) fragment(k + 1, (k + 1) & 1);
             const float* av = reinterpret_cast<const float*>(fa[k & 1]);
-            const float* bv = reinterpret_cast<const float*>(fb[k & 1]);
+            const float* bv = reinterpret_cast<const float*>(&fb[k & 1]);
 #pragma unroll
             for (int i = 0; i < TMR; ++i)
 #pragma unroll
@@ -234,36 +213,27 @@ __device__ __forceinline__ void tile_f32(const DGemm& g, int tm, int tn, float* 
                 }
         }
     };
-    // Slices 0 .. D-1 are loaded up front; step kt loads slice kt + D into
-    // the set that held slice kt (stored to LDS in step kt - 1), computes
-    // slice kt from LDS buffer kt % 2 and stores slice kt + 1 into the other
-    // buffer, so each load has D - 1 steps of compute to arrive in.
-#pragma unroll
-    for (int s = 0; s < D; ++s)
-        if (s == 0 || s < nk) load(s, s * BK);  // slice 0 even when K = 0 (zeros)
+    // Step kt loads slice kt + 1, computes slice kt from LDS buffer kt % 2 and
+    // stores slice kt + 1 into the other buffer.
+    load(0);  // also when K = 0 (zeros)
     __syncthreads();  // the previous item is done with LDS
-    store(0, 0);
+    store(0);
     __syncthreads();
-    for (int64_t kt0 = 0; kt0 < nk; kt0 += D) {
-#pragma unroll
-        for (int s = 0; s < D; ++s) {
-            const int64_t kt = kt0 + s;
-            if (kt >= nk) break;
-            if (kt + D < nk) load(s, (kt + D) * BK);
-            compute((int)(kt & 1), kt);
-            // The other buffer was last read in step kt - 1, which every
-            // thread finished before the barrier that ended it.
-            if (kt + 1 < nk) store((s + 1) % D, (int)((kt + 1) & 1));
-            __syncthreads();
-        }
+    for (int64_t kt = 0; kt < nk; ++kt) {
+        if (kt + 1 < nk) load((kt + 1) * BK);
+        compute((int)(kt & 1), kt);
+        // The other buffer was last read in step kt - 1, which every thread
+        // finished before the barrier that ended it.
+        if (kt + 1 < nk) store((int)((kt + 1) & 1));
+        __syncthreads();
     }
 #pragma unroll
     for (int i = 0; i < TMR; ++i) {
-        const int64_t m = m0 + (i / FR) * (BM / GR) + ty * FR + (i % FR);
+        const int64_t m = m0 + (i / 4) * 64 + ty * 4 + (i % 4);
         if (m >= M) continue;
 #pragma unroll
         for (int j = 0; j < TNR; ++j) {
-            const int64_t n = n0 + (j / FC) * (BN / GC) + tx * FC + (j % FC);
+            const int64_t n = n0 + tx * 4 + j;
             if (n < N) {
                 gfloat* c = gC + m * g.ldc + n;
                 const float v = g.alpha * outer[i][j];
@@ -634,7 +604,7 @@ __global__ __launch_bounds__(NT, KIND == KBIG ? 2 : 4) void grouped_kernel(PArgs
                     break;
                 case C128x64:
                     if constexpr (KIND == KBIG)
-                        tile_f32<128, 64, 8, 4, 1>(p.gemms[w.inst], w.tm, w.tn, smem);
+                        tile_128x64(p.gemms[w.inst], w.tm, w.tn, smem);
                     break;
                 case CSPLIT:
                     if constexpr (KIND >= KSPLIT6)
@@ -1081,7 +1051,7 @@ extern "C" omb_status omb_autotune_group(const omb_gemm_desc* gemms, int32_t n_g
         if (gemms[i].M > 0 && gemms[i].N > 0) buckets[key_of(mode, gemms[i])].push_back(gemms[i]);
     const int batch = 64;
     // 128x64 is not a candidate: timed alone it can win a bucket, but it
-    // needs the larger-register kernel (2 workgroups per CU instead of 3),
+    // needs the larger-register kernel (2 workgroups per CU instead of 4),
     // which slows every other item of the plan (see default_class); a
     // table loaded with omb_autotune_load may still name it.
     const std::vector<int> cands = mode == OMB_MODE_PLAIN_F32 ? std::vector<int>{C32, C64}

@@ -19,8 +19,6 @@ constexpr int NT = 256;                      // threads per workgroup (4 wavefro
 // Tile rows per L2 group: with 4 (against 8, 6 and 5) split BF16 of 8192^3 took 5408 us
 // (5496, 5516, 5544), scaled FP16 3292 (3371, 3409, 3465); 4096^3 and below the same.
 constexpr int kGroupM = 4;
-constexpr int SLICE_A = 3 * TM * TK;         // bf16 elements per A slice (3 planes)
-constexpr int SLICE_B = 3 * TN * TK;
 constexpr int kFoldSlices = 16;              // inner MFMA accumulation spans 256 k
 
 __device__ inline f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
@@ -98,29 +96,6 @@ __device__ inline void split2_f16(float xs, _Float16& h0, _Float16& h1) {
     h0 = (_Float16)xs;
     h1 = (_Float16)(xs - (float)h0);
 }
-
-// Split 8 consecutive-k values into the three 16-byte plane chunks.
-__device__ inline void split8(float4 lo, float4 hi, uint4& p0, uint4& p1, uint4& p2) {
-    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    bf16x8 a, b, c;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        __bf16 t0, t1, t2;
-        split3(v[j], t0, t1, t2);
-        a[j] = t0;
-        b[j] = t1;
-        c[j] = t2;
-    }
-    p0 = *reinterpret_cast<const uint4*>(&a);
-    p1 = *reinterpret_cast<const uint4*>(&b);
-    p2 = *reinterpret_cast<const uint4*>(&c);
-}
-
-}  // namespace split
-}  // namespace omb
-
-namespace omb {
-namespace split {
 
 // Fragments of one k slice for one wavefront owning BI x BJ blocks of 32x32
 // of C (rows wrow0.., columns wcol0.. of the slice), from the swizzled LDS
