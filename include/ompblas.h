@@ -316,7 +316,9 @@ omb_status omb_server_close(omb_server* server, omb_serve_stats* stats);
 /* The workspace bytes omb_serve_run will hold for request r while it runs
  * (the value it fills into ws_bytes), for sizing hbm_budget; -1 for an
  * invalid request.  Split-BF16 GEMMs hold their packed operands, GEMMs
- * whose K is split hold the partial sums, dots their partials. */
+ * whose K is split hold the partial sums, dots their partials.  The bytes do
+ * not depend on which kernel takes a product: one whose kernel needs no
+ * workspace holds them too, and waits or is refused (OMB_EBUSY) by them. */
 int64_t omb_serve_request_bytes(const omb_request* r);
 
 /* ----------------------------------------------- host-pointer helpers ----

@@ -13,9 +13,9 @@
 // counter took 12 us, in groups of 32 2.4 us.  Below 2^24 elements this beats
 // a second launch (20000: 7.5 -> 5.1 us a call, 1000003: 7.3 -> 6.0); from
 // there the second launch adds the partials, hidden behind the first one's
-// start (2^28: 308 us, 310 with arrivals).  omb_sdot_noalloc and served
-// requests have no counters of their own and take the second launch too, in
-// the same order.  The grid depends on n only and the loads do not depend on
+// start (2^28: 308 us, 310 with arrivals).  omb_sdot_noalloc and captured
+// calls use no counters and take the second launch too, in the same order;
+// served requests use their slot's.  The grid depends on n only and the loads do not depend on
 // alignment, so the result is bitwise reproducible for any placement of the
 // operands.
 #include <algorithm>
