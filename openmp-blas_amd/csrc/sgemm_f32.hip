@@ -227,7 +227,10 @@ __global__ __launch_bounds__(NT, occ_of(BM * BN)) void sgemm_f32_kernel(Args q) 
     Side<BN, !B_NC, Off> sb;
     sa.init(p.A, p.lda, m0, p.M, kbeg, tid);
     sb.init(p.B, p.ldb, n0, p.N, kbeg, tid);
-    const int64_t nfull = full_slices(p.K, q.K - kbeg - p.K, max(sa.tail(), sb.tail()));
+    // (in 32 bits: in 64 the accumulators of one slice in two moved to B's register
+    // banks, and 8192^3 took 0.4% longer)
+    const int after = (int)std::min<int64_t>(q.K - kbeg - p.K, BK);
+    const int64_t nfull = full_slices(p.K, after, max(sa.tail(), sb.tail()));
     int64_t kt = 0;
     if (nfull > 0) {
         // Slices kt and kt+1 in LDS buffers 0 and 1, loads two slices ahead in

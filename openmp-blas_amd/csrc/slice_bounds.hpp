@@ -35,8 +35,8 @@ __host__ __device__ __forceinline__ int slice_tail(int n, int64_t ld) {
 // last three k begin in the block of 128 before the last.  (As a lower bound of
 // two ends, min(len, len + after - tail), the same cost products of a partial slice
 // up to 2%: 1000 x 700 x 100 9.44 us, 9.30 so.)
-template <typename T>
-__host__ __device__ __forceinline__ T full_slices(T len, int64_t after, int tail) {
+template <typename T, typename U>
+__host__ __device__ __forceinline__ T full_slices(T len, U after, int tail) {
     const T n = len - (after < tail ? tail - (int)after : 0);
     return n > 0 ? n / kSliceK : 0;
 }
