@@ -570,7 +570,7 @@ constexpr int kSmemFloats = 2 * (16 * (128 + 4) + 16 * (64 + 4)) + 16;
 // 860 us instead of 783).  All but KBIG are bounded to 4 workgroups per CU (at
 // most 128 VGPRs): the plain plan of 4096 GEMMs and 4096 GEMVs measured 3.48 ms
 // so, against 3.55-3.63 ms for builds of 129 and 165 VGPRs (3 per CU).  KBIG (128x64
-// tiles too) is bounded to 2.
+// tiles too) is bounded to 2 and runs 3 (154 VGPRs).
 enum Kind { KPLAIN, KBIG, KSPLIT6, KSPLIT3, KSPLIT16, NKIND };
 
 template <int KIND>
@@ -668,7 +668,7 @@ Key key_of(int mode, const omb_gemm_desc& d) { return Key{mode, lg(d.M), lg(d.N)
 // 32x32 with K shared by the wavefronts when the smaller output dimension is under
 // 48 and K has three accumulation blocks or more (4096 GEMMs: 621 us so, 648 with
 // every short side in 32x32, 613 with none, 684 with every such K).  (The
-// 128x64 class needs the larger-register kernel, 2 workgroups per CU instead
+// 128x64 class needs the larger-register kernel, 3 workgroups per CU instead
 // of 4, which slows every other item of a mixed plan, so it is used only when a
 // loaded tuning table names it.)
 int default_class(int mode, const omb_gemm_desc& d) {
@@ -1051,7 +1051,7 @@ extern "C" omb_status omb_autotune_group(const omb_gemm_desc* gemms, int32_t n_g
         if (gemms[i].M > 0 && gemms[i].N > 0) buckets[key_of(mode, gemms[i])].push_back(gemms[i]);
     const int batch = 64;
     // 128x64 is not a candidate: timed alone it can win a bucket, but it
-    // needs the larger-register kernel (2 workgroups per CU instead of 4),
+    // needs the larger-register kernel (3 workgroups per CU instead of 4),
     // which slows every other item of the plan (see default_class); a
     // table loaded with omb_autotune_load may still name it.
     const std::vector<int> cands = mode == OMB_MODE_PLAIN_F32 ? std::vector<int>{C32, C64}

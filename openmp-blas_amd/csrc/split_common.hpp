@@ -18,6 +18,8 @@ constexpr int TM = 128, TN = 128, TK = 16;  // C tile and k slice of one workgro
 constexpr int NT = 256;                      // threads per workgroup (4 wavefronts)
 // Tile rows per L2 group: with 4 (against 8, 6 and 5) split BF16 of 8192^3 took 5408 us
 // (5496, 5516, 5544), scaled FP16 3292 (3371, 3409, 3465); 4096^3 and below the same.
+// The workgroups of an XCD do not keep in step, and with 4 rows miss its L2 less: split
+// BF16 of 8192^3 13 to 15 GB a launch, 15 to 17 with 8.
 constexpr int kGroupM = 4;
 constexpr int kFoldSlices = 16;              // inner MFMA accumulation spans 256 k
 
