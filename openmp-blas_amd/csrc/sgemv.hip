@@ -265,6 +265,9 @@ __global__ __launch_bounds__(NT) void sgemv_col_combine_kernel(int64_t M, float 
 // blocks would leave as many chunks as CUs to add per row (100 x 14000: 55 us
 // with 219 chunks added by one thread per row).
 constexpr int64_t kColNarrow = 1024;
+// Tall matrices of at most 256 columns are read with the non-temporal hint from here
+// on (163474 x 64, 42 MB: 7.8 us without, 6.5 with; x 50, 33 MB: 5.0 and 5.8).
+constexpr int64_t kTallStreamBytes = (int64_t)40 << 20;
 
 template <int LR, int U, bool STREAM, bool TINY = false>
 omb_status launch_col(int64_t M, int64_t N, float alpha, const float* A, int64_t lda,
@@ -352,10 +355,40 @@ omb_status launch_sgemv_col(int64_t M, int64_t N, float alpha, const float* A, i
         return OMB_OK;
     }
     if (M < 4) return launch_col<1, 4, false, true>(M, N, alpha, A, lda, x, beta, y, s);
-    if (M <= kColNarrow) return launch_col<16, 8, false>(M, N, alpha, A, lda, x, beta, y, s);
-    if (M * N * (int64_t)sizeof(float) <= kStreamBytes)
-        return launch_col<64, 16, false>(M, N, alpha, A, lda, x, beta, y, s);
-    return launch_col<64, 16, true>(M, N, alpha, A, lda, x, beta, y, s);
+    // Few columns: no more loads in flight per lane than they give one (64 / LR
+    // lane groups of 4 wavefronts take columns apart), since the clamped rest cost
+    // as much as the others: 400000 x 1 10.0 us with 16, 3.7 so.  The sums are the
+    // same for any number of loads.
+    const int64_t bytes = M * N * (int64_t)sizeof(float);
+    const std::true_type stream;
+    const std::false_type cached;
+    auto launch = [&](auto lanes, auto loads, auto hint) {
+        return launch_col<decltype(lanes)::value, decltype(loads)::value, decltype(hint)::value>(
+            M, N, alpha, A, lda, x, beta, y, s);
+    };
+    const std::integral_constant<int, 1> l1;
+    const std::integral_constant<int, 2> l2;
+    const std::integral_constant<int, 4> l4;
+    const std::integral_constant<int, 8> l8;
+    const std::integral_constant<int, 16> l16;
+    const std::integral_constant<int, 64> l64;
+    if (M <= kColNarrow) {
+        if (N <= 16) return launch(l16, l1, cached);
+        if (N <= 32) return launch(l16, l2, cached);
+        return N <= 64 ? launch(l16, l4, cached) : launch(l16, l8, cached);
+    }
+    if (N <= 4) return bytes <= kTallStreamBytes ? launch(l64, l1, cached) : launch(l64, l1, stream);
+    // Tall ones have more workgroups than CUs, of one chunk: several resident on a CU
+    // hide the loads better than more of them per lane (3000000 x 33: 92.8 us with
+    // 16, 66.7 with 4).
+    if (N <= 256 && ceil_div(M, (int64_t)256) >= cus) {
+        if (N <= 128)
+            return bytes <= kTallStreamBytes ? launch(l64, l4, cached) : launch(l64, l4, stream);
+        return bytes <= kTallStreamBytes ? launch(l64, l8, cached) : launch(l64, l8, stream);
+    }
+    if (N <= 16) return launch(l64, l4, cached);
+    if (N <= 32) return launch(l64, l8, cached);
+    return bytes <= kStreamBytes ? launch(l64, l16, cached) : launch(l64, l16, stream);
 }
 
 }  // namespace omb

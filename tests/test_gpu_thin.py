@@ -1,0 +1,26 @@
+"""Thin operands, whose kernels are chosen by their short side: GEMV of few long
+rows or few tall columns, transposes that are one row or one column of tiles.
+Integer operands keep sums exact; a transpose moves bits, its surroundings
+included."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m", [5, 1024, 1025, 65280, 65281, 65537, 163474])
+@pytest.mark.parametrize("n,off", [(1, 0), (4, 1), (5, 0), (16, 3), (17, 0), (32, 0), (33, 1),
+                                   (64, 0), (65, 0), (128, 1), (129, 0), (256, 3), (257, 0)])
+def test_few_columns(dev, ompblas, m, n, off):
+    g = torch.Generator(device=dev).manual_seed(m + n)
+    ld = m + off
+    buf = torch.randint(-9, 10, (n * ld + off,), device=dev, generator=g).float()
+    a = buf[off:].view(n, ld)[:, :m].t()
+    x = torch.randint(-9, 10, (n,), device=dev, generator=g).float()
+    y0 = torch.randint(-9, 10, (m,), device=dev, generator=g).float()
+    for alpha, beta in ((1.0, 1.0), (-2.0, 0.0)):
+        y = y0.clone() if beta else torch.full_like(y0, float("nan"))
+        ompblas.check(ompblas.sgemv(m, n, alpha, a.data_ptr(), 1, ld, x.data_ptr(), beta,
+                                    y.data_ptr()))
+        want = alpha * (a.double() @ x.double()) + beta * y0.double()
+        assert torch.equal(y.double(), want)
