@@ -304,6 +304,11 @@ omb_status launch_col(int64_t M, int64_t N, float alpha, const float* A, int64_t
 // Rows of up to this many columns take 4 rows x 2 loads per wavefront (more
 // loads per row would be past its end: 16000 x 600 9.6 us with 2 x 8, 8.7 us).
 constexpr int64_t kRowShort = 1024;
+// From this many columns on, few rows (up to two wavefronts per CU) are chains of
+// rounds: 8 loads per row without the barrier, so that rounds overlap, with addresses
+// of their own (1 x 34882 9.4 us with 4 x BATCH, 7.8 with 8, 5.9 so; 300 x 12000 5.7
+// and 5.5; but 8 x 8000 4.4 and 4.8, 1000 x 12000 8.9 and 10.0).
+constexpr int64_t kRowLong = 10240;
 
 omb_status launch_sgemv_row(int64_t M, int64_t N, float alpha, const float* A, int64_t lda,
                             const float* x, float beta, float* y, hipStream_t s) {
@@ -333,6 +338,8 @@ omb_status launch_sgemv_row(int64_t M, int64_t N, float alpha, const float* A, i
         launch(sgemv_row_kernel<16, 1, true, true, false>, 16, cus);
     } else if (N <= kRowShort) {
         launch(sgemv_row_kernel<4, 2, false, true, true>, 4, 4 * cus);
+    } else if (M <= 2 * cus && N > kRowLong && !stream) {
+        launch(sgemv_row_kernel<1, 8, false, false, false>, 1, 4 * cus);
     } else if (M < 6 * waves_per_wg * cus) {
         launch(stream ? sgemv_row_kernel<1, 8, true, true, true>
                       : sgemv_row_kernel<1, 4, false, true, true>, 1, 4 * cus);

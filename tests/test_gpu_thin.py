@@ -8,6 +8,30 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("m", [1, 3, 17, 512, 513])
+@pytest.mark.parametrize("n,off", [(10240, 0), (10241, 1), (12003, 0), (34882, 3)])
+def test_few_long_rows(dev, ompblas, m, n, off):
+    g = torch.Generator(device=dev).manual_seed(m * 31 + n)
+    lda = n + off
+    for make in (lambda k: torch.randint(-9, 10, (k,), device=dev, generator=g).float(),
+                 lambda k: torch.rand(k, device=dev, generator=g) * 2 - 1):
+        buf = make(m * lda + off)
+        a, x, y0 = buf[off:].view(m, lda)[:, :n], make(n), make(m)
+        y, z = y0.clone(), y0.clone()
+        ompblas.check(ompblas.sgemv(m, n, -2.0, a.data_ptr(), lda, 1, x.data_ptr(), 1.5,
+                                    y.data_ptr()))
+        plan = ompblas.GroupPlan([], [(m, n, a.data_ptr(), lda, x.data_ptr(), z.data_ptr(), -2.0,
+                                       1.5)])
+        plan.launch()
+        torch.cuda.synchronize()
+        assert torch.equal(y, z)  # the grouped item's bits
+        want = -2.0 * (a.double() @ x.double()) + 1.5 * y0.double()
+        err = (y.double() - want).abs().max().item()
+        assert err <= 2.0 * n * 2.0 ** -24 * 2.0 * a.abs().double().matmul(x.abs().double()).max().item()
+        if buf[0].item() == round(buf[0].item()):
+            assert torch.equal(y.double(), want)
+
+
 @pytest.mark.parametrize("m", [5, 1024, 1025, 65280, 65281, 65537, 163474])
 @pytest.mark.parametrize("n,off", [(1, 0), (4, 1), (5, 0), (16, 3), (17, 0), (32, 0), (33, 1),
                                    (64, 0), (65, 0), (128, 1), (129, 0), (256, 3), (257, 0)])
