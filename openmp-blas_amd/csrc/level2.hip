@@ -249,7 +249,14 @@ __global__ __launch_bounds__(NT) void transpose_lines_kernel(int64_t R, int64_t 
         } else {  // clamped indices: what lies outside S is not stored
 #pragma unroll
             for (int k = 0; k < LR / RPI; ++k) {
-                const int64_t r = r0 - kLine + rr + RPI * k, c = c0 + 4 * cq;
+                // steps of no row of S at all are left out (65 x 2000000: 321 us with
+                // them, 289 so)
+                const int64_t first = r0 - kLine + RPI * k;
+                if (first >= R || first + RPI <= 0) {
+                    v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    continue;
+                }
+                const int64_t r = first + rr, c = c0 + 4 * cq;
                 const float* p = S + std::min(std::max<int64_t>(r, 0), R - 1) * lds;
                 if (c + 3 < Cc) {
                     v[k] = ld4u(p + c);
@@ -292,6 +299,34 @@ __global__ __launch_bounds__(NT) void transpose_lines_kernel(int64_t R, int64_t 
                 }
             }
         }
+    }
+}
+
+// The same for thin matrices, which are one row or one column of tiles: 64 x 64
+// tiles with guards, one per step.  (µs: this, transpose_lines_kernel.)
+//  - R < 64: D's rows are short, and moving them back to lines spreads each over
+//    more lanes that store little: 1 x 2000000 26 and 71, 9 x 2000000 39 and 76
+//    (176 in its large tiles), 48 x 2000000 129 and 196.
+//  - Cc <= 10: few of a tile's columns are there: 2000000 x 1 23 and 30, 300000 x 9
+//    6.4 and 7.3, 2000000 x 12 50 and 38.
+//  - 32 < Cc < 64 where D's rows start on lines: 2000000 x 40 113 and 175 (where
+//    they do not: 227 and 158).
+bool thin_transpose(int64_t R, int64_t Cc, bool on_lines) {
+    return R < 64 || Cc <= 10 || (on_lines && Cc > 32 && Cc < 64);
+}
+__global__ __launch_bounds__(NT) void transpose_thin_kernel(int64_t R, int64_t Cc, int64_t ntiles,
+                                                            const float* __restrict__ S,
+                                                            int64_t lds, float* __restrict__ D,
+                                                            int64_t ldd) {
+    __shared__ float tile[TT][TPAD];
+    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        const int64_t r0 = R < TT ? 0 : t * TT, c0 = R < TT ? t * TT : 0;
+        float4 v[TT / 16];
+        tile_regs(v, S, lds, R, Cc, r0, c0);
+        __syncthreads();  // the previous tile has been written out
+        tile_put(tile, v);
+        __syncthreads();
+        tile_store_t(tile, D, ldd, R, Cc, r0, c0);
     }
 }
 
@@ -409,11 +444,16 @@ extern "C" omb_status omb_stranspose(int64_t M, int64_t N, const float* A, int64
     //   A col,         C col (M x N as stored) = S^T    -> tiles
     const int64_t R = a_row ? M : N, Cc = a_row ? N : M;
     hipStream_t s = (hipStream_t)stream;
-    if (a_row == c_row) {
-        const bool on_lines = reinterpret_cast<uintptr_t>(C) % (kLine * sizeof(float)) == 0 &&
-                              ldc % kLine == 0;
+    const bool on_lines = reinterpret_cast<uintptr_t>(C) % (kLine * sizeof(float)) == 0 &&
+                          ldc % kLine == 0;
+    if (a_row == c_row && thin_transpose(R, Cc, on_lines)) {
+        const int64_t ntiles = ceil_div(R < TT ? Cc : R, (int64_t)TT);
+        const dim3 grid((unsigned)std::min<int64_t>(ntiles, kLaunchItems / NT / 4));
+        hipLaunchKernelGGL(transpose_thin_kernel, grid, dim3(NT), 0, s, R, Cc, ntiles, A, lda, C, ldc);
+    } else if (a_row == c_row) {
         const bool diag = on_lines && (lda % 8192 == 0 || ldc % 8192 == 0);
-        const bool big = R * Cc >= (int64_t)1 << 24;
+        // (2000000 x 12: 101 us in the large tiles, 38 so; 64 x 300000 36 and 29)
+        const bool big = R * Cc >= (int64_t)1 << 24 && R > 64 && Cc > 32;
         const int64_t rt = big ? 128 : 64, ct = big ? 64 : 32;
         // rows of D moved back by up to 31 floats can need one tile more
         const int64_t GR = ceil_div(R + (on_lines ? 0 : kLine - 1), rt), GC = ceil_div(Cc, ct);

@@ -48,3 +48,20 @@ def test_few_columns(dev, ompblas, m, n, off):
                                     y.data_ptr()))
         want = alpha * (a.double() @ x.double()) + beta * y0.double()
         assert torch.equal(y.double(), want)
+
+
+@pytest.mark.parametrize("m,n", [(1, 70001), (4, 128000), (9, 70000), (10, 6401), (11, 70001),
+                                 (31, 6400), (33, 70016), (40, 70001), (63, 70016), (64, 70001),
+                                 (64, 300001), (65, 300000), (12, 1500001)])
+@pytest.mark.parametrize("pad,off", [(0, 0), (1, 0), (0, 5), (32, 32)])
+def test_thin_transpose(dev, ompblas, m, n, pad, off):
+    for rows, cols in ((m, n), (n, m)):
+        src = torch.arange(rows * (cols + pad), device=dev, dtype=torch.int32).view(torch.float32)
+        a = src.view(rows, cols + pad)[:, :cols]
+        buf = torch.full((cols * (rows + pad) + off,), -1, device=dev, dtype=torch.int32)
+        guard = buf.clone()
+        c = buf.view(torch.float32)[off:].view(cols, rows + pad)[:, :rows]
+        ompblas.transpose(c, a)()
+        guard[off:].view(cols, rows + pad)[:, :rows] = \
+            src.view(torch.int32).view(rows, cols + pad)[:, :cols].t()
+        assert torch.equal(buf, guard)
